@@ -7,9 +7,9 @@
 // Reference: operatorlib::gemm_f16 / gemm_f32 (src/gemm.cu:440-479). The
 // reference dispatches between WMMA, cp.async register-tiled and scalar
 // kernels on divisibility; here the dispatch is, in order:
-//   * M <= 16 (decode shapes; the matrix-core one up to 32 fp16 / 64 fp32
-//     rows): the skinny kernels (namespace skinny), an HBM stream over B
-//     with split K and an ordered split sum;
+//   * M <= 2 (fp16, B from 8 MiB) or M <= 4 (fp32): the skinny kernel
+//     (namespace skinny), an HBM stream over B with split K and an ordered
+//     split sum (M <= 16 where K or N passes the 32-bit limits below);
 //   * N <= 16 (matrix-vector products): namespace narrow, an HBM stream
 //     over A, one launch;
 //   * gemm_dma_kernel (any K, N and alignment, K below 2^22 fp16 / 2^21
@@ -25,8 +25,8 @@
 //     4-byte alignment (every fp32 shape; fp16 with even K and N), or
 //     element-wise with zero fill (any shape and alignment); fp32 uses
 //     128 x 128 tiles on small grids.
-// Every path but the vector-ALU skinny kernel (M <= 4 fp16, M <= 8 fp32)
-// runs on the matrix cores.
+// Every path but the vector-ALU skinny and narrow kernels runs on the matrix
+// cores.
 //
 // Register-staged tiling (gemm_mfma_kernel, both precisions):
 //   * 256 x 256 C tile per workgroup. fp16: 2 x 2 wavefronts (256 threads),
@@ -53,7 +53,9 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstddef>
 #include <cstdint>
 #include <type_traits>
@@ -1129,8 +1131,8 @@ __global__ __launch_bounds__(256) void sum_tail_kernel(float* __restrict__ C, in
 //   * K is split over enough workgroups to fill the GPU; per-split partials
 //     go to scratch (arena or workspace) and a second kernel sums them in split
 //     order, so results are deterministic;
-//   * from M = 5 (fp16) or 9 (fp32) the vector-ALU dot products cost more
-//     than the B stream, and skinny_mfma_kernel (below) takes over.
+//   * from M = 3 (fp16) or 5 (fp32) ksplit_kernel is faster and takes over
+//     (Cfg::kUpToM).
 namespace skinny {
 
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
@@ -1148,17 +1150,15 @@ struct Cfg {
   static constexpr int kPerLane = 16 / sizeof(T);       // columns per lane
   static constexpr int kBlockN = kLanesPerRow * kPerLane;  // 64 fp32, 128 fp16
   static constexpr int kRowsPerStep = sizeof(T) == 2 ? 2 : 1;  // dot2 pairs
-  // From this M on the matrix-core variant is faster (measured on MI355X,
-  // N = K = 4096: fp16 M 4 -> 11.3 us vector ALU, M 6 -> 12.3 us matrix
-  // cores; fp32 M 8 -> 18.7 / 20.6 us, M 12 -> 27.9 / 21.9 us).
-  static constexpr int kMfmaMinM = sizeof(T) == 2 ? 5 : 9;
-  // The matrix-core kernel's largest M: 2 row blocks of 16 (fp16) or 4
-  // (fp32). Beyond, the 128 x 128-tile kernel split along K is faster.
-  // Measured on MI355X, N = K = 4096 (us, skinny vs 128 x 128 tiles split
-  // along K): fp16 M = 17 15.7 vs 19.6, M = 32 17.6 vs 20.8, M = 48 25.0
-  // vs 21.9, M = 64 27.5 vs 23.1; fp32 M = 17 23.6 vs 43.3, M = 32 25.0 vs
-  // 44.2, M = 48 41.1 vs 45.1, M = 64 42.1 vs 46.0.
-  static constexpr int kMaxMfmaM = sizeof(T) == 2 ? 32 : 64;
+  // The largest M this kernel takes, while B holds at least kMinBytes;
+  // beyond, and on smaller B, ksplit_kernel. Measured on MI355X (us, this
+  // kernel vs ksplit_kernel): fp16 M = 1 4096 x 4096 8.9 vs 10.2, 12288 x
+  // 4096 (N x K) 20.0 vs 22.0; M = 4 4096^2 10.8 vs 10.4, 4096 x 11008 22.1
+  // vs 18.2; M = 1 1024^2 5.5 vs 4.2, 768 x 3072 7.9 vs 5.7. fp32 M = 1
+  // 4096^2 14.0 vs 15.6, 1024^2 5.0 vs 6.3; M = 8 4096^2 17.7 vs 15.8,
+  // 1024^2 6.7 vs 6.5.
+  static constexpr int kUpToM = sizeof(T) == 2 ? 2 : 4;
+  static constexpr std::size_t kMinBytes = sizeof(T) == 2 ? std::size_t(8) << 20 : 0;
 };
 
 // Row steps (16-byte loads of one or two rows) in flight per thread per
@@ -1345,210 +1345,6 @@ void skinny_kernel(
   }
 }
 
-// Matrix-core variant for larger M (up to 32 fp16, 64 fp32, in row blocks
-// of 16): one v_mfma_f32_16x16x16_f16 (fp16) or v_mfma_f32_16x16x4_f32
-// (fp32) turns 16 rows of A times a 16 x 16 block of B into a 16 x 16 block
-// of C, where the vector-ALU kernel spends one dot product per (m, column
-// pair) and becomes ALU-bound as M grows.
-// B is never transposed: the MFMA only needs A and B to agree on which k
-// fills each of its k slots. K is walked in blocks of 16 rows; lane (g, c)
-// (g = lane / 16, c = lane % 16) owns rows 4g .. 4g+3 of each block (fp32
-// with unaligned A: blocks of 4 rows, row g each, 16 blocks in flight, as
-// the element loads gain nothing from the grouping):
-//   * it loads a 16-byte chunk (columns P*c .. P*c+P-1) of each of those
-//     rows, and MFMA j takes column j of every lane's chunk, so tile column
-//     c of MFMA j is matrix column P*c + j and P MFMAs cover the
-//     workgroup's 16 P columns;
-//   * its A operand values A[c][4g .. 4g+3] are contiguous, one 8-byte
-//     (fp16) or 16-byte (fp32) load straight from global memory (A is
-//     L2-resident), issued with the B loads, so nothing waits on a staging
-//     barrier; rows that are not 4-aligned fall back to element loads;
-//   * fp16 feeds the four rows to one 16x16x16 MFMA (k slots 4g .. 4g+3);
-//     fp32 issues four 16x16x4 MFMAs, the u-th taking row 4g + u in k slot
-//     g.
-// Splits, the workgroup shape and the partial sums are those of
-// skinny_kernel.
-template <typename T>
-struct MfmaCfg;
-template <>
-struct MfmaCfg<_Float16> {
-  typedef _Float16 AOp __attribute__((ext_vector_type(4)));
-  typedef _Float16 AVec __attribute__((ext_vector_type(4)));
-  static constexpr int kBatch = 4;    // 16-row k blocks in flight per wavefront
-  __device__ static floatx4v mma(AOp a, AOp b, floatx4v c) {
-    return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0);
-  }
-};
-template <>
-struct MfmaCfg<float> {
-  typedef float AOp;
-  typedef float AVec __attribute__((ext_vector_type(4)));
-  static constexpr int kBatch = 4;
-  __device__ static floatx4v mma(AOp a, AOp b, floatx4v c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-};
-
-// Rows of a k block that one lane owns (and the MFMA k slots they fill).
-constexpr int kLaneRows = 4;
-
-// kVecA: K % 4 == 0 and A aligned to 4 elements, so each lane's four A
-// values of a block are one aligned vector, wholly inside or outside k_end.
-// kMB row blocks of 16 (M up to 16 kMB): every B chunk a lane loads feeds
-// one MFMA per row block, so B is still streamed once.
-template <typename T, bool kVecA, int kMB>
-__global__ __launch_bounds__(kThreads) void skinny_mfma_kernel(
-    const T* __restrict__ A, const T* __restrict__ B, float* __restrict__ out,
-    int m_rows, int n, int k, int chunk) {
-  using MC = MfmaCfg<T>;
-  using Vec = typename RowChunk<T>::Vec;  // one 16-byte chunk of a B row
-  constexpr int P = Cfg<T>::kPerLane;     // columns per lane
-  constexpr int BN = Cfg<T>::kBlockN;     // 16 * P
-  // Rows per lane and k block: 4, or 1 for fp32 without vector A loads.
-  constexpr int R = sizeof(T) == 4 && !kVecA ? 1 : kLaneRows;
-  constexpr int KB = 4 * R;  // rows per k block
-  // k blocks in flight, halved at four row blocks (fp32 only): the full
-  // batch compiled to 193 VGPRs there, one wavefront per SIMD, the half to
-  // 78
-  constexpr int kBatch = (R == 1 ? 16 : MC::kBatch) / (kMB >= 4 ? 2 : 1);
-  using AVec = typename std::conditional<R == 1, T, typename MC::AVec>::type;
-  // k slot q of a lane's A values
-  auto a_at = [](const AVec& a, int q) -> T {
-    if constexpr (R == 1) return a; else return a[q];
-  };
-  __shared__ float red[kWaves * opl::kWaveSize * P * 4];
-
-  const int n0 = blockIdx.x * BN;
-  const int k0 = blockIdx.y * chunk;
-  const int k_end = min(k, k0 + chunk);
-  const int tid = threadIdx.x;
-  const int lane = tid % opl::kWaveSize;
-  const int wave = tid / opl::kWaveSize;
-  const int g = lane / 16;
-  const int c = lane % 16;
-  // Columns past N: read a valid chunk (n % P == 0), results not stored.
-  const int col = min(n0 + c * P, n - P);
-  const int blocks = (k_end - k0 + KB - 1) / KB;
-
-  // k block b, lane group g: k rows k0 + KB b + R g + q (q < R). B: a
-  // 16-byte chunk of each row; A: A[16 mb + c][row] of each row block mb
-  // (read from L2, every workgroup of the split reads the same A). Rows
-  // past k_end read valid memory and are zeroed, as are A rows past m_rows.
-  auto load_block = [&](int b, Vec (&v)[R], AVec (&a)[kMB]) {
-    const int r0 = k0 + KB * b + R * g;
-#pragma unroll
-    for (int q = 0; q < R; ++q) {
-      const int r = r0 + q;
-      const bool in = r < k_end;
-      const int rc = in ? r : k_end - 1;
-      // Non-temporal B loads for fp32 only. Measured on MI355X (us, cached
-      // -> non-temporal): fp32 M = 16 20.07 -> 19.51, M = 64 41.98 ->
-      // 41.24; fp16 M = 16 13.53 -> 14.04, M = 32 17.91 -> 19.58 (N = K =
-      // 4096).
-      const Vec* const src = reinterpret_cast<const Vec*>(B + static_cast<std::size_t>(rc) * n + col);
-      Vec x;
-      if constexpr (sizeof(T) == 4)
-        x = __builtin_nontemporal_load(src);
-      else
-        x = *src;
-#pragma unroll
-      for (int j = 0; j < P; ++j) x[j] = in ? x[j] : T(0);
-      v[q] = x;
-      if constexpr (!kVecA) {
-        // element loads, each issued beside its B row's load
-#pragma unroll
-        for (int mb = 0; mb < kMB; ++mb) {
-          const int arow = 16 * mb + c;
-          const bool a_in = in && arow < m_rows;
-          const T av = A[a_in ? static_cast<std::size_t>(arow) * k + r : 0];
-          if constexpr (R == 1)
-            a[mb] = a_in ? av : T(0);
-          else
-            a[mb][q] = a_in ? av : T(0);
-        }
-      }
-    }
-    if constexpr (kVecA) {
-      // r0 % 4 == 0 and k_end % 4 == 0: rows r0 .. r0+3 are all in or all
-      // out. Out-of-range lanes read A[0 .. 3] (k >= 4) and zero it.
-#pragma unroll
-      for (int mb = 0; mb < kMB; ++mb) {
-        const int arow = 16 * mb + c;
-        const bool a_in = r0 < k_end && arow < m_rows;
-        AVec x = *reinterpret_cast<const AVec*>(
-            A + (a_in ? static_cast<std::size_t>(arow) * k + r0 : 0));
-#pragma unroll
-        for (int q = 0; q < R; ++q) a[mb][q] = a_in ? x[q] : T(0);
-      }
-    }
-  };
-
-  floatx4v acc[kMB][P];
-#pragma unroll
-  for (int mb = 0; mb < kMB; ++mb)
-#pragma unroll
-    for (int j = 0; j < P; ++j)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) acc[mb][j][e] = 0.0f;
-
-  Vec v[kBatch][R];
-  AVec a[kBatch][kMB];
-  for (int b0 = wave; b0 < blocks; b0 += kWaves * kBatch) {
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      const int b = b0 + kWaves * u;
-      load_block(b < blocks ? b : blocks - 1, v[u], a[u]);
-    }
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      if (b0 + kWaves * u < blocks) {  // wave-uniform
-#pragma unroll
-        for (int j = 0; j < P; ++j) {
-          if constexpr (sizeof(T) == 2) {
-            typename MC::AOp bop;
-#pragma unroll
-            for (int q = 0; q < R; ++q) bop[q] = v[u][q][j];
-#pragma unroll
-            for (int mb = 0; mb < kMB; ++mb) acc[mb][j] = MC::mma(a[u][mb], bop, acc[mb][j]);
-          } else {
-#pragma unroll
-            for (int q = 0; q < R; ++q)
-#pragma unroll
-              for (int mb = 0; mb < kMB; ++mb)
-                acc[mb][j] = MC::mma(a_at(a[u][mb], q), v[u][q][j], acc[mb][j]);
-          }
-        }
-      }
-    }
-  }
-
-  // acc[mb][j][i] = C[16 mb + 4 g + i][n0 + P c + j] of this wavefront's
-  // k blocks; the wavefronts' sums go through LDS one row block at a time.
-  float* dst = out + static_cast<std::size_t>(blockIdx.y) * m_rows * n;
-#pragma unroll
-  for (int mb = 0; mb < kMB; ++mb) {
-    if (mb > 0) __syncthreads();  // the previous block's reads are done
-#pragma unroll
-    for (int j = 0; j < P; ++j)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        red[((wave * opl::kWaveSize + lane) * P + j) * 4 + i] = acc[mb][j][i];
-    __syncthreads();
-    for (int o = tid; o < 16 * BN; o += kThreads) {
-      const int m = o / BN;
-      const int co = o % BN;
-      const int row = 16 * mb + m;
-      if (row < m_rows && n0 + co < n) {
-        const int src = ((16 * (m / 4) + co / P) * P + co % P) * 4 + m % 4;
-        float s = red[src];
-#pragma unroll
-        for (int w = 1; w < kWaves; ++w) s += red[w * opl::kWaveSize * P * 4 + src];
-        dst[static_cast<std::size_t>(row) * n + n0 + co] = s;
-      }
-    }
-  }
-}
-
 // out[i] = sum over splits s (in order) of part[s][i]. Each thread issues
 // the loads of up to kSplitBatch splits before adding them, so a sum costs
 // one memory round trip per batch instead of one per split.
@@ -1576,26 +1372,29 @@ __global__ __launch_bounds__(kSumThreads) void sum_splits_kernel(
   }
 }
 
+// Enqueues the split sum of `count` outputs as the sequence's last launch.
+inline hipError_t sum_splits(const float* part, float* out, long long count, int splits,
+                             opl::ScratchLease* lease) {
+  const long long blocks = (count + kSumThreads - 1) / kSumThreads;
+  return lease->launch_last(sum_splits_kernel,
+                            dim3(static_cast<unsigned>(blocks < 16384 ? blocks : 16384)),
+                            dim3(kSumThreads), part, out, count, splits);
+}
+
 template <typename T, int M>
 void launch_m(const T* a, const T* b, float* dst, int m, int n, int k,
               int chunk, dim3 grid, hipStream_t stream) {
   skinny_kernel<T, M><<<grid, dim3(kThreads), 0, stream>>>(a, b, dst, m, n, k, chunk);
 }
 
-template <typename T, int kMB>
-void launch_mfma(bool vec_a, const T* a, const T* b, float* dst, int m, int n, int k,
-                 int chunk, dim3 grid, hipStream_t stream) {
-  if (vec_a)
-    skinny_mfma_kernel<T, true, kMB><<<grid, dim3(kThreads), 0, stream>>>(a, b, dst, m, n, k,
-                                                                        chunk);
-  else
-    skinny_mfma_kernel<T, false, kMB><<<grid, dim3(kThreads), 0, stream>>>(a, b, dst, m, n, k,
-                                                                         chunk);
-}
-
+// wide: K or N past the other kernels' 32-bit offsets, where this kernel
+// takes every M up to kMaxM.
 template <typename T>
-bool applies(const T* b, int m, int n) {
-  return m <= Cfg<T>::kMaxMfmaM && n % Cfg<T>::kPerLane == 0 && opl::aligned16(b);
+bool applies(const T* b, int m, int n, int k, bool wide) {
+  return n % Cfg<T>::kPerLane == 0 && opl::aligned16(b) &&
+         (wide ? m <= kMaxM
+               : m <= Cfg<T>::kUpToM &&
+                     static_cast<std::size_t>(k) * n * sizeof(T) >= Cfg<T>::kMinBytes);
 }
 
 // K split of one call: `splits` workgroup rows of `chunk` K rows each (a
@@ -1650,34 +1449,14 @@ hipError_t launch(const T* a, const T* b, float* c, int m, int n, int k, const P
   float* dst = p.splits > 1 ? static_cast<float*>(partials) : c;
   const int chunk = p.chunk;
   const dim3 grid(static_cast<unsigned>(blocks_n), static_cast<unsigned>(p.splits));
-  if (m >= C::kMfmaMinM) {
-    const bool vec_a =
-        k % kLaneRows == 0 &&
-        reinterpret_cast<std::uintptr_t>(a) % (kLaneRows * sizeof(T)) == 0;
-    if (m <= 16) {
-      launch_mfma<T, 1>(vec_a, a, b, dst, m, n, k, chunk, grid, stream);
-    } else if (m <= 32) {
-      launch_mfma<T, 2>(vec_a, a, b, dst, m, n, k, chunk, grid, stream);
-    } else {
-      if constexpr (C::kMaxMfmaM > 32)
-        launch_mfma<T, 4>(vec_a, a, b, dst, m, n, k, chunk, grid, stream);
-    }
-  } else if (m == 1) launch_m<T, 1>(a, b, dst, m, n, k, chunk, grid, stream);
+  if (m == 1) launch_m<T, 1>(a, b, dst, m, n, k, chunk, grid, stream);
   else if (m <= 2) launch_m<T, 2>(a, b, dst, m, n, k, chunk, grid, stream);
   else if (m <= 4) launch_m<T, 4>(a, b, dst, m, n, k, chunk, grid, stream);
   else if (m <= 8) launch_m<T, 8>(a, b, dst, m, n, k, chunk, grid, stream);
   else launch_m<T, 16>(a, b, dst, m, n, k, chunk, grid, stream);
-  if (p.splits > 1) {
-    const hipError_t status = hipGetLastError();
-    if (status != hipSuccess) return status;
-    const long long count = static_cast<long long>(m) * n;
-    const long long blocks = (count + kSumThreads - 1) / kSumThreads;
-    return lease->launch_last(sum_splits_kernel,
-                              dim3(static_cast<unsigned>(blocks < 16384 ? blocks : 16384)),
-                              dim3(kSumThreads), static_cast<const float*>(dst), c, count,
-                              p.splits);
-  }
-  return hipGetLastError();
+  const hipError_t status = hipGetLastError();
+  if (status != hipSuccess || p.splits == 1) return status;
+  return sum_splits(dst, c, static_cast<long long>(m) * n, p.splits, lease);
 }
 
 }  // namespace skinny
@@ -1820,6 +1599,431 @@ hipError_t launch(const T* a, const T* b, float* c, int m, int n, int k, hipStre
 }
 
 }  // namespace narrow
+
+// ---------------------------------------------------------------------------
+// Wavefront-split GEMM, for grids that 128 x 128 or 256 x 256 tiles would
+// leave mostly idle (medium M: a prompt of some tens to some hundreds of
+// tokens; small square products). A workgroup owns a 16 FM x 64 tile of C and
+// its W = 8 (Wide) or 4 (Deep) wavefronts split K between them: wavefront w
+// computes the whole tile over K steps w, w + W, ... of the workgroup's range,
+// from two LDS stages of its own, so the loop has no barrier: each wavefront
+// waits for its own copies only. The partial tiles are summed through LDS in
+// a fixed order at the end.
+//   * A stage is one substep of K (32 fp16, 16 fp32) or, Deep, two: 64- or
+//     128-byte A rows and as many K rows of B (64 columns). A wavefront reads
+//     its fragments into registers (a whole 16 FM x 64 tile per wavefront
+//     needs fewer LDS bytes per flop than sub-tiles of it would), refills the
+//     stage at once with its step after next and runs the MFMAs: up to 80-160
+//     KiB per CU are in flight, which is what the L2's latency asks for.
+//   * K is split over `splits` workgroups as well where the tiles are fewer
+//     than the CUs; their partial sums go to scratch and sum_splits_kernel
+//     adds them in order. The split inside the workgroup keeps those
+//     partials few: at most 6 M x N at M = 16, N = K = 4096, where the skinny
+//     matrix-core kernel this one replaced wrote 16.
+//   * Workgroups of one panel of the longer operand and one K range are
+//     neighbours on one XCD, so that operand is read from memory once and
+//     the shorter one comes from the XCD's L2.
+//   * Operands are read in place at any alignment and length, as by
+//     gemm_dma_kernel; the last partial step is repaired in registers
+//     (kEdge): A's k past K become zero, and the two fp16 end elements the
+//     dword range check zeroes are put back.
+// What bounds it: the L2s. With every copy reading cached addresses 300 x
+// 4096 x 4096 took 15.8 us, with the copies but no MFMAs 21.3, whole 20.2
+// (Wide). 256 workgroups of 80 x 64 move (80 + 64) K 2 bytes each, 302 MB in
+// all, at 17 TB/s. fp32 is bound by its MFMAs from 32 rows on.
+// Measured on MI355X (us, inputs cycling through three sets; the kernels that
+// ran before -> this one): fp16 16 x 4096 x 4096 13.4 -> 11.0, 32 17.6 ->
+// 11.5, 64 21.5 -> 12.9, 128 22.7 -> 14.4, 200 22.9 -> 16.5, 300 31.9 ->
+// 18.7, 640 49.7 -> 37.3; 300 x 4096 x 11008 69.4 -> 54.7; 1024^3 21.9 ->
+// 8.6, 333 x 777 x 999 12.3 -> 7.8; fp32 1000^3 31.5 -> 22.4, 512^3 22.5 ->
+// 6.2, 64 x 4096 x 4096 41.5 -> 24.3, 300 x 4096 x 4096 108 -> 82.
+// ---------------------------------------------------------------------------
+namespace ksplit {
+
+using dma::Elem;
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef __fp16 fp16x4 __attribute__((ext_vector_type(4)));
+#define OPL_LDS __attribute__((address_space(3)))
+
+constexpr int kBN = 64;
+constexpr int kFN = kBN / 16;
+
+// How a workgroup splits its K range: kWaves wavefronts, each with two LDS
+// stages of kSubs substeps (kSubK of K each: 64 bytes of an A row, 4 KiB of B
+// rows).
+template <int Waves, int Subs>
+struct Shape {
+  static constexpr int kWaves = Waves;
+  static constexpr int kSubs = Subs;
+  static constexpr int kThreads = Waves * opl::kWaveSize;
+  static constexpr int kARowBytes = 64 * Subs;
+  static constexpr int kAChunks = kARowBytes / 16;
+  static constexpr int kBBytes = 4096 * Subs;
+  static constexpr int kBCopies = kBBytes / 1024;
+  // XOR swizzle of A row m's 16-byte chunks (rows 16 apart share it).
+  __device__ static int swizzle_a(int m) { return Subs == 2 ? (m >> 1) & 7 : (m >> 2) & 3; }
+};
+// Two wavefronts per SIMD, 64-byte A rows; and one, with 128-byte A rows.
+using Wide = Shape<8, 1>;
+using Deep = Shape<4, 2>;
+
+template <typename T>
+__device__ __forceinline__ int swizzle_b(int k) {
+  // fp16: 128-byte rows, ds_read_b64_tr_b16 of rows k & 3 and bit 3 of k;
+  // the low row bit already picks the 128-byte half of the banks.
+  // fp32: 256-byte rows, the four lane groups of a ds_read_b32 on rows 4
+  // apart.
+  if constexpr (sizeof(T) == 2)
+    return 4 * ((k >> 1) & 1) ^ 2 * ((k >> 3) & 1);
+  else
+    return 4 * ((k >> 2) & 3);
+}
+template <typename T, int FM, typename S, bool kEdge>
+__global__ __launch_bounds__(S::kThreads)
+__attribute__((amdgpu_waves_per_eu(S::kWaves / 4, S::kWaves / 4 * (FM == 1 ? 2 : 1))))
+void ksplit_kernel(const T* __restrict__ A, const T* __restrict__ B, float* __restrict__ out,
+                   int M, int N, int K, int tiles_m, int tiles_n, int splits) {
+  constexpr int kWaves = S::kWaves, kSubs = S::kSubs, kThreads = S::kThreads;
+  constexpr int kARowBytes = S::kARowBytes, kAChunks = S::kAChunks;
+  constexpr int kBBytes = S::kBBytes, kBCopies = S::kBCopies;
+  constexpr int kStages = 2;
+  using Frag = typename Elem<T>::Frag;
+  constexpr int kSize = static_cast<int>(sizeof(T));
+  constexpr int kSubK = Elem<T>::kSubK;
+  constexpr int kBK = kSubs * kSubK;                 // K per step
+  constexpr int kBM = 16 * FM;
+  constexpr int kABytes = kBM * kARowBytes;
+  constexpr int kStage = kABytes + kBBytes;
+  constexpr int kElems = 16 / kSize;                 // per 16-byte chunk
+  constexpr int kBRowBytes = kBN * kSize;
+  constexpr int kBChunks = kBRowBytes / 16;
+  constexpr int kACopies = kABytes / 1024;
+  constexpr int kCopies = kACopies + kBCopies;       // per wavefront and stage
+  constexpr int kPitch = kBN + 4;                    // floats per merged row
+  constexpr int kMergeBytes = kBM * kPitch * 4;
+  static_assert(2 * kMergeBytes <= kWaves * kStage, "two partial tiles per stage array");
+  // One array per stage: the compiler then sees that copies into one do not
+  // touch the others.
+  __shared__ __attribute__((aligned(1024))) unsigned char stage0[kWaves * kStage];
+  __shared__ __attribute__((aligned(1024))) unsigned char stage1[kWaves * kStage];
+
+  // Items (panel of the longer side, K range, tile of the shorter side),
+  // the last fastest, in one contiguous range per XCD (workgroups are dealt
+  // to the XCDs round-robin): an XCD then reads its panels of the longer
+  // operand once and all of the shorter one. (With the row tiles always
+  // fastest every XCD read all of a tall A: 5184 x 896 x 11712 244 us.)
+  const bool tall = M > N;
+  const int inner = tall ? tiles_n : tiles_m;
+  const int items = tiles_m * tiles_n * splits;
+  const int per_xcd = (items + kXcds - 1) / kXcds;
+  const int item = static_cast<int>(blockIdx.x % kXcds) * per_xcd +
+                   static_cast<int>(blockIdx.x / kXcds);
+  if (item >= items) return;  // whole workgroup: padding of the grid to a multiple of 8
+  const int split = item / inner % splits;
+  const int outer = item / inner / splits;
+  const int m0 = (tall ? outer : item % inner) * kBM;
+  const int n0 = (tall ? item % inner : outer) * kBN;
+  const int total_steps = (K + kBK - 1) / kBK;
+  const int per = total_steps / splits, extra = total_steps % splits;
+  const int step0 = split * per + min(split, extra);
+  const int steps = per + (split < extra ? 1 : 0);
+
+  const int lane = threadIdx.x % opl::kWaveSize;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / opl::kWaveSize);
+  const int group = lane / 16;
+  const int gl = lane % 16;
+
+  // Copy j of this lane fills 16-byte slot 64 j + lane of the operand tile.
+  int a_dma[kACopies], b_dma[kBCopies];
+#pragma unroll
+  for (int j = 0; j < kACopies; ++j) {
+    const int slot = 64 * j + lane;
+    const int m = slot / kAChunks;
+    a_dma[j] = (min(m0 + m, M - 1) - m0) * K * kSize + 16 * ((slot % kAChunks) ^ S::swizzle_a(m));
+  }
+#pragma unroll
+  for (int j = 0; j < kBCopies; ++j) {
+    const int slot = 64 * j + lane;
+    const int k = slot / kBChunks;
+    b_dma[j] = k * N * kSize + 16 * ((slot % kBChunks) ^ swizzle_b<T>(k));
+  }
+  auto span = [](long long bytes) {
+    return static_cast<unsigned>(bytes < 0xffffffffLL ? bytes : 0xffffffffLL);
+  };
+  const long long a_total = static_cast<long long>(M - m0) * K * kSize;
+  const long long b_total = static_cast<long long>(K) * N * kSize - static_cast<long long>(kSize) * n0;
+  // Local step s of the workgroup (steps past its range read an empty range:
+  // zeros, no memory access).
+  auto issue = [&](unsigned char* st, int s) {
+    const unsigned live = s < steps ? ~0u : 0u;
+    const int k0 = (step0 + (s < steps ? s : 0)) * kBK;
+    const T* a_base = A + static_cast<std::size_t>(m0) * K + k0;
+    const T* b_base = B + static_cast<std::size_t>(k0) * N + n0;
+    const unsigned a_span = span(a_total - static_cast<long long>(kSize) * k0) & live;
+    const unsigned b_span = span(b_total - static_cast<long long>(kSize) * k0 * N) & live;
+#pragma unroll
+    for (int j = 0; j < kACopies; ++j)
+      opl::buffer_copy16_lds(a_base, a_span, st + j * 1024, a_dma[j]);
+#pragma unroll
+    for (int j = 0; j < kBCopies; ++j)
+      opl::buffer_copy16_lds(b_base, b_span, st + kABytes + j * 1024, b_dma[j]);
+  };
+
+  // Fragment offsets inside a stage: lane l supplies row / column l % 16 and
+  // the 16-byte k chunk l / 16 of a substep. Rows 16 apart share A's swizzle,
+  // substeps B's.
+  int a_lane[kSubs];
+#pragma unroll
+  for (int u = 0; u < kSubs; ++u)
+    a_lane[u] = gl * kARowBytes + (((4 * u + group) ^ S::swizzle_a(gl)) * 16);
+  int b_lane[kFN];
+#pragma unroll
+  for (int t = 0; t < kFN; ++t) {
+    if constexpr (kSize == 2) {
+      const int n = 16 * t + 4 * (gl % 4);
+      const int k = 8 * group + gl / 4;
+      b_lane[t] = kABytes + k * kBRowBytes + (((n / 8) ^ swizzle_b<T>(k)) * 16) + (n % 8) * 2;
+    } else {
+      const int n = 16 * t + gl;
+      const int k = 4 * group;
+      b_lane[t] = kABytes + k * kBRowBytes + (((n / 4) ^ swizzle_b<T>(k)) * 16) + (n % 4) * 4;
+    }
+  }
+
+  // The elements a copy's dword range check drops (fp16, odd row length).
+  T a_end_value = T(0), b_end_value = T(0);
+  const bool a_end = kSize == 2 && (K & 1) != 0 && m0 + kBM >= M;
+  const bool b_end = kSize == 2 && (N & 1) != 0 && n0 + kBN >= N;
+  if constexpr (kEdge) {
+    if (a_end) a_end_value = A[static_cast<std::size_t>(M) * K - 1];
+    if (b_end) b_end_value = B[static_cast<std::size_t>(K) * N - 1];
+  }
+
+  // Four wavefronts have registers for two sets of sums, one per stage: the
+  // chains of additions are then as short as eight wavefronts' (fp16 300 x
+  // 4096 x 4096, error against 64 bits: 2.1e-7 with one set).
+  constexpr int kSets = kWaves == 4 ? 2 : 1;
+  floatx4 sums[kSets][FM][kFN];
+#pragma unroll
+  for (int q = 0; q < kSets; ++q)
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < kFN; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sums[q][i][j][e] = 0.0f;
+
+  // One step of this wavefront: its stage has landed once all but the newer
+  // stage's copies have; the stage is refilled as soon as its fragments are
+  // in registers.
+  auto tile = [&](unsigned char* st, int s, floatx4 (&acc)[FM][kFN]) {
+    // vmcnt(kCopies): all but the newer stage's copies
+    __builtin_amdgcn_s_waitcnt((kCopies & 15) | ((kCopies >> 4) << 14) | 0xf70);
+    __builtin_amdgcn_sched_barrier(0);
+    Frag fa[kSubs][FM], fb[kSubs][kFN];
+#pragma unroll
+    for (int u = 0; u < kSubs; ++u) {
+#pragma unroll
+      for (int t = 0; t < FM; ++t)
+        fa[u][t] = *reinterpret_cast<const Frag*>(st + a_lane[u] + t * 16 * kARowBytes);
+#pragma unroll
+      for (int t = 0; t < kFN; ++t) {
+        const int rows = u * kSubK * kBRowBytes;
+        if constexpr (kSize == 2) {
+          const fp16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4f16(
+              (OPL_LDS fp16x4*)(st + b_lane[t] + rows));
+          const fp16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4f16(
+              (OPL_LDS fp16x4*)(st + b_lane[t] + rows + 4 * kBRowBytes));
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            fb[u][t][e] = lo[e];
+            fb[u][t][4 + e] = hi[e];
+          }
+        } else {
+          const OPL_LDS unsigned char* const bb =
+              (const OPL_LDS unsigned char*)(st + b_lane[t] + rows);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) fb[u][t][e] = *(const OPL_LDS float*)(bb + e * kBRowBytes);
+        }
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the fragments are in registers
+    __builtin_amdgcn_sched_barrier(0);
+    issue(st, s + kStages * kWaves);
+    if constexpr (kEdge) {
+      if (step0 + s == total_steps - 1) {
+        // k of element e of this lane's chunk, and its row and column of
+        // fragment 0; an element past K is zero (A), the last one put back.
+#pragma unroll
+        for (int u = 0; u < kSubs; ++u) {
+          int past = K - ((total_steps - 1) * kBK + u * kSubK + kElems * group);
+          asm volatile("" : "+v"(past));  // tests stay in this branch, not kept across the loop
+          const int a_row = a_end ? M - 1 - m0 - gl : -1;  // 16 t from there on: clamped rows
+          const int b_col = b_end ? N - 1 - n0 - gl : -1;
+#pragma unroll
+          for (int e = 0; e < kElems; ++e) {
+#pragma unroll
+            for (int t = 0; t < FM; ++t) {
+              if (e >= past) fa[u][t][e] = T(0);
+              if (e == past - 1 && a_end && 16 * t >= a_row) fa[u][t][e] = a_end_value;
+            }
+#pragma unroll
+            for (int t = 0; t < kFN; ++t)
+              if (e == past - 1 && b_end && 16 * t == b_col) fb[u][t][e] = b_end_value;
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kSubs; ++u) {
+      if constexpr (kSize == 2) {
+#pragma unroll
+        for (int ti = 0; ti < FM; ++ti)
+#pragma unroll
+          for (int tj = 0; tj < kFN; ++tj)
+            acc[ti][tj] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa[u][ti], fb[u][tj], acc[ti][tj],
+                                                                 0, 0, 0);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int ti = 0; ti < FM; ++ti)
+#pragma unroll
+            for (int tj = 0; tj < kFN; ++tj)
+              acc[ti][tj] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[u][ti][e], fb[u][tj][e],
+                                                                 acc[ti][tj], 0, 0, 0);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  unsigned char* const st0 = stage0 + wave * kStage;
+  unsigned char* const st1 = stage1 + wave * kStage;
+  int s = wave;
+  issue(st0, s);
+  issue(st1, s + kWaves);
+  for (; s + kWaves < steps; s += 2 * kWaves) {
+    tile(st0, s, sums[0]);
+    tile(st1, s + kWaves, sums[kSets - 1]);
+  }
+  if (s < steps) tile(st0, s, sums[0]);
+  floatx4 (&acc)[FM][kFN] = sums[0];
+  if constexpr (kSets == 2) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < kFN; ++j) acc[i][j] += sums[1][i][j];
+  }
+
+  // Sum of the wavefronts' partial tiles through LDS: of eight, 4-7 hand
+  // theirs to 0-3 first; the four sums are added in order on the way out.
+  __builtin_amdgcn_s_waitcnt(0);  // the last (empty) copies
+  __syncthreads();
+  auto slot = [&](int i) -> OPL_LDS float* {
+    return (OPL_LDS float*)((i < 2 ? stage0 : stage1) + (i & 1) * kMergeBytes);
+  };
+  OPL_LDS float* const mine = slot(wave & 3);
+  auto word = [&](int ti, int tj, int e) -> OPL_LDS float& {
+    return mine[(16 * ti + 4 * group + e) * kPitch + 16 * tj + gl];
+  };
+  auto write_partial = [&] {
+#pragma unroll
+    for (int ti = 0; ti < FM; ++ti)
+#pragma unroll
+      for (int tj = 0; tj < kFN; ++tj)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) word(ti, tj, e) = acc[ti][tj][e];
+  };
+  if constexpr (kWaves == 8) {
+    if (wave >= 4) write_partial();
+    __syncthreads();
+    if (wave < 4) {
+#pragma unroll
+      for (int ti = 0; ti < FM; ++ti)
+#pragma unroll
+        for (int tj = 0; tj < kFN; ++tj)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[ti][tj][e] += word(ti, tj, e);
+      write_partial();  // each lane rewrites the words it read
+    }
+  } else {
+    write_partial();
+  }
+  __syncthreads();
+  float* const dst = out + static_cast<std::size_t>(split) * M * N;
+  for (int i = threadIdx.x; i < kBM * (kBN / 4); i += kThreads) {
+    const int r = i / (kBN / 4);
+    const int c = 4 * (i % (kBN / 4));
+    floatx4 v = *(const OPL_LDS floatx4*)(slot(0) + r * kPitch + c);
+#pragma unroll
+    for (int g = 1; g < 4; ++g) v += *(const OPL_LDS floatx4*)(slot(g) + r * kPitch + c);
+    if (m0 + r < M) {
+      float* const p = dst + static_cast<std::size_t>(m0 + r) * N + n0 + c;
+      typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
+      if (n0 + c + 4 <= N) {
+        *reinterpret_cast<floatx4u*>(p) = v;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n0 + c + e < N) p[e] = v[e];
+      }
+    }
+  }
+}
+
+constexpr int kMaxSplits = 16;
+
+struct Plan {
+  int fm = 0;  // row fragments per tile; 0: not this kernel
+  int splits = 1;
+  bool deep = false;  // Deep instead of Wide
+  std::size_t bytes = 0;
+};
+
+template <typename T, int FM, typename S>
+void launch_shape(const T* a, const T* b, float* dst, int m, int n, int k, int splits,
+                  hipStream_t stream) {
+  const int tiles_m = (m + 16 * FM - 1) / (16 * FM);
+  const int tiles_n = (n + kBN - 1) / kBN;
+  const int items = tiles_m * tiles_n * splits;
+  const dim3 grid(static_cast<unsigned>((items + kXcds - 1) / kXcds * kXcds)), block(S::kThreads);
+  const bool edge = k % (S::kSubs * Elem<T>::kSubK) != 0 || (sizeof(T) == 2 && n % 2 != 0);
+  if (edge)
+    ksplit_kernel<T, FM, S, true><<<grid, block, 0, stream>>>(a, b, dst, m, n, k, tiles_m,
+                                                             tiles_n, splits);
+  else
+    ksplit_kernel<T, FM, S, false><<<grid, block, 0, stream>>>(a, b, dst, m, n, k, tiles_m,
+                                                             tiles_n, splits);
+}
+
+template <typename T, int FM>
+void launch_fm(const T* a, const T* b, float* dst, int m, int n, int k, const Plan& p,
+               hipStream_t stream) {
+  if constexpr (sizeof(T) == 2 && FM > 1) {
+    if (p.deep) return launch_shape<T, FM, Deep>(a, b, dst, m, n, k, p.splits, stream);
+  }
+  launch_shape<T, FM, Wide>(a, b, dst, m, n, k, p.splits, stream);
+}
+
+// Runs plan `p` (p.fm > 0); `partials` holds p.bytes of scratch when p.splits > 1.
+template <typename T>
+hipError_t launch(const T* a, const T* b, float* c, int m, int n, int k, const Plan& p,
+                  void* partials, opl::ScratchLease* lease, hipStream_t stream) {
+  float* const dst = p.splits > 1 ? static_cast<float*>(partials) : c;
+  switch (p.fm) {
+    case 1: launch_fm<T, 1>(a, b, dst, m, n, k, p, stream); break;
+    case 2: launch_fm<T, 2>(a, b, dst, m, n, k, p, stream); break;
+    case 3: launch_fm<T, 3>(a, b, dst, m, n, k, p, stream); break;
+    case 4: launch_fm<T, 4>(a, b, dst, m, n, k, p, stream); break;
+    case 5: launch_fm<T, 5>(a, b, dst, m, n, k, p, stream); break;
+    default: launch_fm<T, 6>(a, b, dst, m, n, k, p, stream); break;
+  }
+  const hipError_t status = hipGetLastError();
+  if (status != hipSuccess || p.splits == 1) return status;
+  return skinny::sum_splits(dst, c, static_cast<long long>(m) * n, p.splits, lease);
+}
+
+#undef OPL_LDS
+}  // namespace ksplit
 
 typedef unsigned uint4v __attribute__((ext_vector_type(4)));
 
@@ -2178,6 +2382,98 @@ TailPlan tail_plan(int m, int n, int k, std::size_t capacity) {
   return t;
 }
 
+// Time estimates (ns) that choose between ksplit_kernel's tile heights and
+// splits and the 128 x 128 tiles, from sweeps on MI355X of 150 shapes with M
+// 1..8000, N and K 100..12288. What bounds these grids is the L2: a CU's
+// copies arrive at 64-75 bytes/ns (the eight L2s together deliver about 17
+// TB/s), so a tile of R x C costs (R + C) K elements per round of
+// workgroups; fp32 tiles cost their matrix-core time, 4.1 ns per 16 rows
+// and k of a 64-column tile. Rows off 64 bytes straddle twice the lines.
+// B's stream from memory grows with the workgroups that ask for it (4500
+// bytes/ns when all do); partial sums cost a launch and their traffic.
+constexpr double kNsLaunch = 1000, kNsRound = 2500, kNsSum = 2300;
+constexpr double kTileBytesPerNs = 75, kOffLineFactor = 1.8, kStreamBytesPerNs = 4500;
+
+template <typename T>
+double ksplit_ns(int fm, int splits, int m, int n, int k, int cus) {
+  const double size = sizeof(T);
+  const double tiles = static_cast<double>((m + 16 * fm - 1) / (16 * fm)) * ((n + 63) / 64);
+  const double wgs = tiles * splits;
+  // fm = 1 workgroups (80 KiB of LDS) share a CU in pairs
+  const double rounds = std::ceil(wgs / cus) / (fm == 1 && splits > 1 && wgs <= 2.0 * cus ? 2 : 1);
+  const bool off_line = (n * sizeof(T)) % 64 != 0 || (k * sizeof(T)) % 64 != 0;
+  const double copies = (16.0 * fm + 64) * k * size / splits / kTileBytesPerNs *
+                        (off_line ? kOffLineFactor : 1.0);
+  const double mfma = sizeof(T) == 4 ? fm * static_cast<double>(k) / splits * 4.1 : 0.0;
+  // (the shorter operand is read by every XCD, mostly from the Infinity Cache)
+  const double operands = (std::max(m, n) + 4.0 * std::min(m, n)) * k * size;
+  const double uneven = wgs > cus ? std::max(1.0, rounds * cus / wgs) : 1.0;
+  const double stream = operands / (kStreamBytesPerNs * wgs / (wgs + 60)) * uneven;
+  return kNsLaunch + std::max(1.0, rounds) * kNsRound +
+         std::max(std::max(1.0, rounds) * std::max(copies, mfma), stream) +
+         (splits > 1 ? kNsSum + 8.0 * splits * m * n / 2500 : 0.0);
+}
+
+// The 128 x 128 tiles, split along K where tail_plan would.
+template <typename T>
+double small_tiles_ns(int m, int n, int k, int cus, const TailPlan& tail) {
+  const double tiles = static_cast<double>((m + 127) / 128) * ((n + 127) / 128);
+  const int splits = tail.splits > 0 ? tail.splits : 1;
+  const double rounds = std::ceil(tiles * splits / cus);
+  const double depth = static_cast<double>(k) / splits;
+  // two workgroups of a CU fetch faster than one: 70 against 55 bytes/ns
+  const double copies = 256 * depth * sizeof(T) / (rounds > 1 ? 70 : 55);
+  const double mfma = sizeof(T) == 4 ? depth * 59 : 0.0;
+  return 3000 + rounds * std::max(copies, mfma) +
+         (splits > 1 ? kNsSum + splits * tiles * 131072.0 / kStreamBytesPerNs : 0.0);
+}
+
+// ksplit_kernel's plan for shapes it is the fastest estimate for (fm == 0:
+// it is not). Every shape of the skinny range, whose rows would fill an
+// eighth of a 128-row tile; otherwise grids of few 256 x 256 tiles.
+template <typename T>
+ksplit::Plan ksplit_plan(int m, int n, int k, bool few_rows, std::size_t capacity) {
+  const long long big_tiles = static_cast<long long>((m + 255) / 256) * ((n + 255) / 256);
+  if (!few_rows && big_tiles >= DmaTiles<T>::kSmallBelow) return ksplit::Plan{};
+  int cus = device_cus();
+  if (cus <= 0) cus = 256;
+  ksplit::Plan best;
+  double best_ns = 0;
+  for (int fm = 1; fm <= 6; ++fm) {
+    const long long rows = (m + 16 * fm - 1) / (16 * fm);
+    if (fm > 1 && (m + 16 * (fm - 1) - 1) / (16 * (fm - 1)) == rows) continue;  // more padding
+    const long long tiles = rows * ((n + ksplit::kBN - 1) / ksplit::kBN);
+    if (tiles > 0x3fffffffLL) continue;
+    const long long slots = static_cast<long long>(cus) * (fm == 1 ? 2 : 1);
+    for (int splits = 1; splits <= ksplit::kMaxSplits; ++splits) {
+      // one split, or a grid the CUs hold at once with a step per wavefront
+      if (splits > 1 && (tiles * splits > slots || k / (8 * dma::Elem<T>::kSubK) < splits)) break;
+      const std::size_t bytes =
+          splits > 1 ? static_cast<std::size_t>(splits) * m * n * sizeof(float) : 0;
+      if (bytes > capacity) break;
+      const double ns = ksplit_ns<T>(fm, splits, m, n, k, cus);
+      if (best.fm == 0 || ns < best_ns) {
+        best_ns = ns;
+        best.fm = fm;
+        best.splits = splits;
+        best.bytes = bytes;
+      }
+    }
+  }
+  if (!few_rows) {
+    // (whole rounds of unsplit tiles are estimated closely: a near tie there,
+    // fp16 5184 x 896 x 11712 170 against 175 us, is theirs)
+    const TailPlan tail = tail_plan<T>(m, n, k, capacity);
+    if (small_tiles_ns<T>(m, n, k, cus, tail) * (tail.splits > 0 ? 1.0 : 0.95) < best_ns)
+      return ksplit::Plan{};
+  }
+  // 128-byte A rows once each wavefront walks enough of them. Measured on
+  // MI355X, fp16 (us, Wide vs Deep): 300 x 4096 x 4096 20.2 vs 18.4, 300 x
+  // 4096 x 11008 59.9 vs 54.7; 1024^3 8.6 vs 8.8, 1000^3 10.8 vs 11.9.
+  best.deep = k / best.splits >= 2048;
+  return best;
+}
+
 // The direct-to-LDS kernel (any K, N and alignment) on 128 x 128 or 256 x 256
 // tiles, with `tail` split into `partials` (tail.bytes of scratch).
 template <typename T>
@@ -2206,8 +2502,9 @@ hipError_t launch_gemm_dma(const T* a, const T* b, float* c, int m, int n, int k
 
 // One call's plan and the scratch it needs.
 struct GemmPlan {
-  enum Kind { kSkinny, kNarrow, kDma, kRegister } kind = kRegister;
+  enum Kind { kSkinny, kNarrow, kSplit, kDma, kRegister } kind = kRegister;
   skinny::Plan skinny;
+  ksplit::Plan split;
   TailPlan tail;  // kDma
   PadPlan pad;    // kDma
   int staging = kElementwise;  // kRegister
@@ -2217,7 +2514,11 @@ struct GemmPlan {
 template <typename T>
 GemmPlan plan_gemm(const T* a, const T* b, int m, int n, int k, std::size_t capacity) {
   GemmPlan p;
-  if (skinny::applies(b, m, n)) {
+  // The copy kernels' per-lane offsets inside a tile are 32-bit: up to
+  // 255 rows of A (255 * K * sizeof(T) bytes) and one K step of B rows (64
+  // fp16 or 32 fp32 rows: 128 * N bytes).
+  const bool dma_offsets_fit = k < (sizeof(T) == 2 ? (1 << 22) : (1 << 21)) && n < (1 << 24);
+  if (skinny::applies(b, m, n, k, !dma_offsets_fit)) {
     p.skinny = skinny::plan<T>(m, n, k, capacity);
     if (p.skinny.ok) {
       p.kind = GemmPlan::kSkinny;
@@ -2225,14 +2526,19 @@ GemmPlan plan_gemm(const T* a, const T* b, int m, int n, int k, std::size_t capa
       return p;
     }
   }
-  if (narrow::applies(a, b, n, k)) {
+  const bool few_rows = m <= (sizeof(T) == 2 ? 32 : 64);
+  if (!(few_rows && n % skinny::Cfg<T>::kPerLane == 0) && narrow::applies(a, b, n, k)) {
     p.kind = GemmPlan::kNarrow;
     return p;
   }
-  // The copy kernel's per-lane offsets inside a tile are 32-bit: up to
-  // 255 rows of A (255 * K * sizeof(T) bytes) and one K step of B rows (64
-  // fp16 or 32 fp32 rows: 128 * N bytes).
-  const bool dma_offsets_fit = k < (sizeof(T) == 2 ? (1 << 22) : (1 << 21)) && n < (1 << 24);
+  if (dma_offsets_fit) {
+    p.split = ksplit_plan<T>(m, n, k, few_rows, capacity);
+    if (p.split.fm > 0) {
+      p.kind = GemmPlan::kSplit;
+      p.bytes = p.split.bytes;
+      return p;
+    }
+  }
   if (dma_offsets_fit) {
     p.kind = GemmPlan::kDma;
     p.pad = pad_plan<T>(a, b, m, n, k);
@@ -2256,6 +2562,8 @@ hipError_t run_gemm(const GemmPlan& p, const T* a, const T* b, float* c, int m, 
   switch (p.kind) {
     case GemmPlan::kSkinny:
       return skinny::launch<T>(a, b, c, m, n, k, p.skinny, scratch, lease, stream);
+    case GemmPlan::kSplit:
+      return ksplit::launch<T>(a, b, c, m, n, k, p.split, scratch, lease, stream);
     case GemmPlan::kNarrow:
       return narrow::launch<T>(a, b, c, m, n, k, stream);
     case GemmPlan::kDma: {

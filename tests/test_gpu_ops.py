@@ -491,6 +491,53 @@ def test_gemm_skinny_row_blocks(hip, mnk, dtype):
     assert np.isfinite(y).all()
 
 
+# ksplit_kernel, whose wavefronts split K: every tile height (16 to 96 rows)
+# one row short, exact and one over; N around its 64-column tiles; K around
+# its steps (32 / 16, 64 at K >= 2048) and fewer steps than wavefronts; odd K
+# and N (the end elements a copy's range check drops); K split over
+# workgroups too (first and last range of uneven ones); M > N, whose items
+# run in the other order.
+KSPLIT = [(15, 64, 256), (17, 65, 31), (33, 63, 33), (47, 130, 95), (80, 4096, 512),
+          (81, 200, 1001), (97, 127, 64), (96, 3000, 2048), (300, 4100, 2049), (64, 4096, 2111),
+          (5, 203, 4099), (16, 512, 8191), (3, 1, 1), (64, 33, 4097), (700, 40, 999),
+          (1000, 70, 2050), (301, 333, 7)]
+
+
+@pytest.mark.parametrize("mnk", KSPLIT)
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("dtype", ["f32", "f16"])
+def test_gemm_ksplit(hip, mnk, offset, dtype):
+    """Against the oracle: fp16 products of values in [-1, 1] summed in fp32
+    (K 2^-24 sqrt(K) stays under 1e-4, the bound is the fp16 bar's 2e-3),
+    fp32 at the Frobenius bar. NaN just past both operands and around C: an
+    element read past them, or a store outside C, would show. Twice: the sum
+    order is fixed."""
+    m, n, k = mnk
+    a, b = oracle.uniform(900 + m, (m, k)), oracle.uniform(901 + n, (k, n))
+    if dtype == "f16":
+        a, b = oracle.to_f16_bits(a), oracle.to_f16_bits(b)
+        ref = oracle.gemm(oracle.from_f16_bits(a), oracle.from_f16_bits(b))
+        fn, nan = hip.lib.operatorlib_gemm_f16, np.uint16(0x7e00)
+    else:
+        ref = oracle.gemm(a, b)
+        fn, nan = hip.lib.operatorlib_gemm_f32, np.float32("nan")
+    pad = np.full(256, nan, dtype=a.dtype)
+    da, db = (to_device(np.concatenate([x.ravel(), pad]), offset) for x in (a, b))
+    outs = []
+    for _ in range(2):
+        out = torch.full((m * n + 512,), float("nan"), device="cuda")
+        check(fn(ptr(da), ptr(db), ptr(out[256:]), m, n, k, stream_handle()), "gemm")
+        torch.cuda.synchronize()
+        outs.append(out.cpu().numpy())
+    assert np.isnan(outs[0][:256]).all() and np.isnan(outs[0][256 + m * n:]).all()
+    y = outs[0][256:256 + m * n].reshape(m, n).astype(np.float64)
+    assert np.array_equal(outs[0], outs[1], equal_nan=True)
+    if dtype == "f16":
+        assert np.max(np.abs(y - ref)) <= 2e-3
+    else:
+        assert np.linalg.norm(y - ref) <= 1e-4 * np.linalg.norm(ref)
+
+
 # Narrow N (<= 16) past the skinny kernels: matrix-vector products and a
 # few right-hand columns on the narrow kernel. Rows past M in the last
 # wavefront, a partial last K step (K = 1000: 125 fp16 / 250 fp32 chunks),
