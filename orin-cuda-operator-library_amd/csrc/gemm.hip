@@ -269,7 +269,8 @@ __device__ __forceinline__ void grouped_tile(int idx, int tiles_m, int tiles_n,
 // Launch index b of `blocks` -> grouped-order index: regroups the
 // round-robin XCD dispatch so that consecutive tiles land on one XCD.
 __device__ __forceinline__ int xcd_regroup(int b, int blocks) {
-  return blocks % kXcds == 0 ? (b % kXcds) * (blocks / kXcds) + b / kXcds : b;
+  const int x = b % kXcds;
+  return x * (blocks / kXcds) + min(x, blocks % kXcds) + b / kXcds;
 }
 
 // Maps the launch index to a C tile: XCD regrouping, then the grouped order.
@@ -540,9 +541,10 @@ struct Tile {
   static constexpr int kBBytes = BK * kBRowBytes;
   static constexpr int kBChunks = kBRowBytes / 16;
   static constexpr int kStage = kABytes + kBBytes;
-  // DMA chunks per thread per operand.
-  static constexpr int kCopies = kABytes / 16 / kThreads;
-  static_assert(kABytes == kBBytes && kCopies * 16 * kThreads == kABytes,
+  // DMA chunks per thread and operand.
+  static constexpr int kACopies = kABytes / 16 / kThreads;
+  static constexpr int kBCopies = kBBytes / 16 / kThreads;
+  static_assert(kACopies * 16 * kThreads == kABytes && kBCopies * 16 * kThreads == kBBytes,
                 "both operand tiles split evenly into 16-byte copies");
   static_assert(64 % kBChunks == 0, "a wavefront copies whole B rows");
   static_assert((kARowBytes == 128 && Stages == 2) || (kARowBytes == 64 && Stages == 4),
@@ -567,6 +569,11 @@ struct Tile {
 using BigTile = Tile<_Float16, 256, 256, 2, 4, 64, 2>;
 // The same for K % 64 == 32.
 using BigTileK32 = Tile<_Float16, 256, 256, 2, 4, 32, 4>;
+// 192 x 256 and 128 x 256: the same wavefronts on 96 or 64 rows, for grids
+// that 256 x 256 tiles would not fill (one round only: over several rounds
+// they only add copies, 6144 x 6144 x 2048 163 against 169 and 180 us).
+using Tile192 = Tile<_Float16, 192, 256, 2, 4, 64, 2>;
+using Tile128 = Tile<_Float16, 128, 256, 2, 4, 64, 2>;
 // 128 x 128: 4 wavefronts of 64 x 64, four times the workgroups for the
 // same C, for grids that would leave CUs idle with BigTile.
 using SmallTile = Tile<_Float16, 128, 128, 2, 2, 32, 4>;
@@ -593,11 +600,12 @@ void gemm_dma_kernel(const typename Cfg::Type* __restrict__ A,
   constexpr int kBM = Cfg::kBM, kBN = Cfg::kBN, kBK = Cfg::kBK;
   constexpr int kWM = Cfg::kWM, kWN = Cfg::kWN;
   constexpr int kFM = Cfg::kFM, kFN = Cfg::kFN;
-  constexpr int kABytes = Cfg::kABytes, kCopies = Cfg::kCopies;
+  constexpr int kABytes = Cfg::kABytes;
+  constexpr int kACopies = Cfg::kACopies, kBCopies = Cfg::kBCopies;
   constexpr int kBChunks = Cfg::kBChunks;
   constexpr int kSize = static_cast<int>(sizeof(T));
   constexpr int kReads = kFM + E::kBReads * kFN;  // LDS read instructions per substep
-  constexpr int kIssues = 2 * kCopies;            // DMA instructions per K step
+  constexpr int kIssues = kACopies + kBCopies;    // DMA instructions per K step
   static_assert(kWM == 2, "A fragment offsets assume two wavefront rows");
 
   const int tiles_m = (M + kBM - 1) / kBM;
@@ -640,7 +648,7 @@ void gemm_dma_kernel(const typename Cfg::Type* __restrict__ A,
   const int gl = lane % 16;
 
   // DMA sources: copy j of this thread fills LDS chunk slot
-  // (wave * kCopies + j) * 64 + lane of each operand tile. They are byte
+  // (wave * copies + j) * 64 + lane of each operand tile. They are byte
   // offsets from the step's scalar bases A + m0 * lda + k0 and
   // B + k0 * ldb + n0 (A rows clamped to M - 1), read through buffer
   // resources: no 64-bit vector address math per copy. The copies need no
@@ -649,15 +657,18 @@ void gemm_dma_kernel(const typename Cfg::Type* __restrict__ A,
   // any length are read in place. A chunk that runs past its row's end
   // reads the next row's first elements: past N those fill columns that
   // are never stored; past K, see fix_stage.
-  int a_dma[kCopies];
-  int b_dma[kCopies];
+  int a_dma[kACopies];
+  int b_dma[kBCopies];
 #pragma unroll
-  for (int j = 0; j < kCopies; ++j) {
-    const int slot = (wave * kCopies + j) * 64 + lane;
+  for (int j = 0; j < kACopies; ++j) {
+    const int slot = (wave * kACopies + j) * 64 + lane;
     const int m = slot / Cfg::kAChunks;
     const int chunk = (slot % Cfg::kAChunks) ^ Cfg::swizzle_a(m);
     a_dma[j] = (min(m0 + m, M - 1) - m0) * lda * kSize + 16 * chunk;
-    const int kk = (wave * kCopies + j) * (64 / kBChunks) + lane / kBChunks;
+  }
+#pragma unroll
+  for (int j = 0; j < kBCopies; ++j) {
+    const int kk = (wave * kBCopies + j) * (64 / kBChunks) + lane / kBChunks;
     const int col = Cfg::kChunkElems * ((lane % kBChunks) ^ Cfg::swizzle_b(kk));
     b_dma[j] = kk * ldb * kSize + col * kSize;
   }
@@ -700,11 +711,12 @@ void gemm_dma_kernel(const typename Cfg::Type* __restrict__ A,
     const T* a_base = a_tile + k0;
     const T* b_base = b_tile + static_cast<std::size_t>(k0) * ldb;
 #pragma unroll
-    for (int j = 0; j < kCopies; ++j) {
-      opl::buffer_copy16_lds(a_base, a_span, stage + (wave * kCopies + j) * 1024,
-                             a_dma[j]);
-      opl::buffer_copy16_lds(b_base, b_span, stage + kABytes + (wave * kCopies + j) * 1024,
-                             b_dma[j]);
+    for (int j = 0; j < std::max(kACopies, kBCopies); ++j) {
+      if (j < kACopies)
+        opl::buffer_copy16_lds(a_base, a_span, stage + (wave * kACopies + j) * 1024, a_dma[j]);
+      if (j < kBCopies)
+        opl::buffer_copy16_lds(b_base, b_span, stage + kABytes + (wave * kBCopies + j) * 1024,
+                               b_dma[j]);
     }
   };
 
@@ -2210,6 +2222,13 @@ int staging_for(const T* a, const T* b, int n, int k) {
 
 int device_cus();
 
+// Shapes with a partly filled last K step, or fp16 rows of odd length.
+template <typename Cfg>
+bool dma_edge(int k, int lda, int ldb) {
+  return k % Cfg::kBK != 0 ||
+         (sizeof(typename Cfg::Type) == 2 && (lda % 2 != 0 || ldb % 2 != 0));
+}
+
 template <typename Cfg>
 hipError_t launch_dma_tiles(const typename Cfg::Type* a, const typename Cfg::Type* b, float* c,
                             int m, int n, int k, int lda, int ldb, hipStream_t stream,
@@ -2222,7 +2241,7 @@ hipError_t launch_dma_tiles(const typename Cfg::Type* a, const typename Cfg::Typ
   // Shapes with a partly filled last K step, or fp16 rows of odd length,
   // run the instance that repairs that step (the others keep the plain
   // schedule: the repair's code cost the aligned 4096^3 product 2%).
-  const bool edge = k % Cfg::kBK != 0 || (sizeof(typename Cfg::Type) == 2 && (lda % 2 != 0 || ldb % 2 != 0));
+  const bool edge = dma_edge<Cfg>(k, lda, ldb);
   // C is stored non-temporally when later rounds re-read operand panels
   // that cached C lines would evict: fp16 256 x 256 grids (whose whole
   // tiles leave through LDS as full cache lines) of two or more rounds,
@@ -2243,15 +2262,18 @@ hipError_t launch_dma_tiles(const typename Cfg::Type* a, const typename Cfg::Typ
   const bool stream_c = kCanStream && tail.splits == 0 && operand_bytes >= (192LL << 20) &&
                         device_cus() > 0 && tiles >= 2LL * device_cus();
   const dim3 grid(static_cast<unsigned>(blocks)), block(Cfg::kThreads);
-  if (tail.splits > 0) {
-    if (edge)
-      dma::gemm_dma_kernel<Cfg, true, true><<<grid, block, 0, stream>>>(a, b, c, m, n, k, lda,
-                                                                        ldb, tail);
-    else
-      dma::gemm_dma_kernel<Cfg, true><<<grid, block, 0, stream>>>(a, b, c, m, n, k, lda, ldb,
-                                                                  tail);
-    dma::sum_tail_kernel<Cfg><<<dim3(Cfg::kBM * Cfg::kBN / 4 / 256, tail.tiles), dim3(256), 0,
-                                stream>>>(c, m, n, tail);
+  constexpr bool kCanSplit = Cfg::kBM == Cfg::kBN;  // (one-round tiles never are)
+  if (kCanSplit && tail.splits > 0) {
+    if constexpr (kCanSplit) {
+      if (edge)
+        dma::gemm_dma_kernel<Cfg, true, true><<<grid, block, 0, stream>>>(a, b, c, m, n, k, lda,
+                                                                          ldb, tail);
+      else
+        dma::gemm_dma_kernel<Cfg, true><<<grid, block, 0, stream>>>(a, b, c, m, n, k, lda, ldb,
+                                                                    tail);
+      dma::sum_tail_kernel<Cfg><<<dim3(Cfg::kBM * Cfg::kBN / 4 / 256, tail.tiles), dim3(256), 0,
+                                  stream>>>(c, m, n, tail);
+    }
   } else if (stream_c) {
     if constexpr (kCanStream) {
       if (edge)
@@ -2316,6 +2338,7 @@ struct DmaTiles<_Float16> {
   using BigHalfK = dma::BigTileK32;  // K % 64 == 32
   using Small = dma::SmallTile;
   static constexpr long long kSmallBelow = kSmallGridTiles;
+  static constexpr bool kOneRound = true;  // one_round_rows applies
 };
 template <>
 struct DmaTiles<float> {
@@ -2323,7 +2346,32 @@ struct DmaTiles<float> {
   using BigHalfK = dma::BigTileF32K16;  // K % 32 == 16
   using Small = dma::SmallTileF32;
   static constexpr long long kSmallBelow = kSmallGridTilesF32;
+  static constexpr bool kOneRound = false;  // (2% at most: 3072 x 4096 x 4096 700 vs 686 us)
 };
+
+// Rows of the tiles that cover an fp16 grid in one round when 256 x 256 ones
+// would leave CUs idle: 128 (x 256) for more than half a round and at most
+// one of them, else 192 likewise, else 0 (neither). One workgroup per CU, so
+// the round's time falls with the tile. Measured on MI355X (us, 256 x 256 /
+// 192 x 256 / 128 x 256 / 128 x 128 tiles, on a slow box): 2048 x 4096 x
+// 4096 77 / 69 / 67 / 77, 1280 x 4096 x 4096 72 / 62 / 57 / 67, 3000^3 70 /
+// 64 / 106 / 93, 1536 x 8192 x 4096 106 / 100 / 155 / 130, 3072 x 4096 x
+// 4096 108 / 101 / 121 / 114. Half a round or less of 128 x 256 tiles leaves
+// a CU per 128 x 128 tile, whose copies are then faster (1000 x 4096 x 4096
+// 40). Against the tiles chosen before (us): 3000^3 93.8 -> 62.5, 2048 x 4096
+// x 4096 74.3 -> 64.3, 1500 x 6000 x 700 30.9 -> 22.3, 2000 x 3000 x 512 17.6
+// -> 14.5, 1536 x 8192 x 4096 106.3 -> 99.5. (The tiles of a partly filled
+// last round as 128 x 256 halves in a second launch lost: 2000 x 11008 x 4096
+// 188 -> 203.)
+int one_round_rows(int m, int n) {
+  const long long cus = device_cus();
+  const long long cols = (n + 255) / 256;
+  const long long tiles128 = (m + 127) / 128 * cols, tiles192 = (m + 191) / 192 * cols;
+  // (not where 256-column tiles pad N by over a tenth more than 128-column ones)
+  if (tiles128 <= cus / 2 || 20 * cols > 11LL * ((n + 127) / 128)) return 0;
+  if (tiles128 <= cus) return 128;
+  return tiles192 <= cus ? 192 : 0;
+}
 
 // Split of the last round of a 256 x 256-tile grid (splits == 0: none).
 struct TailPlan {
@@ -2352,6 +2400,7 @@ TailPlan tail_plan(int m, int n, int k, std::size_t capacity) {
       ((n + dma::BigTile::kBN - 1) / dma::BigTile::kBN);
   long long split_tiles = 0, full = 0, want = 0;
   std::size_t tile_bytes = 0;
+  if (DmaTiles<T>::kOneRound && one_round_rows(m, n) > 0) return t;
   if (big_tiles < DmaTiles<T>::kSmallBelow) {
     using Small = typename DmaTiles<T>::Small;
     const long long tiles = static_cast<long long>((m + Small::kBM - 1) / Small::kBM) *
@@ -2414,9 +2463,16 @@ double ksplit_ns(int fm, int splits, int m, int n, int k, int cus) {
          (splits > 1 ? kNsSum + 8.0 * splits * m * n / 2500 : 0.0);
 }
 
-// The 128 x 128 tiles, split along K where tail_plan would.
+// The 128 x 128 tiles, split along K where tail_plan would, or one round of
+// 128 x 256 or 192 x 256 ones (8 us and 7 ns per k, and what the round's
+// workgroups take from the L2s).
 template <typename T>
 double small_tiles_ns(int m, int n, int k, int cus, const TailPlan& tail) {
+  const int one_round = DmaTiles<T>::kOneRound ? one_round_rows(m, n) : 0;
+  if (one_round > 0) {
+    const double wgs = static_cast<double>((m + one_round - 1) / one_round) * ((n + 255) / 256);
+    return 8000 + k * (7 + (one_round == 128 ? 7.4 : 15.6) * wgs / cus);
+  }
   const double tiles = static_cast<double>((m + 127) / 128) * ((n + 127) / 128);
   const int splits = tail.splits > 0 ? tail.splits : 1;
   const double rounds = std::ceil(tiles * splits / cus);
@@ -2491,6 +2547,13 @@ hipError_t launch_gemm_dma(const T* a, const T* b, float* c, int m, int n, int k
   if (tail.splits > 0)
     split = dma::TailSplit{static_cast<int>(tail.full), static_cast<int>(tail.last), tail.splits,
                            static_cast<float*>(partials)};
+  if constexpr (Tiles::kOneRound) {
+    switch (one_round_rows(m, n)) {
+      case 128: return launch_dma_tiles<dma::Tile128>(a, b, c, m, n, k, lda, ldb, stream);
+      case 192: return launch_dma_tiles<dma::Tile192>(a, b, c, m, n, k, lda, ldb, stream);
+      default: break;
+    }
+  }
   if (big_tiles < Tiles::kSmallBelow)
     return launch_dma_tiles<typename Tiles::Small>(a, b, c, m, n, k, lda, ldb, stream, split);
   // A last step at most half full runs on the half-deep stages.

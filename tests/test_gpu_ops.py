@@ -538,6 +538,26 @@ def test_gemm_ksplit(hip, mnk, offset, dtype):
         assert np.linalg.norm(y - ref) <= 1e-4 * np.linalg.norm(ref)
 
 
+# fp16 grids that one round of 128 x 256 tiles (first four) or 192 x 256 tiles
+# covers: ragged M, N and K, rows at a 2-byte phase, one K step and several,
+# a tile count that is no multiple of the eight XCDs.
+ONE_ROUND = [(1290, 4090, 130), (2000, 3000, 512), (1409, 3330, 65), (3840, 2304, 33),
+             (3000, 3000, 96), (3001, 2999, 161), (2300, 5120, 64), (1537, 8000, 127)]
+
+
+@pytest.mark.parametrize("mnk", ONE_ROUND)
+def test_gemm_f16_one_round(hip, mnk):
+    m, n, k = mnk
+    ab = oracle.to_f16_bits(oracle.uniform(930 + k, (m, k)))
+    bb = oracle.to_f16_bits(oracle.uniform(931 + n, (k, n)))
+    rows = np.unique(np.concatenate([np.arange(0, m, 191), np.arange(127, m, 128),
+                                     np.arange(max(0, m - 3), m)]))
+    y = hip.gemm_f16(ab, bb)
+    ref = oracle.gemm(oracle.from_f16_bits(ab), oracle.from_f16_bits(bb), rows)
+    assert np.max(np.abs(y[rows] - ref)) <= 2e-3
+    assert np.isfinite(y).all()
+
+
 # Narrow N (<= 16) past the skinny kernels: matrix-vector products and a
 # few right-hand columns on the narrow kernel. Rows past M in the last
 # wavefront, a partial last K step (K = 1000: 125 fp16 / 250 fp32 chunks),
