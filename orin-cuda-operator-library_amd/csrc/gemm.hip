@@ -269,8 +269,7 @@ __device__ __forceinline__ void grouped_tile(int idx, int tiles_m, int tiles_n,
 // Launch index b of `blocks` -> grouped-order index: regroups the
 // round-robin XCD dispatch so that consecutive tiles land on one XCD.
 __device__ __forceinline__ int xcd_regroup(int b, int blocks) {
-  const int x = b % kXcds;
-  return x * (blocks / kXcds) + min(x, blocks % kXcds) + b / kXcds;
+  return blocks % kXcds == 0 ? (b % kXcds) * (blocks / kXcds) + b / kXcds : b;
 }
 
 // Maps the launch index to a C tile: XCD regrouping, then the grouped order.
@@ -2438,29 +2437,31 @@ TailPlan tail_plan(int m, int n, int k, std::size_t capacity) {
 // TB/s), so a tile of R x C costs (R + C) K elements per round of
 // workgroups; fp32 tiles cost their matrix-core time, 4.1 ns per 16 rows
 // and k of a 64-column tile. Rows off 64 bytes straddle twice the lines.
-// B's stream from memory grows with the workgroups that ask for it (4500
-// bytes/ns when all do); partial sums cost a launch and their traffic.
+// The operands' stream from memory grows with the workgroups that ask for it
+// (towards 8000 bytes/ns); partial sums cost a launch and their traffic.
 constexpr double kNsLaunch = 1000, kNsRound = 2500, kNsSum = 2300;
-constexpr double kTileBytesPerNs = 75, kOffLineFactor = 1.8, kStreamBytesPerNs = 4500;
+constexpr double kTileBytesPerNs = 75, kOffLineFactor = 1.8, kStreamBytesPerNs = 8000;
+constexpr double kPartialBytesPerNs = 2500, kTilePartialBytesPerNs = 4500;
 
 template <typename T>
 double ksplit_ns(int fm, int splits, int m, int n, int k, int cus) {
   const double size = sizeof(T);
   const double tiles = static_cast<double>((m + 16 * fm - 1) / (16 * fm)) * ((n + 63) / 64);
   const double wgs = tiles * splits;
+  const double rounds = std::ceil(wgs / cus);
   // fm = 1 workgroups (80 KiB of LDS) share a CU in pairs
-  const double rounds = std::ceil(wgs / cus) / (fm == 1 && splits > 1 && wgs <= 2.0 * cus ? 2 : 1);
+  const double starts = fm == 1 && wgs <= 2.0 * cus ? 1 : rounds;
   const bool off_line = (n * sizeof(T)) % 64 != 0 || (k * sizeof(T)) % 64 != 0;
   const double copies = (16.0 * fm + 64) * k * size / splits / kTileBytesPerNs *
                         (off_line ? kOffLineFactor : 1.0);
   const double mfma = sizeof(T) == 4 ? fm * static_cast<double>(k) / splits * 4.1 : 0.0;
   // (the shorter operand is read by every XCD, mostly from the Infinity Cache)
   const double operands = (std::max(m, n) + 4.0 * std::min(m, n)) * k * size;
-  const double uneven = wgs > cus ? std::max(1.0, rounds * cus / wgs) : 1.0;
-  const double stream = operands / (kStreamBytesPerNs * wgs / (wgs + 60)) * uneven;
-  return kNsLaunch + std::max(1.0, rounds) * kNsRound +
-         std::max(std::max(1.0, rounds) * std::max(copies, mfma), stream) +
-         (splits > 1 ? kNsSum + 8.0 * splits * m * n / 2500 : 0.0);
+  const double uneven = std::max(1.0, rounds * cus / std::max<double>(wgs, cus));
+  const double asked = wgs / (wgs + (sizeof(T) == 2 ? 25 : 60));
+  const double stream = operands / (kStreamBytesPerNs * asked) * uneven;
+  return kNsLaunch + starts * kNsRound + std::max(rounds * std::max(copies, mfma), stream) +
+         (splits > 1 ? kNsSum + 8.0 * splits * m * n / kPartialBytesPerNs : 0.0);
 }
 
 // The 128 x 128 tiles, split along K where tail_plan would, or one round of
@@ -2481,7 +2482,7 @@ double small_tiles_ns(int m, int n, int k, int cus, const TailPlan& tail) {
   const double copies = 256 * depth * sizeof(T) / (rounds > 1 ? 70 : 55);
   const double mfma = sizeof(T) == 4 ? depth * 59 : 0.0;
   return 3000 + rounds * std::max(copies, mfma) +
-         (splits > 1 ? kNsSum + splits * tiles * 131072.0 / kStreamBytesPerNs : 0.0);
+         (splits > 1 ? kNsSum + splits * tiles * 131072.0 / kTilePartialBytesPerNs : 0.0);
 }
 
 // ksplit_kernel's plan for shapes it is the fastest estimate for (fm == 0:
