@@ -1810,10 +1810,11 @@ void ksplit_kernel(const T* __restrict__ A, const T* __restrict__ B, float* __re
     if (b_end) b_end_value = B[static_cast<std::size_t>(K) * N - 1];
   }
 
-  // Four wavefronts have registers for two sets of sums, one per stage: the
-  // chains of additions are then as short as eight wavefronts' (fp16 300 x
-  // 4096 x 4096, error against 64 bits: 2.1e-7 with one set).
-  constexpr int kSets = kWaves == 4 ? 2 : 1;
+  // Two or four sets of sums, taken in turn, where the registers hold them:
+  // chains of additions as short as the kernels' before (error against 64
+  // bits, fp16 300 x 4096 x 4096: 2.1e-7 with one set, 1.5e-7 with two, 1.9e-7
+  // before; 7 x 8960 x 11456: @@E@@).
+  constexpr int kSets = FM <= 2 ? 4 : (kWaves == 4 || FM <= 5) ? 2 : 1;
   floatx4 sums[kSets][FM][kFN];
 #pragma unroll
   for (int q = 0; q < kSets; ++q)
@@ -1912,18 +1913,26 @@ void ksplit_kernel(const T* __restrict__ A, const T* __restrict__ B, float* __re
   int s = wave;
   issue(st0, s);
   issue(st1, s + kWaves);
+  if constexpr (kSets == 4) {
+    for (; s + 3 * kWaves < steps; s += 4 * kWaves) {
+      tile(st0, s, sums[0]);
+      tile(st1, s + kWaves, sums[1]);
+      tile(st0, s + 2 * kWaves, sums[2]);
+      tile(st1, s + 3 * kWaves, sums[3]);
+    }
+  }
   for (; s + kWaves < steps; s += 2 * kWaves) {
     tile(st0, s, sums[0]);
-    tile(st1, s + kWaves, sums[kSets - 1]);
+    tile(st1, s + kWaves, sums[kSets > 1]);
   }
   if (s < steps) tile(st0, s, sums[0]);
   floatx4 (&acc)[FM][kFN] = sums[0];
-  if constexpr (kSets == 2) {
+#pragma unroll
+  for (int q = 1; q < kSets; ++q)
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int j = 0; j < kFN; ++j) acc[i][j] += sums[1][i][j];
-  }
+      for (int j = 0; j < kFN; ++j) acc[i][j] += sums[q][i][j];
 
   // Sum of the wavefronts' partial tiles through LDS: of eight, 4-7 hand
   // theirs to 0-3 first; the four sums are added in order on the way out.
@@ -2438,9 +2447,11 @@ TailPlan tail_plan(int m, int n, int k, std::size_t capacity) {
 // workgroups; fp32 tiles cost their matrix-core time, 4.1 ns per 16 rows
 // and k of a 64-column tile. Rows off 64 bytes straddle twice the lines.
 // The operands' stream from memory grows with the workgroups that ask for it
-// (towards 8000 bytes/ns); partial sums cost a launch and their traffic.
+// (towards 5500 bytes/ns, or 8000 where they fit the Infinity Cache several
+// times over); partial sums cost a launch and their traffic.
 constexpr double kNsLaunch = 1000, kNsRound = 2500, kNsSum = 2300;
-constexpr double kTileBytesPerNs = 75, kOffLineFactor = 1.8, kStreamBytesPerNs = 8000;
+constexpr double kTileBytesPerNs = 75, kOffLineFactor = 1.8;
+constexpr double kCacheBytesPerNs = 8000, kMemoryBytesPerNs = 5500, kCachedUpTo = 80e6;
 constexpr double kPartialBytesPerNs = 2500, kTilePartialBytesPerNs = 4500;
 
 template <typename T>
@@ -2457,9 +2468,11 @@ double ksplit_ns(int fm, int splits, int m, int n, int k, int cus) {
   const double mfma = sizeof(T) == 4 ? fm * static_cast<double>(k) / splits * 4.1 : 0.0;
   // (the shorter operand is read by every XCD, mostly from the Infinity Cache)
   const double operands = (std::max(m, n) + 4.0 * std::min(m, n)) * k * size;
-  const double uneven = std::max(1.0, rounds * cus / std::max<double>(wgs, cus));
-  const double asked = wgs / (wgs + (sizeof(T) == 2 ? 25 : 60));
-  const double stream = operands / (kStreamBytesPerNs * asked) * uneven;
+  const bool cached = operands < kCachedUpTo;
+  const double asked = wgs / (wgs + (cached && sizeof(T) == 2 ? 25 : 60));
+  const double uneven = std::sqrt(std::max(1.0, rounds * cus / std::max<double>(wgs, cus)));
+  const double stream =
+      operands / ((cached ? kCacheBytesPerNs : kMemoryBytesPerNs) * asked) * uneven;
   return kNsLaunch + starts * kNsRound + std::max(rounds * std::max(copies, mfma), stream) +
          (splits > 1 ? kNsSum + 8.0 * splits * m * n / kPartialBytesPerNs : 0.0);
 }
