@@ -1813,7 +1813,8 @@ void ksplit_kernel(const T* __restrict__ A, const T* __restrict__ B, float* __re
   // Two or four sets of sums, taken in turn, where the registers hold them:
   // chains of additions as short as the kernels' before (error against 64
   // bits, fp16 300 x 4096 x 4096: 2.1e-7 with one set, 1.5e-7 with two, 1.9e-7
-  // before; 7 x 8960 x 11456: @@E@@).
+  // before; 7 x 8960 x 11456
+  // 2.5e-7 with one, 1.1e-7 with four, 1.3e-7 before).
   constexpr int kSets = FM <= 2 ? 4 : (kWaves == 4 || FM <= 5) ? 2 : 1;
   floatx4 sums[kSets][FM][kFN];
 #pragma unroll
@@ -2358,15 +2359,15 @@ struct DmaTiles<float> {
 };
 
 // Rows of the tiles that cover an fp16 grid in one round when 256 x 256 ones
-// would leave CUs idle: 128 (x 256) for more than half a round and at most
-// one of them, else 192 likewise, else 0 (neither). One workgroup per CU, so
+// would leave CUs idle: 128 (x 256) where that is at most one round but a
+// round or more of 128 x 128 tiles, else 192 likewise, else 0 (neither). One workgroup per CU, so
 // the round's time falls with the tile. Measured on MI355X (us, 256 x 256 /
 // 192 x 256 / 128 x 256 / 128 x 128 tiles, on a slow box): 2048 x 4096 x
 // 4096 77 / 69 / 67 / 77, 1280 x 4096 x 4096 72 / 62 / 57 / 67, 3000^3 70 /
 // 64 / 106 / 93, 1536 x 8192 x 4096 106 / 100 / 155 / 130, 3072 x 4096 x
-// 4096 108 / 101 / 121 / 114. Half a round or less of 128 x 256 tiles leaves
-// a CU per 128 x 128 tile, whose copies are then faster (1000 x 4096 x 4096
-// 40). Against the tiles chosen before (us): 3000^3 93.8 -> 62.5, 2048 x 4096
+// 4096 108 / 101 / 121 / 114. Less than a round of 128 x 128 tiles splits K (1316 x
+// 2880 x 3062 48.8 against 52.5 on 128 x 256), and a round of them has faster
+// copies (1000 x 4096 x 4096 40). Against the tiles chosen before (us): 3000^3 93.8 -> 62.5, 2048 x 4096
 // x 4096 74.3 -> 64.3, 1500 x 6000 x 700 30.9 -> 22.3, 2000 x 3000 x 512 17.6
 // -> 14.5, 1536 x 8192 x 4096 106.3 -> 99.5. (The tiles of a partly filled
 // last round as 128 x 256 halves in a second launch lost: 2000 x 11008 x 4096
@@ -2376,7 +2377,8 @@ int one_round_rows(int m, int n) {
   const long long cols = (n + 255) / 256;
   const long long tiles128 = (m + 127) / 128 * cols, tiles192 = (m + 191) / 192 * cols;
   // (not where 256-column tiles pad N by over a tenth more than 128-column ones)
-  if (tiles128 <= cus / 2 || 20 * cols > 11LL * ((n + 127) / 128)) return 0;
+  const long long small = (m + 127LL) / 128 * ((n + 127) / 128);
+  if (small < cus || 20 * cols > 11LL * ((n + 127) / 128)) return 0;
   if (tiles128 <= cus) return 128;
   return tiles192 <= cus ? 192 : 0;
 }
