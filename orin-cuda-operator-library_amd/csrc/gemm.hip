@@ -2374,8 +2374,8 @@ struct DmaTiles<float> {
 // 188 -> 203.)
 int one_round_rows(int m, int n) {
   const long long cus = device_cus();
-  const long long cols = (n + 255) / 256;
-  const long long tiles128 = (m + 127) / 128 * cols, tiles192 = (m + 191) / 192 * cols;
+  const long long cols = (n + 255LL) / 256;
+  const long long tiles128 = (m + 127LL) / 128 * cols, tiles192 = (m + 191LL) / 192 * cols;
   // (not where 256-column tiles pad N by over a tenth more than 128-column ones)
   const long long small = (m + 127LL) / 128 * ((n + 127) / 128);
   if (small < cus || 20 * cols > 11LL * ((n + 127) / 128)) return 0;

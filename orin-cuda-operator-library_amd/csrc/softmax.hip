@@ -58,6 +58,19 @@ __device__ __forceinline__ float exp_shift_sum(float (&x)[N], float m) {
   return sum;
 }
 
+// The same with four running sums (rows of a whole workgroup, up to 64 values
+// per thread): chains as short as the split rows' 8 to 16 values.
+template <int N>
+__device__ __forceinline__ float exp_shift_sum4(float (&x)[N], float m) {
+  float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    x[i] = opl::fast_exp2((x[i] - m) * kLog2e);
+    sum[i % 4] += x[i];
+  }
+  return (sum[0] + sum[1]) + (sum[2] + sum[3]);
+}
+
 template <int N>
 __device__ __forceinline__ void scale(float (&x)[N], float s) {
 #pragma unroll
@@ -90,7 +103,7 @@ __global__ __launch_bounds__(opl::kRowBlockThreads) void softmax_block_kernel(
   const float m = opl::block_reduce<opl::MaxOp, opl::kRowBlockWaves>(
       local_max(s.x), max_slots);
   const float sum = opl::block_reduce<opl::SumOp, opl::kRowBlockWaves>(
-      exp_shift_sum(s.x, m), sum_slots);
+      exp_shift_sum4(s.x, m), sum_slots);
   scale(s.x, 1.0f / sum);
   s.store(output + offset, cols, threadIdx.x);
 }
@@ -437,7 +450,7 @@ int softmax_launch(const T* input, T* output, int rows, int cols,
   const std::size_t bytes = split_bytes(rows, split);
   if (src.workspace_mode && !opl::workspace_ok(src.data, src.bytes, bytes))
     return hipErrorInvalidValue;
-  if (split.segments > 0) {
+  if (split.run<T>(cols, opl::same_phase16(input, output))) {
     // 8 bytes per (row, segment): fewer than 2 * kSplitTargetBlocks pairs
     // for split rows, one per row otherwise (a matrix that fits in HBM has
     // far fewer rows than the arena holds pairs).

@@ -195,6 +195,32 @@ def test_softmax_masked_rows(hip, shape):
     assert np.all(y[x == -np.inf] == 0.0)
 
 
+# A few rows of 4097 to 32768 columns: one workgroup per row up to 24576 fp32
+# columns (16384 when input and output phases differ), split above. Both
+# sides of those widths and of the powers of two that set a thread's share.
+FEW_ROWS = [(1, 4097), (3, 8192), (16, 8193), (2, 16384), (5, 16385), (2, 24576), (2, 24577),
+            (1, 32767)]
+
+
+@pytest.mark.parametrize("shape", FEW_ROWS)
+@pytest.mark.parametrize("in_off,out_off", [(0, 0), (3, 3), (1, 0)])
+def test_few_long_rows(lib, shape, in_off, out_off):
+    """Softmax (one row -inf but for its last column: every other value is 0)
+    and RMSNorm against the oracle at the operators' tolerance."""
+    from gpu_util import to_device
+    rows, cols = shape
+    x = oracle.normal(240 + cols % 991, shape, 0.0, 3.0)
+    x[rows - 1, :cols - 1] = -np.inf
+    y = _rows_call(lib, "operatorlib_softmax_f32", x, in_off, out_off)
+    elem, norm = rel_errors(y, oracle.softmax(x))
+    assert elem <= 1e-5 and norm <= 1e-5, (elem, norm)
+    x = oracle.normal(241, shape)
+    w = oracle.uniform(242, cols, 0.5, 1.5)
+    y = _rows_call(lib, "operatorlib_rmsnorm_f32", x, in_off, out_off, to_device(w), 1e-6)
+    elem, norm = rel_errors(y, oracle.rmsnorm(x, w, 1e-6))
+    assert elem <= 1e-5 and norm <= 1e-5, (elem, norm)
+
+
 # Input and output in different 16-byte phases (rows cannot share one
 # float4 layout): the element-wise paths. The weight of RMSNorm may sit at
 # any alignment on every path.
