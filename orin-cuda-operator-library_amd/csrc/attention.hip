@@ -666,7 +666,8 @@ constexpr float kLazyLog2 = 8.0f;
 
 // K/V tile layout in LDS for element type T (rows keep their global
 // layout, D elements each).
-template <typename T, int D, int kTileKeys>
+// Dc: the dims computed with (D, or 96 in rows of 128).
+template <typename T, int D, int kTileKeys, int Dc = D>
 struct Layout {
   static constexpr int kSize = static_cast<int>(sizeof(T));
   static constexpr int kElems = 16 / kSize;  // elements per 16-byte chunk
@@ -677,8 +678,8 @@ struct Layout {
   // QK^T fragment steps over d: one 16-byte chunk per lane group covers 32
   // fp16 dims (one MFMA 16x16x32) or 16 fp32 dims (four MFMA 16x16x4).
   static constexpr int kSubK = 4 * kElems;
-  static constexpr int kSteps = D / kSubK;
-  static constexpr int kDBlocks = D / 16;  // 16-dim blocks of O^T
+  static constexpr int kSteps = Dc / kSubK;
+  static constexpr int kDBlocks = Dc / 16;  // 16-dim blocks of O^T
   // K rows: 16 consecutive rows read one logical chunk (one 16-lane group)
   // and land on 16 different physical chunks.
   __device__ static int swizzle_k(int row) {
@@ -697,11 +698,12 @@ struct Layout {
   }
 };
 
-// Scores of one 32-key half for a wavefront's 32 query rows: [kb][qc] is
+// Scores of one 32-key half for a wavefront's 16 kQ query rows: [kb][qc] is
 // the 16 x 16 block of keys 16 kb.. and queries 16 qc.. (S^T layout: lane l
 // holds query l % 16, keys 4 (l / 16) + e).
+template <int kQ>
 struct HalfScores {
-  floatx4 v[2][2];
+  floatx4 v[2][kQ];
 };
 
 // kGroups > 1 (small grids): kGroups groups of kW wavefronts share the
@@ -709,8 +711,8 @@ struct HalfScores {
 // each group with its own K/V stages; at the end the groups merge their
 // (O, max, sum) through LDS in group order, every wavefront taking a share
 // of the rows.
-// kW = wavefronts per group, 32 query rows each: 4 (128-row blocks), or 2
-// (64-row blocks) for the smallest grids, whose 128-row blocks would leave
+// kW = wavefronts per group, 32 query rows each: 4 (128-row blocks), or 2 or 1
+// (64- or 32-row blocks) for the smallest grids, whose 128-row blocks would leave
 // CUs idle.
 // kTileKeys = keys per K/V tile: 64 (two 32-key halves per tile), or 32,
 // which halves the stages so that four groups fit the LDS of two.
@@ -731,17 +733,20 @@ template <typename T, int D, int kGroups, int kW, int kTileKeys>
 constexpr int kMinWavesPerSimd =
     2 * kGroups * Layout<T, D, kTileKeys>::kStage > 80 * 1024 && kGroups * kW == 4 ? 1 : 2;
 
-template <typename T, int D, int kGroups, int kW, int kTileKeys>
+// kQ: 16-row query blocks per wavefront, 2 except in the fp32 D = 64
+// instances of one wavefront per group.
+template <typename T, int D, int kGroups, int kW, int kTileKeys, int Dc = D, int kQ = 2>
 __global__ __launch_bounds__(kW * opl::kWaveSize * kGroups)
 __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<T, D, kGroups, kW, kTileKeys>, 2)))
 void attention_dma_kernel(const T* __restrict__ Q, const T* __restrict__ K,
                           const T* __restrict__ V, float* __restrict__ O, int BH, int S,
                           int dm, int causal, float score_scale_log2) {
-  using L = Layout<T, D, kTileKeys>;
+  using L = Layout<T, D, kTileKeys, Dc>;
+  constexpr int kRowsPerWave = 16 * kQ;
   constexpr bool kHalf = L::kSize == 2;
   using Frag = typename std::conditional<kHalf, half8, floatx4>::type;
   static_assert(kGroups == 1 || kGroups == 2 || kGroups == 4, "1, 2 or 4 key groups");
-  static_assert(kW == 2 || kW == 4, "2 or 4 wavefronts per group");
+  static_assert(kW == 1 || kW == 2 || kW == 4, "1, 2 or 4 wavefronts per group");
   static_assert(kTileKeys == 32 || kTileKeys == 64, "32- or 64-key tiles");
   constexpr int kRows = kW * kRowsPerWave;  // query rows per workgroup
   // 16-byte copies per lane and tile: the group's lanes share each tile
@@ -810,9 +815,9 @@ void attention_dma_kernel(const T* __restrict__ Q, const T* __restrict__ K,
 
   // Q^T operand of query block qc: query wave_row0 + 16 qc + col, the
   // 16-byte chunk quad of step c (dims kSubK c + kElems quad ..).
-  Frag qf[2][L::kSteps];
+  Frag qf[kQ][L::kSteps];
 #pragma unroll
-  for (int qc = 0; qc < 2; ++qc)
+  for (int qc = 0; qc < kQ; ++qc)
 #pragma unroll
     for (int c = 0; c < L::kSteps; ++c) {
       const int dim = L::kSubK * c + L::kElems * quad;
@@ -894,18 +899,23 @@ void attention_dma_kernel(const T* __restrict__ Q, const T* __restrict__ K,
 
   // O^T of query block qc, dim block db: lane l holds query 16 qc + col,
   // dims 16 db + 4 quad + e.
-  floatx4 o[2][L::kDBlocks];
+  floatx4 o[kQ][L::kDBlocks];
 #pragma unroll
-  for (int qc = 0; qc < 2; ++qc)
+  for (int qc = 0; qc < kQ; ++qc)
 #pragma unroll
     for (int db = 0; db < L::kDBlocks; ++db)
 #pragma unroll
       for (int e = 0; e < 4; ++e) o[qc][db][e] = 0.0f;
-  // Online-softmax state of the lane's two query rows.
-  float row_max[2] = {-FLT_MAX, -FLT_MAX};
+  // Online-softmax state of the lane's query rows.
+  float row_max[kQ];
   // Raw score above which the running max must move; -inf until the first
   // visible score.
-  float move_above[2] = {-INFINITY, -INFINITY};
+  float move_above[kQ];
+#pragma unroll
+  for (int qc = 0; qc < kQ; ++qc) {
+    row_max[qc] = -FLT_MAX;
+    move_above[qc] = -INFINITY;
+  }
   // Row sums on the matrix cores: an all-ones A operand times P^T gives
   // every accumulator row the column sums of P^T, i.e. each lane the full
   // sum of its query row's p (as rounded to fp16 for P.V) in all four
@@ -914,12 +924,12 @@ void attention_dma_kernel(const T* __restrict__ Q, const T* __restrict__ K,
   // fp32 keeps them on the vector ALUs instead (the matrix cores are its
   // busier pipe): each lane sums its 8 of the row's p per 32 keys, and the
   // four lanes of a row are combined once, after the loop.
-  floatx4 sums[2];
+  floatx4 sums[kQ];
 #pragma unroll
-  for (int qc = 0; qc < 2; ++qc)
+  for (int qc = 0; qc < kQ; ++qc)
 #pragma unroll
     for (int e = 0; e < 4; ++e) sums[qc][e] = 0.0f;
-  float lane_sum[2] = {0.0f, 0.0f};
+  float lane_sum[kQ] = {};
   half8 ones;
 #pragma unroll
   for (int e = 0; e < 8; ++e) ones[e] = static_cast<_Float16>(1.0f);
@@ -947,11 +957,11 @@ void attention_dma_kernel(const T* __restrict__ Q, const T* __restrict__ K,
       // halves (vector ALUs), and the scheduler can interleave them. A
       // 32-key tile is one such half.
       auto scores = [&](int j) {
-        HalfScores s;
+        HalfScores<kQ> s;
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-          for (int qc = 0; qc < 2; ++qc)
+          for (int qc = 0; qc < kQ; ++qc)
 #pragma unroll
             for (int e = 0; e < 4; ++e) s.v[kb][qc][e] = 0.0f;
         if constexpr (kHalf) {
@@ -971,7 +981,7 @@ void attention_dma_kernel(const T* __restrict__ Q, const T* __restrict__ K,
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-              for (int qc = 0; qc < 2; ++qc)
+              for (int qc = 0; qc < kQ; ++qc)
                 s.v[kb][qc] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
                     a[kb][c], qf[qc][c], s.v[kb][qc], 0, 0, 0);
         } else {
@@ -989,18 +999,18 @@ void attention_dma_kernel(const T* __restrict__ Q, const T* __restrict__ K,
 #pragma unroll
               for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-                for (int qc = 0; qc < 2; ++qc)
+                for (int qc = 0; qc < kQ; ++qc)
                   s.v[kb][qc] = __builtin_amdgcn_mfma_f32_16x16x4f32(
                       a[kb][e], qf[qc][c][e], s.v[kb][qc], 0, 0, 0);
           }
         }
         return s;
       };
-      auto mask = [&](HalfScores& s, int j) {
+      auto mask = [&](HalfScores<kQ>& s, int j) {
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-          for (int qc = 0; qc < 2; ++qc)
+          for (int qc = 0; qc < kQ; ++qc)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
               const int key = key0 + 32 * j + 16 * kb + 4 * quad + e;
@@ -1011,7 +1021,7 @@ void attention_dma_kernel(const T* __restrict__ Q, const T* __restrict__ K,
       // Max of this lane's 8 raw scores of query block qc in a half. The
       // row's other 24 sit in lanes l ^ 16, l ^ 32, l ^ 48; they are
       // combined only when the max has to move (move_max).
-      auto lane_max = [&](const HalfScores& s, int qc) {
+      auto lane_max = [&](const HalfScores<kQ>& s, int qc) {
         float m = s.v[0][qc][0];
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
@@ -1026,16 +1036,17 @@ void attention_dma_kernel(const T* __restrict__ Q, const T* __restrict__ K,
       // skipped on almost every half-tile. Softmax is shift-invariant: the
       // result is the same up to rounding. The test compares raw scores
       // with move_above = (m + kLazyLog2) / scale, updated when m moves.
-      auto needs_move = [&](float raw0, float raw1) {
-        return __builtin_amdgcn_ballot_w64(raw0 > move_above[0] ||
-                                           raw1 > move_above[1]) != 0;
+      auto needs_move = [&](const float (&raw)[kQ]) {
+        bool move = false;
+#pragma unroll
+        for (int qc = 0; qc < kQ; ++qc) move |= raw[qc] > move_above[qc];
+        return __builtin_amdgcn_ballot_w64(move) != 0;
       };
       // Wave-uniform branch: every lane runs it, and the four lanes of a
       // row combine their maxima, so they move to the same max.
-      auto move_max = [&](float raw0, float raw1) {
-        const float lane_raw[2] = {raw0, raw1};
+      auto move_max = [&](const float (&lane_raw)[kQ]) {
 #pragma unroll
-        for (int qc = 0; qc < 2; ++qc) {
+        for (int qc = 0; qc < kQ; ++qc) {
           const float raw = opl::max_lane_xor32(
               opl::combine_xor16_f32<opl::MaxOp>(lane_raw[qc]));
           const float new_max = fmaxf(row_max[qc], raw * score_scale_log2);
@@ -1058,10 +1069,10 @@ void attention_dma_kernel(const T* __restrict__ Q, const T* __restrict__ K,
       // + e are keys 4 quad + e of block 0, slots 8 quad + 4 + e those of
       // block 1. fp32: [qc][kb][e] is key 16 kb + 4 quad + e, the operand of
       // MFMA e over key block kb; the lane's sum of them is kept.
-      using PHalf = typename std::conditional<kHalf, half8[2], floatx4[2][2]>::type;
-      auto exponentiate = [&](const HalfScores& s, PHalf& pb) {
+      using PHalf = typename std::conditional<kHalf, half8[kQ], floatx4[kQ][2]>::type;
+      auto exponentiate = [&](const HalfScores<kQ>& s, PHalf& pb) {
 #pragma unroll
-        for (int qc = 0; qc < 2; ++qc)
+        for (int qc = 0; qc < kQ; ++qc)
 #pragma unroll
           for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -1092,7 +1103,7 @@ void attention_dma_kernel(const T* __restrict__ Q, const T* __restrict__ K,
 #pragma unroll
               for (int db = 0; db < L::kDBlocks; ++db)
 #pragma unroll
-                for (int qc = 0; qc < 2; ++qc)
+                for (int qc = 0; qc < kQ; ++qc)
                   o[qc][db] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[db], pb[qc][kb][e],
                                                                    o[qc][db], 0, 0, 0);
             }
@@ -1110,11 +1121,11 @@ void attention_dma_kernel(const T* __restrict__ Q, const T* __restrict__ K,
               a[4 + e] = hi[e];
             }
 #pragma unroll
-            for (int qc = 0; qc < 2; ++qc)
+            for (int qc = 0; qc < kQ; ++qc)
               o[qc][db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, pb[qc], o[qc][db], 0, 0, 0);
           }
 #pragma unroll
-          for (int qc = 0; qc < 2; ++qc)
+          for (int qc = 0; qc < kQ; ++qc)
             sums[qc] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, pb[qc], sums[qc], 0, 0, 0);
         }
       };
@@ -1135,19 +1146,21 @@ void attention_dma_kernel(const T* __restrict__ Q, const T* __restrict__ K,
         // 2127 / 262.5 with the same instruction order and no priority;
         // priority 3 instead of 1: 2091 / 258.8. Results bit-identical.
         __builtin_amdgcn_s_setprio(1);
-        HalfScores s0 = scores(0);
-        HalfScores s1;
+        HalfScores<kQ> s0 = scores(0);
+        HalfScores<kQ> s1;
         if constexpr (kTileKeys == 64) s1 = scores(1);
         __builtin_amdgcn_s_setprio(0);
         if constexpr (kMasked) mask(s0, 0);
-        float a0 = lane_max(s0, 0);
-        float a1 = lane_max(s0, 1);
+        float raw[kQ];
+#pragma unroll
+        for (int qc = 0; qc < kQ; ++qc) raw[qc] = lane_max(s0, qc);
         if constexpr (kTileKeys == 64) {
           if constexpr (kMasked) mask(s1, 1);
-          a0 = __builtin_elementwise_maximum(a0, lane_max(s1, 0));
-          a1 = __builtin_elementwise_maximum(a1, lane_max(s1, 1));
+#pragma unroll
+          for (int qc = 0; qc < kQ; ++qc)
+            raw[qc] = __builtin_elementwise_maximum(raw[qc], lane_max(s1, qc));
         }
-        if (needs_move(a0, a1)) move_max(a0, a1);
+        if (needs_move(raw)) move_max(raw);
         exponentiate(s0, p0);
         accumulate(0, p0);
         if constexpr (kTileKeys == 64) {
@@ -1175,9 +1188,9 @@ void attention_dma_kernel(const T* __restrict__ Q, const T* __restrict__ K,
     tile(st1, st0, i + 1);
   }
   if (i < iters) tile(st0, st1, i);
-  float row_sum[2];
+  float row_sum[kQ];
 #pragma unroll
-  for (int qc = 0; qc < 2; ++qc) {
+  for (int qc = 0; qc < kQ; ++qc) {
     if constexpr (kHalf)
       row_sum[qc] = sums[qc][0];
     else  // the four lanes of the row: l, l ^ 16, l ^ 32, l ^ 48
@@ -1185,15 +1198,16 @@ void attention_dma_kernel(const T* __restrict__ Q, const T* __restrict__ K,
   }
 
   // After the loop every stage is free (the last iteration ended with a
-  // barrier and issued no copy). Merge and staging blocks tile the two
-  // stage arrays: block (g, w) holds wavefront w of group g's 32 rows of O,
-  // 32 * D floats.
-  constexpr int kBlockBytes = 2 * L::kDBlocks * 16 * opl::kWaveSize;
-  static_assert(kArray % kBlockBytes == 0 && kW * kBlockBytes <= 2 * kArray,
-                "blocks tile the two stage arrays");
+  // barrier and issued no copy). Merge and staging blocks lie in the two
+  // stage arrays: block (g, w) holds wavefront w of group g's rows of O,
+  // kRowsPerWave * D floats.
+  constexpr int kBlockBytes = kRowsPerWave * D * 4;
+  constexpr int kPerArray = kArray / kBlockBytes;
+  static_assert(kPerArray >= 1 && kGroups * kW <= 2 * kPerArray, "blocks fit the stage arrays");
   auto block = [&](int index) -> float4* {
-    const int byte = index * kBlockBytes;
-    return reinterpret_cast<float4*>(byte < kArray ? stage0 + byte : stage1 + (byte - kArray));
+    return reinterpret_cast<float4*>(index < kPerArray
+                                         ? stage0 + index * kBlockBytes
+                                         : stage1 + (index - kPerArray) * kBlockBytes);
   };
   // Key-split groups (kGroups > 1): every wavefront merges and stores a
   // share of the rows. (1) Each writes its rows' (max, sum) to LDS; (2)
@@ -1212,20 +1226,20 @@ void attention_dma_kernel(const T* __restrict__ Q, const T* __restrict__ K,
     float* const xs = reinterpret_cast<float*>(stage0);
     const int slot = (group * kW + wave) * opl::kWaveSize + lane;
 #pragma unroll
-    for (int qc = 0; qc < 2; ++qc) {
+    for (int qc = 0; qc < kQ; ++qc) {
       xs[qc * kSlots + slot] = row_max[qc];
-      xs[(2 + qc) * kSlots + slot] = row_sum[qc];
+      xs[(kQ + qc) * kSlots + slot] = row_sum[qc];
     }
     __syncthreads();
-    float coef[2];
+    float coef[kQ];
 #pragma unroll
-    for (int qc = 0; qc < 2; ++qc) {
+    for (int qc = 0; qc < kQ; ++qc) {
       float mg[kGroups], lg[kGroups];
 #pragma unroll
       for (int g = 0; g < kGroups; ++g) {
         const int sl = (g * kW + wave) * opl::kWaveSize + lane;
         mg[g] = xs[qc * kSlots + sl];
-        lg[g] = xs[(2 + qc) * kSlots + sl];
+        lg[g] = xs[(kQ + qc) * kSlots + sl];
       }
       float m = mg[0];
 #pragma unroll
@@ -1240,7 +1254,7 @@ void attention_dma_kernel(const T* __restrict__ Q, const T* __restrict__ K,
     {
       float4* const stg = block(group * kW + wave);
 #pragma unroll
-      for (int qc = 0; qc < 2; ++qc)
+      for (int qc = 0; qc < kQ; ++qc)
 #pragma unroll
         for (int db = 0; db < L::kDBlocks; ++db) {
           const int r = 16 * qc + col;
@@ -1287,15 +1301,15 @@ void attention_dma_kernel(const T* __restrict__ Q, const T* __restrict__ K,
   // 64 / (D / 4) whole rows. Float4 c of row r sits at position
   // c ^ (r % (D / 4)): both the writes (16 rows, one float4 position each)
   // and the reads (one row per 32 or 16 lanes) spread over the banks.
-  float inv[2];
+  float inv[kQ];
 #pragma unroll
-  for (int qc = 0; qc < 2; ++qc)
+  for (int qc = 0; qc < kQ; ++qc)
     inv[qc] = 1.0f / row_sum[qc];
   {
     constexpr int kChunks4 = D / 4;  // float4s per output row
     float4* const stg = block(wave);
 #pragma unroll
-    for (int qc = 0; qc < 2; ++qc)
+    for (int qc = 0; qc < kQ; ++qc)
 #pragma unroll
       for (int db = 0; db < L::kDBlocks; ++db) {
         const int r = 16 * qc + col;
@@ -1320,6 +1334,115 @@ void attention_dma_kernel(const T* __restrict__ Q, const T* __restrict__ K,
 }
 
 #undef OPL_LDS
+
+// One launch of an instance: rows of 16 kQ kW query rows per workgroup, a
+// multiple of 8 workgroups (one contiguous range of work per XCD).
+template <typename T, int D, int kGroups, int kW, int kTileKeys, int Dc = D, int kQ = 2>
+void launch_instance(const T* q, const T* k, const T* v, float* out, int bh, int s, int dm,
+                     int causal, float scale, hipStream_t stream) {
+  constexpr int kRows = 16 * kQ * kW;
+  const long long wgs = (s + kRows - 1LL) / kRows * bh;
+  const dim3 grid(static_cast<unsigned>((wgs + kXcds - 1) / kXcds * kXcds));
+  attention_dma_kernel<T, D, kGroups, kW, kTileKeys, Dc, kQ>
+      <<<grid, dim3(kGroups * kW * opl::kWaveSize), 0, stream>>>(q, k, v, out, bh, s, dm, causal,
+                                                               scale);
+}
+
+// Blocks of 32 rows on four key groups of one wavefront each, while their
+// grid is one round (a CU each): four times the CUs of 128-row blocks, and no
+// two wavefronts wait for each other's tile. Measured on MI355X (us, 64-row
+// blocks before -> 32-row; non-causal / causal): fp16 D128 B1 H12 S128 7.9 ->
+// 6.4 / 8.4 -> 7.0, B1 H32 S256 9.5 -> 8.4 / 10.6 -> 9.3, B1 H12 S512 11.6 ->
+// 11.0 / 12.6 -> 11.7, S1000 17.2 -> 30.8; D64 S512 8.0 -> 7.4 / 8.9 -> 7.7;
+// fp32 D64 S128 9.4 -> 7.4 / 10.4 -> 8.1, S512 24.1 -> 16.7 / 24.9 -> 17.1.
+// fp16 stops at 512 tokens (the K and V of a head are fetched once per block).
+constexpr long long kOneRound = 256;
+constexpr int kThirtyTwoRowsUpTo = 512;
+// fp32 D64 causal grids from 512 tokens gain up to three rounds, as the blocks
+// are ordered heaviest first: B1 H12 S1000 (384) 43.3 -> 34.8, B1 H8 S2048
+// (512) 81.3 -> 56.9, B1 H32 S700 (704) 44.9 -> 40.2, B2 H16 S1024 (1024) 57.1
+// -> 65.7; B8 H16 S128 (512) 12.1 -> 14.9. 64 tokens (two tiles for four
+// groups) lose: B1 H8 6.9 -> 7.0.
+constexpr long long kThirtyTwoRowsCausalF32 = 768;
+// fp16 D64, 64-row blocks of one round: four groups of two wavefronts on
+// 32-key tiles instead of two on 64-key ones from this many tokens: B1 H12
+// S1024 11.9 -> 11.0, B1 H8 S2048 19.0 -> 16.9, causal 19.6 -> 17.8; S512 8.0
+// -> 8.1.
+constexpr int kFourGroupsFrom = 768;
+
+// Chooses the instance. `blocks`: 128-row query blocks. Grids too small to
+// fill the CUs split each query block's keys between groups of wavefronts in
+// the workgroup; the smallest also take 64- or 32-row blocks.
+template <typename T>
+void launch(const T* q, const T* k, const T* v, float* out, int bh, int s, int dm, int causal,
+            float scale, long long blocks, hipStream_t stream) {
+  const bool wide = dm > 64;  // 128-dim LDS rows
+  // Head dims of 65..96 compute on 96 of them: fp16 B2 H32 S4096 D96 468 ->
+  // 417 us, causal 268 -> 233; B1 H12 S1024 15.9 -> 14.2.
+  const bool d96 = wide && dm <= 96;
+  const long long half_up_to =
+      wide ? kHalfRowsUpTo : (causal ? kHalfRowsUpToD64Causal : kHalfRowsUpToD64);
+  const bool half_rows = blocks <= half_up_to;
+  const bool split = half_rows || blocks < (causal ? kSplitKeysBelowCausal : kSplitKeysBelow);
+  const long long rows32 = (s + 31LL) / 32 * bh;
+  const long long rows48 = (s + 47LL) / 48 * bh;
+  const long long rows64 = (s + 63LL) / 64 * bh;
+#define OPL_RUN(...) \
+  launch_instance<T, __VA_ARGS__>(q, k, v, out, bh, s, dm, causal, scale, stream)
+  if constexpr (sizeof(T) == 2) {
+    if (rows32 <= kOneRound && s <= kThirtyTwoRowsUpTo) {
+      if (d96) OPL_RUN(128, 4, 1, 32, 96);
+      else if (wide) OPL_RUN(128, 4, 1, 32);
+      else OPL_RUN(64, 4, 1, 32);
+    } else if (s <= kShortSequence && !half_rows) {
+      if (d96) OPL_RUN(128, 1, 2, 32, 96);
+      else if (wide) OPL_RUN(128, 1, 2, 32);
+      else OPL_RUN(64, 1, 2, 32);
+    } else if (wide && half_rows) {
+      if (d96) OPL_RUN(128, 4, 2, 32, 96);
+      else OPL_RUN(128, 4, 2, 32);
+    } else if (wide && split) {
+      if (d96) OPL_RUN(128, 2, 4, 64, 96);
+      else OPL_RUN(128, 2, 4, 64);
+    } else if (wide) {
+      if (d96) OPL_RUN(128, 1, 4, 64, 96);
+      else OPL_RUN(128, 1, 4, 64);
+    } else if (rows64 <= kOneRound && s >= kFourGroupsFrom) {
+      OPL_RUN(64, 4, 2, 32);
+    } else if (half_rows) {
+      OPL_RUN(64, 2, 2, 64);  // (split implies half_rows at D = 64)
+    } else {
+      OPL_RUN(64, 1, 4, 64);
+    }
+  } else {
+    // fp32: 32-key tiles, at most two groups at D = 128 (a group's K/V stages
+    // hold 64 KiB).
+    if (!wide && s > 64 &&
+        (rows32 <= kOneRound ||
+         (causal && s >= kThirtyTwoRowsUpTo && rows32 <= kThirtyTwoRowsCausalF32))) {
+      OPL_RUN(64, 4, 1, 32);
+    } else if (!wide && s > 64 && !causal && rows48 <= kOneRound) {
+      // 48 rows per wavefront, where that is one round: B1 H12 S1000 45.3 ->
+      // 39.3 us
+      OPL_RUN(64, 4, 1, 32, 64, 3);
+    } else if (wide && half_rows) {
+      if (d96) OPL_RUN(128, 2, 2, 32, 96);
+      else OPL_RUN(128, 2, 2, 32);
+    } else if (wide && split) {
+      if (d96) OPL_RUN(128, 2, 4, 32, 96);
+      else OPL_RUN(128, 2, 4, 32);
+    } else if (wide) {
+      if (d96) OPL_RUN(128, 1, 4, 32, 96);
+      else OPL_RUN(128, 1, 4, 32);
+    } else if (half_rows) {
+      OPL_RUN(64, 2, 2, 32);
+    } else {
+      OPL_RUN(64, 1, 4, 32);
+    }
+  }
+#undef OPL_RUN
+}
+
 }  // namespace dma
 
 // True when the fast path applies: aligned tensors whose head dim is 64 or
@@ -1327,8 +1450,6 @@ void attention_dma_kernel(const T* __restrict__ Q, const T* __restrict__ K,
 // the instances of the next of 64 and 128 with the dims past it zero (its
 // K/V chunks take an out-of-range offset of 2^31 bytes, so such heads must
 // stay below that).
-inline int dma_layout(int head_dim) { return head_dim <= 64 ? 64 : 128; }
-
 inline bool dma_ok(const void* q, const void* k, const void* v, const void* out,
                    int sequence, int head_dim, unsigned element_bytes) {
   // one head of K or V must be addressable with 32-bit buffer offsets
@@ -1366,80 +1487,7 @@ int attention_entry(const T* q, const T* k, const T* v, float* out, int batch,
       return hipSuccess;
     }
     const float scale = 1.4426950408889634f / sqrtf(static_cast<float>(head_dim));
-    // Grids too small to fill the CUs split each query block's keys
-    // between groups of wavefronts in the workgroup; the smallest also
-    // halve the query block (and, fp16 at D = 128, split its keys four ways).
-    const int layout = dma_layout(head_dim);
-    const long long half_up_to =
-        layout == 128 ? dma::kHalfRowsUpTo
-                        : (causal ? dma::kHalfRowsUpToD64Causal : dma::kHalfRowsUpToD64);
-    const bool half_rows = blocks <= half_up_to;
-    const bool split = half_rows ||
-        blocks < (causal ? dma::kSplitKeysBelowCausal : dma::kSplitKeysBelow);
-    const long long wgs = half_rows ? 2 * blocks : blocks;
-    // a multiple of 8 workgroups, one contiguous range of work per XCD
-    const long long padded = (wgs + dma::kXcds - 1) / dma::kXcds * dma::kXcds;
-    const dim3 grid(static_cast<unsigned>(padded));
-    if constexpr (sizeof(T) == 2) {
-      if (sequence <= dma::kShortSequence && !half_rows) {
-        const long long tb = (sequence + 63) / 64 * static_cast<long long>(bh);
-        const long long tw = (tb + dma::kXcds - 1) / dma::kXcds * dma::kXcds;
-        const dim3 tgrid(static_cast<unsigned>(tw));
-        if (layout == 128)
-          dma::attention_dma_kernel<T, 128, 1, 2, 32><<<tgrid, dim3(kThreads / 2), 0, stream>>>(
-              q, k, v, out, bh, sequence, head_dim, c, scale);
-        else
-          dma::attention_dma_kernel<T, 64, 1, 2, 32><<<tgrid, dim3(kThreads / 2), 0, stream>>>(
-              q, k, v, out, bh, sequence, head_dim, c, scale);
-        return hipGetLastError();
-      }
-      if (layout == 128) {
-        // 64-row blocks x 4 groups / 128-row blocks x 2 groups: 8 wavefronts
-        const dim3 block(split ? 2 * kThreads : kThreads);
-        if (half_rows)
-          dma::attention_dma_kernel<T, 128, 4, 2, 32><<<grid, block, 0, stream>>>(
-              q, k, v, out, bh, sequence, head_dim, c, scale);
-        else if (split)
-          dma::attention_dma_kernel<T, 128, 2, 4, 64><<<grid, block, 0, stream>>>(
-              q, k, v, out, bh, sequence, head_dim, c, scale);
-        else
-          dma::attention_dma_kernel<T, 128, 1, 4, 64><<<grid, block, 0, stream>>>(
-              q, k, v, out, bh, sequence, head_dim, c, scale);
-      } else {
-        // (split implies half_rows at D = 64; 4 wavefronts either way)
-        const dim3 block(kThreads);
-        if (half_rows)
-          dma::attention_dma_kernel<T, 64, 2, 2, 64><<<grid, block, 0, stream>>>(
-              q, k, v, out, bh, sequence, head_dim, c, scale);
-        else
-          dma::attention_dma_kernel<T, 64, 1, 4, 64><<<grid, block, 0, stream>>>(
-              q, k, v, out, bh, sequence, head_dim, c, scale);
-      }
-    } else {
-      // fp32: 32-key tiles, at most two groups (a group's K/V stages hold
-      // 64 KiB at D = 128): 64-row blocks with two groups of 2 wavefronts,
-      // 128-row blocks with two groups of 4, or one group of 4.
-      if (layout == 128) {
-        const dim3 block(split && !half_rows ? 2 * kThreads : kThreads);
-        if (half_rows)
-          dma::attention_dma_kernel<T, 128, 2, 2, 32><<<grid, block, 0, stream>>>(
-              q, k, v, out, bh, sequence, head_dim, c, scale);
-        else if (split)
-          dma::attention_dma_kernel<T, 128, 2, 4, 32><<<grid, block, 0, stream>>>(
-              q, k, v, out, bh, sequence, head_dim, c, scale);
-        else
-          dma::attention_dma_kernel<T, 128, 1, 4, 32><<<grid, block, 0, stream>>>(
-              q, k, v, out, bh, sequence, head_dim, c, scale);
-      } else {
-        const dim3 block(kThreads);
-        if (half_rows)
-          dma::attention_dma_kernel<T, 64, 2, 2, 32><<<grid, block, 0, stream>>>(
-              q, k, v, out, bh, sequence, head_dim, c, scale);
-        else
-          dma::attention_dma_kernel<T, 64, 1, 4, 32><<<grid, block, 0, stream>>>(
-              q, k, v, out, bh, sequence, head_dim, c, scale);
-      }
-    }
+    dma::launch<T>(q, k, v, out, bh, sequence, head_dim, c, scale, blocks, stream);
     return hipGetLastError();
   }
   const int ndt = (head_dim + 31) / 32;
