@@ -943,6 +943,22 @@ void attention_dma_kernel(const T* __restrict__ Q, const T* __restrict__ K,
   const int t_begin = group * iters;
   const int t_count = kGroups == 1 ? tiles : max(0, min(iters, tiles - t_begin));
 
+  // Between tiles a group of one wavefront waits for nobody: its stages are
+  // its own. Measured on MI355X (us, workgroup barrier -> none): fp32 D64 B1
+  // H12 S1000 39.3 -> 36.2, causal (32-row blocks) 34.8 -> 33.5; fp16 D128 B1
+  // H12 S512 11.0 -> 10.5. (Groups of two meeting through counters in LDS
+  // instead of the workgroup's barrier were no faster: fp16 D128 B1 H12 S1024
+  // 17.0 both ways, causal 16.8 and 16.9.)
+  auto tile_end = [&] {
+    __builtin_amdgcn_s_waitcnt(0);  // this tile's reads and the next DMA
+    if constexpr (kW == 1) {
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+    } else {
+      __syncthreads();
+    }
+  };
+
   auto tile = [&](const unsigned char* cur, unsigned char* nxt, int i) {
     const int key0 = (t_begin + i) * kTileKeys;
     if (i + 1 < t_count) issue(nxt, key0 + kTileKeys);
@@ -1175,8 +1191,7 @@ void attention_dma_kernel(const T* __restrict__ Q, const T* __restrict__ K,
       else
         body(std::false_type{});
     }
-    __builtin_amdgcn_s_waitcnt(0);  // this tile's reads and the next DMA
-    __syncthreads();
+    tile_end();
   };
 
   if (t_count > 0) issue(st0, t_begin * kTileKeys);
@@ -1188,6 +1203,7 @@ void attention_dma_kernel(const T* __restrict__ Q, const T* __restrict__ K,
     tile(st1, st0, i + 1);
   }
   if (i < iters) tile(st0, st1, i);
+  if constexpr (kW == 1) __syncthreads();  // the merge reuses every stage
   float row_sum[kQ];
 #pragma unroll
   for (int qc = 0; qc < kQ; ++qc) {
@@ -1353,17 +1369,22 @@ void launch_instance(const T* q, const T* k, const T* v, float* out, int bh, int
 // two wavefronts wait for each other's tile. Measured on MI355X (us, 64-row
 // blocks before -> 32-row; non-causal / causal): fp16 D128 B1 H12 S128 7.9 ->
 // 6.4 / 8.4 -> 7.0, B1 H32 S256 9.5 -> 8.4 / 10.6 -> 9.3, B1 H12 S512 11.6 ->
-// 11.0 / 12.6 -> 11.7, S1000 17.2 -> 30.8; D64 S512 8.0 -> 7.4 / 8.9 -> 7.7;
-// fp32 D64 S128 9.4 -> 7.4 / 10.4 -> 8.1, S512 24.1 -> 16.7 / 24.9 -> 17.1.
-// fp16 stops at 512 tokens (the K and V of a head are fetched once per block).
+// 10.5 / 12.6 -> 11.4, B1 H4 S700 13.0 -> 12.2 / 13.9 -> 12.2, B1 H12 S1000 (384
+// blocks) 17.2 -> 29.7; D64 S512 8.0 -> 7.2 / 8.9 -> 7.5; fp32 D64 S128 9.4 ->
+// 7.4 / 10.4 -> 8.0, S512 24.1 -> 16.4 / 24.9 -> 16.7. fp16 stops at 768 tokens
+// (the K and V of a head are fetched once per block).
 constexpr long long kOneRound = 256;
-constexpr int kThirtyTwoRowsUpTo = 512;
+constexpr int kThirtyTwoRowsUpTo = 768;
 // fp32 D64 causal grids from 512 tokens gain up to three rounds, as the blocks
-// are ordered heaviest first: B1 H12 S1000 (384) 43.3 -> 34.8, B1 H8 S2048
-// (512) 81.3 -> 56.9, B1 H32 S700 (704) 44.9 -> 40.2, B2 H16 S1024 (1024) 57.1
+// are ordered heaviest first: B1 H12 S1000 (384) 43.3 -> 33.5, B1 H8 S2048
+// (512) 81.3 -> 53.0, B1 H32 S700 (704) 44.9 -> 40.2, B2 H16 S1024 (1024) 57.1
 // -> 65.7; B8 H16 S128 (512) 12.1 -> 14.9. 64 tokens (two tiles for four
 // groups) lose: B1 H8 6.9 -> 7.0.
 constexpr long long kThirtyTwoRowsCausalF32 = 768;
+constexpr int kThirtyTwoRowsCausalFrom = 512;
+// fp16 D64 causal grids from 768 tokens gain up to two: B1 H12 S1000 12.5 ->
+// 11.6, B1 H8 S2048 19.5 -> 16.4.
+constexpr long long kThirtyTwoRowsCausalF16 = 512;
 // fp16 D64, 64-row blocks of one round: four groups of two wavefronts on
 // 32-key tiles instead of two on 64-key ones from this many tokens: B1 H12
 // S1024 11.9 -> 11.0, B1 H8 S2048 19.0 -> 16.9, causal 19.6 -> 17.8; S512 8.0
@@ -1407,6 +1428,8 @@ void launch(const T* q, const T* k, const T* v, float* out, int bh, int s, int d
     } else if (wide) {
       if (d96) OPL_RUN(128, 1, 4, 64, 96);
       else OPL_RUN(128, 1, 4, 64);
+    } else if (causal && rows32 <= kThirtyTwoRowsCausalF16 && s >= kFourGroupsFrom) {
+      OPL_RUN(64, 4, 1, 32);
     } else if (rows64 <= kOneRound && s >= kFourGroupsFrom) {
       OPL_RUN(64, 4, 2, 32);
     } else if (half_rows) {
@@ -1419,11 +1442,11 @@ void launch(const T* q, const T* k, const T* v, float* out, int bh, int s, int d
     // hold 64 KiB).
     if (!wide && s > 64 &&
         (rows32 <= kOneRound ||
-         (causal && s >= kThirtyTwoRowsUpTo && rows32 <= kThirtyTwoRowsCausalF32))) {
+         (causal && s >= kThirtyTwoRowsCausalFrom && rows32 <= kThirtyTwoRowsCausalF32))) {
       OPL_RUN(64, 4, 1, 32);
     } else if (!wide && s > 64 && !causal && rows48 <= kOneRound) {
-      // 48 rows per wavefront, where that is one round: B1 H12 S1000 45.3 ->
-      // 39.3 us
+      // 48 rows per wavefront, where that is one round: B1 H12 S1000 44.5 ->
+      // 36.2 us
       OPL_RUN(64, 4, 1, 32, 64, 3);
     } else if (wide && half_rows) {
       if (d96) OPL_RUN(128, 2, 2, 32, 96);
