@@ -168,14 +168,16 @@ constexpr int kBufferFlags = 0x00020000;
 // touches no memory. The hardware range-checks only the per-lane offset,
 // not the instruction's scalar offset, so this helper passes no scalar
 // offset: callers move a tile's position into `base` and shrink `bytes` to
-// match. Kept out of kernel bodies so the host compilation pass never meets
+// match. Aux: the instruction's cache bits (2: non-temporal). Kept out of
+// kernel bodies so the host compilation pass never meets
 // the device-only resource type.
+template <int Aux = 0>
 __device__ __forceinline__ void buffer_copy16_lds(const void* base, unsigned bytes,
                                                   unsigned char* dst, int voffset) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(
       __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), static_cast<short>(0),
                                         bytes, kBufferFlags),
-      (__attribute__((address_space(3))) void*)dst, 16, voffset, 0, 0, 0);
+      (__attribute__((address_space(3))) void*)dst, 16, voffset, 0, 0, Aux);
 }
 
 // max / sum of v over lanes l and l ^ 32 (the two halves of a wavefront),

@@ -7,7 +7,7 @@
 // Reference: operatorlib::gemm_f16 / gemm_f32 (src/gemm.cu:440-479). The
 // reference dispatches between WMMA, cp.async register-tiled and scalar
 // kernels on divisibility; here the dispatch is, in order:
-//   * M <= 2 (fp16, B from 8 MiB) or M <= 4 (fp32): the skinny kernel
+//   * M <= 2 (fp16, B from 8 MiB) or M <= 4 (fp32, 8 from 128 MiB): the skinny kernel
 //     (namespace skinny), an HBM stream over B with split K and an ordered
 //     split sum (M <= 16 where K or N passes the 32-bit limits below);
 //   * N <= 16 (matrix-vector products): namespace narrow, an HBM stream
@@ -1402,10 +1402,13 @@ void launch_m(const T* a, const T* b, float* dst, int m, int n, int k,
 // takes every M up to kMaxM.
 template <typename T>
 bool applies(const T* b, int m, int n, int k, bool wide) {
+  const std::size_t bytes = static_cast<std::size_t>(k) * n * sizeof(T);
+  // fp32 up to M = 8 on a long B: ksplit_kernel is 7-10% faster there, but its
+  // few splits sum longer chains (8 x 8192 x 8192, error against 64 bits
+  // 1.4e-7 here, 2.1e-7 there).
+  const int up_to = sizeof(T) == 4 && bytes >= (std::size_t(128) << 20) ? 8 : Cfg<T>::kUpToM;
   return n % Cfg<T>::kPerLane == 0 && opl::aligned16(b) &&
-         (wide ? m <= kMaxM
-               : m <= Cfg<T>::kUpToM &&
-                     static_cast<std::size_t>(k) * n * sizeof(T) >= Cfg<T>::kMinBytes);
+         (wide ? m <= kMaxM : m <= up_to && bytes >= Cfg<T>::kMinBytes);
 }
 
 // K split of one call: `splits` workgroup rows of `chunk` K rows each (a
@@ -1689,7 +1692,7 @@ __device__ __forceinline__ int swizzle_b(int k) {
   else
     return 4 * ((k >> 2) & 3);
 }
-template <typename T, int FM, typename S, bool kEdge>
+template <typename T, int FM, typename S, bool kEdge, bool kStreamB = false>
 __global__ __launch_bounds__(S::kThreads)
 __attribute__((amdgpu_waves_per_eu(S::kWaves / 4, S::kWaves / 4 * (FM == 1 ? 2 : 1))))
 void ksplit_kernel(const T* __restrict__ A, const T* __restrict__ B, float* __restrict__ out,
@@ -1777,7 +1780,7 @@ void ksplit_kernel(const T* __restrict__ A, const T* __restrict__ B, float* __re
       opl::buffer_copy16_lds(a_base, a_span, st + j * 1024, a_dma[j]);
 #pragma unroll
     for (int j = 0; j < kBCopies; ++j)
-      opl::buffer_copy16_lds(b_base, b_span, st + kABytes + j * 1024, b_dma[j]);
+      opl::buffer_copy16_lds<kStreamB ? 2 : 0>(b_base, b_span, st + kABytes + j * 1024, b_dma[j]);
   };
 
   // Fragment offsets inside a stage: lane l supplies row / column l % 16 and
@@ -1992,6 +1995,12 @@ void ksplit_kernel(const T* __restrict__ A, const T* __restrict__ B, float* __re
 }
 
 constexpr int kMaxSplits = 16;
+// B that one row of tiles reads once, and that fills half the Infinity Cache
+// or more, is copied with the non-temporal hint. Measured on MI355X (us,
+// cached -> non-temporal, three sets of inputs / twenty): fp16 16 x 8192 x
+// 8192 (128 MiB) 34.4 -> 31.0 / 34.5 -> 31.6; 8 x 11008 x 4096 (86 MiB) 17.8 ->
+// 19.7 / 20.8 -> 20.2; 16 x 4096 x 4096 (32 MiB) 10.8 -> 12.2 / 13.2 -> 12.8.
+constexpr std::size_t kStreamBFrom = std::size_t(128) << 20;
 
 struct Plan {
   int fm = 0;  // row fragments per tile; 0: not this kernel
@@ -2008,6 +2017,17 @@ void launch_shape(const T* a, const T* b, float* dst, int m, int n, int k, int s
   const int items = tiles_m * tiles_n * splits;
   const dim3 grid(static_cast<unsigned>((items + kXcds - 1) / kXcds * kXcds)), block(S::kThreads);
   const bool edge = k % (S::kSubs * Elem<T>::kSubK) != 0 || (sizeof(T) == 2 && n % 2 != 0);
+  if constexpr (FM <= 2) {
+    if (tiles_m == 1 && static_cast<std::size_t>(k) * n * sizeof(T) >= kStreamBFrom) {
+      if (edge)
+        ksplit_kernel<T, FM, S, true, true><<<grid, block, 0, stream>>>(a, b, dst, m, n, k, tiles_m,
+                                                                       tiles_n, splits);
+      else
+        ksplit_kernel<T, FM, S, false, true><<<grid, block, 0, stream>>>(a, b, dst, m, n, k,
+                                                                        tiles_m, tiles_n, splits);
+      return;
+    }
+  }
   if (edge)
     ksplit_kernel<T, FM, S, true><<<grid, block, 0, stream>>>(a, b, dst, m, n, k, tiles_m,
                                                              tiles_n, splits);
@@ -2473,8 +2493,11 @@ double ksplit_ns(int fm, int splits, int m, int n, int k, int cus) {
   const bool cached = operands < kCachedUpTo;
   const double asked = wgs / (wgs + (cached && sizeof(T) == 2 ? 25 : 60));
   const double uneven = std::sqrt(std::max(1.0, rounds * cus / std::max<double>(wgs, cus)));
+  // (a long B from memory is fetched again by a second row of tiles in part:
+  // fp16 32 x 8192 x 8192 44.3 us on 16-row tiles, 31.4 on 32-row ones)
+  const double again = !cached && n >= m && m > 16 * fm ? 1.3 : 1.0;
   const double stream =
-      operands / ((cached ? kCacheBytesPerNs : kMemoryBytesPerNs) * asked) * uneven;
+      operands / ((cached ? kCacheBytesPerNs : kMemoryBytesPerNs) * asked) * uneven * again;
   return kNsLaunch + starts * kNsRound + std::max(rounds * std::max(copies, mfma), stream) +
          (splits > 1 ? kNsSum + 8.0 * splits * m * n / kPartialBytesPerNs : 0.0);
 }
@@ -2505,18 +2528,21 @@ double small_tiles_ns(int m, int n, int k, int cus, const TailPlan& tail) {
 // eighth of a 128-row tile; otherwise grids of few 256 x 256 tiles.
 template <typename T>
 ksplit::Plan ksplit_plan(int m, int n, int k, bool few_rows, std::size_t capacity) {
-  const long long big_tiles = static_cast<long long>((m + 255) / 256) * ((n + 255) / 256);
+  const long long big_tiles = (m + 255LL) / 256 * ((n + 255LL) / 256);
   if (!few_rows && big_tiles >= DmaTiles<T>::kSmallBelow) return ksplit::Plan{};
   int cus = device_cus();
   if (cus <= 0) cus = 256;
   ksplit::Plan best;
   double best_ns = 0;
   for (int fm = 1; fm <= 6; ++fm) {
-    const long long rows = (m + 16 * fm - 1) / (16 * fm);
-    if (fm > 1 && (m + 16 * (fm - 1) - 1) / (16 * (fm - 1)) == rows) continue;  // more padding
+    const long long rows = (m + 16LL * fm - 1) / (16 * fm);
+    if (fm > 1 && (m + 16LL * (fm - 1) - 1) / (16 * (fm - 1)) == rows) continue;  // more padding
     const long long tiles = rows * ((n + ksplit::kBN - 1) / ksplit::kBN);
     if (tiles > 0x3fffffffLL) continue;
-    const long long slots = static_cast<long long>(cus) * (fm == 1 ? 2 : 1);
+    // Pairs of fm = 1 workgroups, but not of fp32 ones that stream from memory
+    // (8 x 8192 x 8192, us: 128 x 2 workgroups 48.0, x 4 55.6).
+    const bool pairs = fm == 1 && (sizeof(T) == 2 || (static_cast<double>(m) + n) * k * sizeof(T) < kCachedUpTo);
+    const long long slots = static_cast<long long>(cus) * (pairs ? 2 : 1);
     for (int splits = 1; splits <= ksplit::kMaxSplits; ++splits) {
       // one split, or a grid the CUs hold at once with a step per wavefront
       if (splits > 1 && (tiles * splits > slots || k / (8 * dma::Elem<T>::kSubK) < splits)) break;

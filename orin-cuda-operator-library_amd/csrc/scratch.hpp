@@ -8,9 +8,10 @@
 // means fewer splits or a slower kernel, never an error):
 //   * reduce: one fp64 partial per workgroup (at most 2 KiB);
 //   * softmax and RMSNorm rows split over workgroups (rows longer than
-//     32768 columns, or few rows longer than 4096): one partial per row
-//     and segment (8 or 4 bytes);
-//   * decode GEMMs (M <= 16): split-K partial sums;
+//     32768 columns, or few rows longer than kSplitAboveCols): one partial
+//     per row and segment (8 or 4 bytes);
+//   * decode and medium GEMMs (skinny_kernel, ksplit_kernel): split-K partial
+//     sums;
 //   * large fp16 GEMMs whose rows are not 4-byte aligned: operand copies
 //     with chunk-padded rows;
 //   * GEMMs whose last round of 256 x 256 tiles fills at most half the CUs,

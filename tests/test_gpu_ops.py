@@ -526,7 +526,8 @@ def test_gemm_skinny_row_blocks(hip, mnk, dtype):
 KSPLIT = [(15, 64, 256), (17, 65, 31), (33, 63, 33), (47, 130, 95), (80, 4096, 512),
           (81, 200, 1001), (97, 127, 64), (96, 3000, 2048), (300, 4100, 2049), (64, 4096, 2111),
           (5, 203, 4099), (16, 512, 8191), (3, 1, 1), (64, 33, 4097), (700, 40, 999),
-          (1000, 70, 2050), (301, 333, 7)]
+          (1000, 70, 2050), (301, 333, 7),
+          (5, 33555, 2001), (20, 8200, 8192)]  # B past 128 MiB: non-temporal copies
 
 
 @pytest.mark.parametrize("mnk", KSPLIT)
