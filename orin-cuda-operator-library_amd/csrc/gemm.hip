@@ -9,7 +9,7 @@
 // kernels on divisibility; here the dispatch is, in order:
 //   * M <= 2 (fp16, B from 8 MiB) or M <= 4 (fp32, 8 from 128 MiB): the skinny kernel
 //     (namespace skinny), an HBM stream over B with split K and an ordered
-//     split sum (M <= 16 where K or N passes the 32-bit limits below);
+//     split sum (M <= 16 where K or N passes ksplit_kernel's 32-bit limits);
 //   * N <= 16 (matrix-vector products): namespace narrow, an HBM stream
 //     over A, one launch;
 //   * gemm_dma_kernel (any K, N and alignment, K below 2^22 fp16 / 2^21
@@ -1995,6 +1995,9 @@ void ksplit_kernel(const T* __restrict__ A, const T* __restrict__ B, float* __re
 }
 
 constexpr int kMaxSplits = 16;
+// Fewer than 8 tiles would leave half the CUs idle at 16 splits (products of few
+// rows and columns and a long K): up to 256 there, in steps of a half.
+constexpr int kMaxSplitsFewTiles = 256;
 // B that one row of tiles reads once, and that fills half the Infinity Cache
 // or more, is copied with the non-temporal hint. Measured on MI355X (us,
 // cached -> non-temporal, three sets of inputs / twenty): fp16 16 x 8192 x
@@ -2543,7 +2546,8 @@ ksplit::Plan ksplit_plan(int m, int n, int k, bool few_rows, std::size_t capacit
     // (8 x 8192 x 8192, us: 128 x 2 workgroups 48.0, x 4 55.6).
     const bool pairs = fm == 1 && (sizeof(T) == 2 || (static_cast<double>(m) + n) * k * sizeof(T) < kCachedUpTo);
     const long long slots = static_cast<long long>(cus) * (pairs ? 2 : 1);
-    for (int splits = 1; splits <= ksplit::kMaxSplits; ++splits) {
+    const int max_splits = tiles < 8 ? ksplit::kMaxSplitsFewTiles : ksplit::kMaxSplits;
+    for (int splits = 1; splits <= max_splits; splits += splits < 16 ? 1 : splits / 2) {
       // one split, or a grid the CUs hold at once with a step per wavefront
       if (splits > 1 && (tiles * splits > slots || k / (8 * dma::Elem<T>::kSubK) < splits)) break;
       const std::size_t bytes =
@@ -2623,7 +2627,13 @@ GemmPlan plan_gemm(const T* a, const T* b, int m, int n, int k, std::size_t capa
   // 255 rows of A (255 * K * sizeof(T) bytes) and one K step of B rows (64
   // fp16 or 32 fp32 rows: 128 * N bytes).
   const bool dma_offsets_fit = k < (sizeof(T) == 2 ? (1 << 22) : (1 << 21)) && n < (1 << 24);
-  if (skinny::applies(b, m, n, k, !dma_offsets_fit)) {
+  // ksplit_kernel of few rows spans up to 31 fp16 or 63 fp32 rows of A, so it
+  // takes a longer K (us, register-staged kernel -> this one: fp16 20 x 16 x
+  // 2^22 132000 -> 92, fp32 20 x 16 x 2^21 149000 -> 106).
+  const bool few_rows = m <= (sizeof(T) == 2 ? 32 : 64);
+  const bool split_offsets_fit =
+      dma_offsets_fit || (few_rows && k < (sizeof(T) == 2 ? (1 << 25) : (1 << 23)) && n < (1 << 24));
+  if (skinny::applies(b, m, n, k, !split_offsets_fit)) {
     p.skinny = skinny::plan<T>(m, n, k, capacity);
     if (p.skinny.ok) {
       p.kind = GemmPlan::kSkinny;
@@ -2631,12 +2641,11 @@ GemmPlan plan_gemm(const T* a, const T* b, int m, int n, int k, std::size_t capa
       return p;
     }
   }
-  const bool few_rows = m <= (sizeof(T) == 2 ? 32 : 64);
   if (!(few_rows && n % skinny::Cfg<T>::kPerLane == 0) && narrow::applies(a, b, n, k)) {
     p.kind = GemmPlan::kNarrow;
     return p;
   }
-  if (dma_offsets_fit) {
+  if (split_offsets_fit) {
     p.split = ksplit_plan<T>(m, n, k, few_rows, capacity);
     if (p.split.fm > 0) {
       p.kind = GemmPlan::kSplit;

@@ -18,6 +18,8 @@ the first and last rows) where it is not.
 
 from __future__ import annotations
 
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -563,6 +565,36 @@ def test_gemm_ksplit(hip, mnk, offset, dtype):
         assert np.max(np.abs(y - ref)) <= 2e-3
     else:
         assert np.linalg.norm(y - ref) <= 1e-4 * np.linalg.norm(ref)
+
+
+# A few tiles and a long K: ksplit_kernel split over more than 16 workgroups per
+# tile (each count of the steps 24, 36, 54 .. from fewest to most), and K from
+# 2^22 (fp16) or 2^21 (fp32) on, past the tiled kernels' 32-bit offsets.
+FEW_TILES = [(5, 40, 8191), (33, 100, 30001), (100, 130, 20000), (20, 64, 262145)]
+FEW_TILES_WIDE = [(18, 16, 2), (32, 5, 1), (3, 40, 3)]
+
+
+@pytest.mark.parametrize("mnk,wide", [(c, False) for c in FEW_TILES] +
+                         [(c, True) for c in FEW_TILES_WIDE])
+@pytest.mark.parametrize("dtype", ["f32", "f16"])
+def test_gemm_few_tiles_long_k(ops, mnk, wide, dtype):
+    """Against a float64 product. Rounding of K fp32 additions in a random
+    walk: a relative 2-norm of at most sqrt(K) 2^-24."""
+    m, n, k = mnk
+    if wide:
+        k += 1 << (22 if dtype == "f16" else 21)
+    g = torch.Generator(device="cuda").manual_seed(940 + m)
+    dt = torch.float16 if dtype == "f16" else torch.float32
+    a = torch.randn(m, k, generator=g, device="cuda").to(dt)
+    b = torch.randn(k, n, generator=g, device="cuda").to(dt)
+    y = ops.gemm(a, b)
+    assert torch.equal(y, ops.gemm(a, b))
+    ref = np.zeros((m, n))
+    ah, bh = a.cpu().numpy(), b.cpu().numpy()
+    for i in range(0, k, 1 << 18):
+        ref += ah[:, i:i + (1 << 18)].astype(np.float64) @ bh[i:i + (1 << 18)].astype(np.float64)
+    error = np.linalg.norm(y.cpu().numpy() - ref) / np.linalg.norm(ref)
+    assert error <= math.sqrt(k) * 2.0 ** -24, error
 
 
 # fp16 grids that one round of 128 x 256 tiles (first four) or 192 x 256 tiles
