@@ -1403,9 +1403,10 @@ void launch_m(const T* a, const T* b, float* dst, int m, int n, int k,
 template <typename T>
 bool applies(const T* b, int m, int n, int k, bool wide) {
   const std::size_t bytes = static_cast<std::size_t>(k) * n * sizeof(T);
-  // fp32 up to M = 8 on a long B: ksplit_kernel is 7-10% faster there, but its
-  // few splits sum longer chains (8 x 8192 x 8192, error against 64 bits
-  // 1.4e-7 here, 2.1e-7 there).
+  // fp32 up to M = 8 on a long B, where neither kernel is the better one
+  // throughout (us, this kernel vs ksplit_kernel): 8 x 8192 x 8192 52.0 vs
+  // 48.8, 8 x 32000 x 4096 100 vs 89, but 5 x 8576 x 9856 62.8 vs 74.5, 8 x
+  // 12288 x 12288 111 vs 119.
   const int up_to = sizeof(T) == 4 && bytes >= (std::size_t(128) << 20) ? 8 : Cfg<T>::kUpToM;
   return n % Cfg<T>::kPerLane == 0 && opl::aligned16(b) &&
          (wide ? m <= kMaxM : m <= up_to && bytes >= Cfg<T>::kMinBytes);
@@ -1662,6 +1663,9 @@ typedef __fp16 fp16x4 __attribute__((ext_vector_type(4)));
 constexpr int kBN = 64;
 constexpr int kFN = kBN / 16;
 
+template <int I>
+using Index = std::integral_constant<int, I>;
+
 // How a workgroup splits its K range: kWaves wavefronts, each with two LDS
 // stages of kSubs substeps (kSubK of K each: 64 bytes of an A row, 4 KiB of B
 // rows).
@@ -1705,6 +1709,7 @@ void ksplit_kernel(const T* __restrict__ A, const T* __restrict__ B, float* __re
   constexpr int kSize = static_cast<int>(sizeof(T));
   constexpr int kSubK = Elem<T>::kSubK;
   constexpr int kBK = kSubs * kSubK;                 // K per step
+  constexpr int kProducts = kSize == 2 ? kSubs : 4 * kSubs;  // MFMAs per block and step
   constexpr int kBM = 16 * FM;
   constexpr int kABytes = kBM * kARowBytes;
   constexpr int kStage = kABytes + kBBytes;
@@ -1813,26 +1818,50 @@ void ksplit_kernel(const T* __restrict__ A, const T* __restrict__ B, float* __re
     if (b_end) b_end_value = B[static_cast<std::size_t>(K) * N - 1];
   }
 
-  // Two or four sets of sums, taken in turn, where the registers hold them:
-  // chains of additions as short as the kernels' before (error against 64
-  // bits, fp16 300 x 4096 x 4096: 2.1e-7 with one set, 1.5e-7 with two, 1.9e-7
-  // before; 7 x 8960 x 11456
-  // 2.5e-7 with one, 1.1e-7 with four, 1.3e-7 before).
-  constexpr int kSets = FM <= 2 ? 4 : (kWaves == 4 || FM <= 5) ? 2 : 1;
+  // Sums. kFold (every instance of few rows, which replaced kernels that cut K
+  // into chunks of 512): the products of each two steps start new chains of
+  // additions in kSets sets of sums, which are then added to `total`; four
+  // steps per chain from kLongSteps steps per wavefront on, where the additions
+  // to the total weigh more than the chains. Elsewhere a step's products go to
+  // one of kSets sets in turn, merged at the end (128 x 128 tiles, which ran
+  // there before, sum all of K in one chain). Measured on MI355X, relative
+  // 2-norm of the error against 64 bits (chunks of 512 before / two or four
+  // sets, no total / now): fp32 40 x 12288 x 12288 2.3e-7 / 5.0e-7 / 1.7e-7,
+  // 64 x 12288 x 12288 2.3e-7 / 3.6e-7 / 1.5e-7, 8 x 12288 x 2700 1.26e-7 /
+  // 1.77e-7 / 1.26e-7, fp16 32 x 12288 x 12288 1.3e-7 / 1.9e-7 / 1.1e-7; times
+  // within 5% of those without a total (fp32 64 x 4096 x 4096 24.2 -> 24.9 us).
+  constexpr bool kFold = FM <= (kSize == 2 ? 2 : 4);
+  constexpr int kSets = FM <= 2 ? 2 : kFold ? 1 : (kWaves == 4 || FM <= 5) ? 2 : 1;
+  constexpr int kLongSteps = 16;
+  const floatx4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
   floatx4 sums[kSets][FM][kFN];
+  floatx4 total[FM][kFN];  // (kFold only until the end)
 #pragma unroll
-  for (int q = 0; q < kSets; ++q)
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < kFN; ++j) {
+#pragma unroll
+      for (int q = 0; q < kSets; ++q) sums[q][i][j] = zero;
+      total[i][j] = zero;
+    }
+  // The sum of the first `used` sets, added to the total or (not kFold) as it.
+  auto fold = [&](auto used) {
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int j = 0; j < kFN; ++j)
+      for (int j = 0; j < kFN; ++j) {
+        floatx4 v = sums[0][i][j];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) sums[q][i][j][e] = 0.0f;
+        for (int q = 1; q < decltype(used)::value; ++q) v += sums[q][i][j];
+        total[i][j] = kFold ? total[i][j] + v : v;
+      }
+  };
 
-  // One step of this wavefront: its stage has landed once all but the newer
+  // One step of this wavefront (`position`: its place among the steps that share
+  // a chain of sums): its stage has landed once all but the newer
   // stage's copies have; the stage is refilled as soon as its fragments are
   // in registers.
-  auto tile = [&](unsigned char* st, int s, floatx4 (&acc)[FM][kFN]) {
+  auto tile = [&](unsigned char* st, int s, auto position) {
     // vmcnt(kCopies): all but the newer stage's copies
     __builtin_amdgcn_s_waitcnt((kCopies & 15) | ((kCopies >> 4) << 14) | 0xf70);
     __builtin_amdgcn_sched_barrier(0);
@@ -1890,26 +1919,27 @@ void ksplit_kernel(const T* __restrict__ A, const T* __restrict__ B, float* __re
         }
       }
     }
+    // Product p of the step: one MFMA per 16 x 16 block.
+    auto product = [&](int p, auto mma) {
+      constexpr int kPosition = decltype(position)::value;
+      const int index = kFold ? kPosition * kProducts + p : kPosition;
+      floatx4(&acc)[FM][kFN] = sums[index % kSets];
+      const bool fresh = kFold && index < kSets;
 #pragma unroll
-    for (int u = 0; u < kSubs; ++u) {
-      if constexpr (kSize == 2) {
+      for (int ti = 0; ti < FM; ++ti)
 #pragma unroll
-        for (int ti = 0; ti < FM; ++ti)
+        for (int tj = 0; tj < kFN; ++tj)
+          acc[ti][tj] = mma(ti, tj, fresh ? zero : acc[ti][tj]);
+    };
 #pragma unroll
-          for (int tj = 0; tj < kFN; ++tj)
-            acc[ti][tj] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa[u][ti], fb[u][tj], acc[ti][tj],
-                                                                 0, 0, 0);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-#pragma unroll
-          for (int ti = 0; ti < FM; ++ti)
-#pragma unroll
-            for (int tj = 0; tj < kFN; ++tj)
-              acc[ti][tj] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[u][ti][e], fb[u][tj][e],
-                                                                 acc[ti][tj], 0, 0, 0);
-      }
-    }
+    for (int p = 0; p < kProducts; ++p)
+      product(p, [&](int ti, int tj, floatx4 c) {
+        if constexpr (kSize == 2)
+          return __builtin_amdgcn_mfma_f32_16x16x32_f16(fa[p][ti], fb[p][tj], c, 0, 0, 0);
+        else
+          return __builtin_amdgcn_mfma_f32_16x16x4f32(fa[p / 4][ti][p % 4], fb[p / 4][tj][p % 4], c,
+                                                      0, 0, 0);
+      });
     __builtin_amdgcn_sched_barrier(0);
   };
   unsigned char* const st0 = stage0 + wave * kStage;
@@ -1917,26 +1947,28 @@ void ksplit_kernel(const T* __restrict__ A, const T* __restrict__ B, float* __re
   int s = wave;
   issue(st0, s);
   issue(st1, s + kWaves);
-  if constexpr (kSets == 4) {
-    for (; s + 3 * kWaves < steps; s += 4 * kWaves) {
-      tile(st0, s, sums[0]);
-      tile(st1, s + kWaves, sums[1]);
-      tile(st0, s + 2 * kWaves, sums[2]);
-      tile(st1, s + 3 * kWaves, sums[3]);
+  if constexpr (FM <= 2) {
+    if (steps >= kLongSteps * kWaves) {
+      for (; s + 3 * kWaves < steps; s += 4 * kWaves) {
+        tile(st0, s, Index<0>{});
+        tile(st1, s + kWaves, Index<1>{});
+        tile(st0, s + 2 * kWaves, Index<2>{});
+        tile(st1, s + 3 * kWaves, Index<3>{});
+        fold(Index<kSets>{});
+      }
     }
   }
   for (; s + kWaves < steps; s += 2 * kWaves) {
-    tile(st0, s, sums[0]);
-    tile(st1, s + kWaves, sums[kSets > 1]);
+    tile(st0, s, Index<0>{});
+    tile(st1, s + kWaves, Index<1>{});
+    if constexpr (kFold) fold(Index<kSets>{});
   }
-  if (s < steps) tile(st0, s, sums[0]);
-  floatx4 (&acc)[FM][kFN] = sums[0];
-#pragma unroll
-  for (int q = 1; q < kSets; ++q)
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < kFN; ++j) acc[i][j] += sums[q][i][j];
+  if (s < steps) {
+    tile(st0, s, Index<0>{});
+    if constexpr (kFold) fold(Index<std::min(kSets, kProducts)>{});
+  }
+  if constexpr (!kFold) fold(Index<kSets>{});
+  floatx4(&acc)[FM][kFN] = total;
 
   // Sum of the wavefronts' partial tiles through LDS: of eight, 4-7 hand
   // theirs to 0-3 first; the four sums are added in order on the way out.

@@ -567,6 +567,28 @@ def test_gemm_ksplit(hip, mnk, offset, dtype):
         assert np.linalg.norm(y - ref) <= 1e-4 * np.linalg.norm(ref)
 
 
+# Few rows on wide products, where K is not split over workgroups: the error
+# against 64 bits stays within that of K summed in chunks of 512. Additions of
+# equal random terms one after another leave a relative error of about 0.43 2^-24
+# (a uniform rounding error over a mantissa's range) times the root of half
+# their number. fp32: chains of 128 per chunk (32 for M <= 8, on 16 lane
+# groups), four (16) merged, K / 512 chunks; fp16: chains of 32, as an MFMA of
+# 16 products rounds four times.
+@pytest.mark.parametrize("dtype,m,n,k,halves", [
+    ("f32", 40, 12288, 12288, 64 + 2), ("f32", 64, 8192, 12288, 64 + 2),
+    ("f32", 33, 9000, 9000, 64 + 2), ("f32", 16, 12288, 12288, 64 + 2),
+    ("f32", 8, 12288, 2700, 16 + 8), ("f32", 8, 8192, 4032, 16 + 8),
+    ("f16", 32, 12288, 12288, 16 + 2), ("f16", 22, 9152, 10624, 16 + 2)])
+def test_gemm_few_rows_error(ops, dtype, m, n, k, halves):
+    g = torch.Generator(device="cuda").manual_seed(950 + m)
+    dt = torch.float16 if dtype == "f16" else torch.float32
+    a = torch.randn(m, k, generator=g, device="cuda").to(dt)
+    b = torch.randn(k, n, generator=g, device="cuda").to(dt)
+    ref = torch.mm(a.double(), b.double())
+    error = ((ops.gemm(a, b) - ref).norm() / ref.norm()).item()
+    assert error <= 0.43 * 2.0 ** -24 * math.sqrt(halves + k / 1024), error
+
+
 # A few tiles and a long K: ksplit_kernel split over more than 16 workgroups per
 # tile (each count of the steps 24, 36, 54 .. from fewest to most), and K from
 # 2^22 (fp16) or 2^21 (fp32) on, past the tiled kernels' 32-bit offsets.
