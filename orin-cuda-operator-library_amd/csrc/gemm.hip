@@ -9,7 +9,8 @@
 // kernels on divisibility; here the dispatch is, in order:
 //   * M <= 2 (fp16, B from 8 MiB) or M <= 4 (fp32, 8 from 128 MiB): the skinny kernel
 //     (namespace skinny), an HBM stream over B with split K and an ordered
-//     split sum (M <= 16 where K or N passes ksplit_kernel's 32-bit limits);
+//     split sum (up to 32 fp16 / 64 fp32 rows, from M = 5 / 9 on the matrix
+//     cores, where K or N passes ksplit_kernel's 32-bit limits);
 //   * N <= 16 (matrix-vector products): namespace narrow, an HBM stream
 //     over A, one launch;
 //   * gemm_dma_kernel (any K, N and alignment, K below 2^22 fp16 / 2^21
@@ -1150,7 +1151,6 @@ typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float floatx4v __attribute__((ext_vector_type(4)));
 
 constexpr int kThreads = 256;
-constexpr int kMaxM = 16;  // the vector-ALU kernel's largest M
 constexpr int kLanesPerRow = 16;                     // one 256-byte row segment
 constexpr int kRowGroups = kThreads / kLanesPerRow;  // 16
 constexpr int kWaves = kThreads / opl::kWaveSize;    // 4
@@ -1170,6 +1170,14 @@ struct Cfg {
   // 1024^2 6.7 vs 6.5.
   static constexpr int kUpToM = sizeof(T) == 2 ? 2 : 4;
   static constexpr std::size_t kMinBytes = sizeof(T) == 2 ? std::size_t(8) << 20 : 0;
+  // Past ksplit_kernel's offsets skinny_mfma_kernel runs from kMfmaMinM to
+  // kMaxMfmaM rows (2 row blocks of 16, fp32 4). Measured on MI355X (us, this
+  // kernel vs skinny_mfma_kernel): fp16 M = 8 (N = 16, K = 2^25) 4190 vs 3860,
+  // M = 16 6150 vs 4020, M = 16 (N = 2^24 + 8, K = 72) 2390 vs 1150; fp32 M = 16
+  // (N = 16, K = 2^23) 1220 vs 950. 20 rows on the register-staged kernel 1.06 s
+  // vs 4210 us (fp16), 598 ms vs 1070 us (fp32).
+  static constexpr int kMfmaMinM = sizeof(T) == 2 ? 5 : 9;
+  static constexpr int kMaxMfmaM = sizeof(T) == 2 ? 32 : 64;
 };
 
 // Row steps (16-byte loads of one or two rows) in flight per thread per
@@ -1356,6 +1364,212 @@ void skinny_kernel(
   }
 }
 
+// Matrix-core variant for M up to 32 (fp16) or 64 (fp32), in row blocks of 16,
+// where K or N passes ksplit_kernel's 32-bit offsets (64-bit addresses here):
+// one v_mfma_f32_16x16x16_f16 (fp16) or v_mfma_f32_16x16x4_f32 (fp32) turns 16
+// rows of A times a 16 x 16 block of B into a 16 x 16 block of C, where the
+// vector-ALU kernel spends one dot product per (m, column pair) and becomes
+// ALU-bound as M grows. What bounds it: B's stream from memory (fp16 N = 16, K =
+// 2^25: 1 GiB of B and 64 MiB of A per row, 4210 us at 20 rows).
+// B is never transposed: the MFMA only needs A and B to agree on which k
+// fills each of its k slots. K is walked in blocks of 16 rows; lane (g, c)
+// (g = lane / 16, c = lane % 16) owns rows 4g .. 4g+3 of each block (fp32
+// with unaligned A: blocks of 4 rows, row g each, 16 blocks in flight, as
+// the element loads gain nothing from the grouping):
+//   * it loads a 16-byte chunk (columns P*c .. P*c+P-1) of each of those
+//     rows, and MFMA j takes column j of every lane's chunk, so tile column
+//     c of MFMA j is matrix column P*c + j and P MFMAs cover the
+//     workgroup's 16 P columns;
+//   * its A operand values A[c][4g .. 4g+3] are contiguous, one 8-byte
+//     (fp16) or 16-byte (fp32) load straight from global memory (A is
+//     L2-resident), issued with the B loads, so nothing waits on a staging
+//     barrier; rows that are not 4-aligned fall back to element loads;
+//   * fp16 feeds the four rows to one 16x16x16 MFMA (k slots 4g .. 4g+3);
+//     fp32 issues four 16x16x4 MFMAs, the u-th taking row 4g + u in k slot
+//     g.
+// Splits, the workgroup shape and the partial sums are those of
+// skinny_kernel.
+template <typename T>
+struct MfmaCfg;
+template <>
+struct MfmaCfg<_Float16> {
+  typedef _Float16 AOp __attribute__((ext_vector_type(4)));
+  typedef _Float16 AVec __attribute__((ext_vector_type(4)));
+  static constexpr int kBatch = 4;    // 16-row k blocks in flight per wavefront
+  __device__ static floatx4v mma(AOp a, AOp b, floatx4v c) {
+    return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0);
+  }
+};
+template <>
+struct MfmaCfg<float> {
+  typedef float AOp;
+  typedef float AVec __attribute__((ext_vector_type(4)));
+  static constexpr int kBatch = 4;
+  __device__ static floatx4v mma(AOp a, AOp b, floatx4v c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+};
+
+// Rows of a k block that one lane owns (and the MFMA k slots they fill).
+constexpr int kLaneRows = 4;
+
+// kVecA: K % 4 == 0 and A aligned to 4 elements, so each lane's four A
+// values of a block are one aligned vector, wholly inside or outside the chunk.
+// kMB row blocks of 16 (M up to 16 kMB): every B chunk a lane loads feeds
+// one MFMA per row block, so B is still streamed once.
+template <typename T, bool kVecA, int kMB>
+__global__ __launch_bounds__(kThreads) void skinny_mfma_kernel(
+    const T* __restrict__ A, const T* __restrict__ B, float* __restrict__ out,
+    int m_rows, int n, int k, int chunk) {
+  using MC = MfmaCfg<T>;
+  using Vec = typename RowChunk<T>::Vec;  // one 16-byte chunk of a B row
+  constexpr int P = Cfg<T>::kPerLane;     // columns per lane
+  constexpr int BN = Cfg<T>::kBlockN;     // 16 * P
+  // Rows per lane and k block: 4, or 1 for fp32 without vector A loads.
+  constexpr int R = sizeof(T) == 4 && !kVecA ? 1 : kLaneRows;
+  constexpr int KB = 4 * R;  // rows per k block
+  // k blocks in flight, halved at four row blocks (fp32 only): the full
+  // batch compiled to 193 VGPRs there, one wavefront per SIMD, the half to
+  // 78
+  constexpr int kBatch = (R == 1 ? 16 : MC::kBatch) / (kMB >= 4 ? 2 : 1);
+  using AVec = typename std::conditional<R == 1, T, typename MC::AVec>::type;
+  // k slot q of a lane's A values
+  auto a_at = [](const AVec& a, int q) -> T {
+    if constexpr (R == 1) return a; else return a[q];
+  };
+  __shared__ float red[kWaves * opl::kWaveSize * P * 4];
+
+  const int n0 = blockIdx.x * BN;
+  const int k0 = blockIdx.y * chunk;
+  const int len = min(k - k0, chunk);  // K rows of this workgroup
+  const int tid = threadIdx.x;
+  const int lane = tid % opl::kWaveSize;
+  const int wave = tid / opl::kWaveSize;
+  const int g = lane / 16;
+  const int c = lane % 16;
+  // Columns past N: read a valid chunk (n % P == 0), results not stored.
+  const int col = min(n0 + c * P, n - P);
+  const int blocks = (len + KB - 1) / KB;
+
+  // k block b, lane group g: k rows KB b + R g + q (q < R) from k0. B: a
+  // 16-byte chunk of each row; A: A[16 mb + c][row] of each row block mb
+  // (read from L2, every workgroup of the split reads the same A). Rows
+  // past the chunk read valid memory and are zeroed, as are A rows past m_rows.
+  auto load_block = [&](int b, Vec (&v)[R], AVec (&a)[kMB]) {
+    const int r0 = KB * b + R * g;
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const int r = r0 + q;
+      const bool in = r < len;
+      const int rc = k0 + (in ? r : len - 1);
+      // Non-temporal B loads for fp32 only. Measured on MI355X (us, cached
+      // -> non-temporal): fp32 M = 16 20.07 -> 19.51, M = 64 41.98 ->
+      // 41.24; fp16 M = 16 13.53 -> 14.04, M = 32 17.91 -> 19.58 (N = K =
+      // 4096).
+      const Vec* const src = reinterpret_cast<const Vec*>(B + static_cast<std::size_t>(rc) * n + col);
+      Vec x;
+      if constexpr (sizeof(T) == 4)
+        x = __builtin_nontemporal_load(src);
+      else
+        x = *src;
+#pragma unroll
+      for (int j = 0; j < P; ++j) x[j] = in ? x[j] : T(0);
+      v[q] = x;
+      if constexpr (!kVecA) {
+        // element loads, each issued beside its B row's load
+#pragma unroll
+        for (int mb = 0; mb < kMB; ++mb) {
+          const int arow = 16 * mb + c;
+          const bool a_in = in && arow < m_rows;
+          const T av = A[a_in ? static_cast<std::size_t>(arow) * k + k0 + r : 0];
+          if constexpr (R == 1)
+            a[mb] = a_in ? av : T(0);
+          else
+            a[mb][q] = a_in ? av : T(0);
+        }
+      }
+    }
+    if constexpr (kVecA) {
+      // k0, r0 and len are multiples of 4: rows r0 .. r0+3 are all in or all
+      // out. Out-of-range lanes read A[0 .. 3] (k >= 4) and zero it.
+#pragma unroll
+      for (int mb = 0; mb < kMB; ++mb) {
+        const int arow = 16 * mb + c;
+        const bool a_in = r0 < len && arow < m_rows;
+        AVec x = *reinterpret_cast<const AVec*>(
+            A + (a_in ? static_cast<std::size_t>(arow) * k + k0 + r0 : 0));
+#pragma unroll
+        for (int q = 0; q < R; ++q) a[mb][q] = a_in ? x[q] : T(0);
+      }
+    }
+  };
+
+  floatx4v acc[kMB][P];
+#pragma unroll
+  for (int mb = 0; mb < kMB; ++mb)
+#pragma unroll
+    for (int j = 0; j < P; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[mb][j][e] = 0.0f;
+
+  Vec v[kBatch][R];
+  AVec a[kBatch][kMB];
+  for (int b0 = wave; b0 < blocks; b0 += kWaves * kBatch) {
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const int b = b0 + kWaves * u;
+      load_block(b < blocks ? b : blocks - 1, v[u], a[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      if (b0 + kWaves * u < blocks) {  // wave-uniform
+#pragma unroll
+        for (int j = 0; j < P; ++j) {
+          if constexpr (sizeof(T) == 2) {
+            typename MC::AOp bop;
+#pragma unroll
+            for (int q = 0; q < R; ++q) bop[q] = v[u][q][j];
+#pragma unroll
+            for (int mb = 0; mb < kMB; ++mb) acc[mb][j] = MC::mma(a[u][mb], bop, acc[mb][j]);
+          } else {
+#pragma unroll
+            for (int q = 0; q < R; ++q)
+#pragma unroll
+              for (int mb = 0; mb < kMB; ++mb)
+                acc[mb][j] = MC::mma(a_at(a[u][mb], q), v[u][q][j], acc[mb][j]);
+          }
+        }
+      }
+    }
+  }
+
+  // acc[mb][j][i] = C[16 mb + 4 g + i][n0 + P c + j] of this wavefront's
+  // k blocks; the wavefronts' sums go through LDS one row block at a time.
+  float* dst = out + static_cast<std::size_t>(blockIdx.y) * m_rows * n;
+#pragma unroll
+  for (int mb = 0; mb < kMB; ++mb) {
+    if (mb > 0) __syncthreads();  // the previous block's reads are done
+#pragma unroll
+    for (int j = 0; j < P; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        red[((wave * opl::kWaveSize + lane) * P + j) * 4 + i] = acc[mb][j][i];
+    __syncthreads();
+    for (int o = tid; o < 16 * BN; o += kThreads) {
+      const int m = o / BN;
+      const int co = o % BN;
+      const int row = 16 * mb + m;
+      if (row < m_rows && n0 + co < n) {
+        const int src = ((16 * (m / 4) + co / P) * P + co % P) * 4 + m % 4;
+        float s = red[src];
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w) s += red[w * opl::kWaveSize * P * 4 + src];
+        dst[static_cast<std::size_t>(row) * n + n0 + co] = s;
+      }
+    }
+  }
+}
+
 // out[i] = sum over splits s (in order) of part[s][i]. Each thread issues
 // the loads of up to kSplitBatch splits before adding them, so a sum costs
 // one memory round trip per batch instead of one per split.
@@ -1398,8 +1612,19 @@ void launch_m(const T* a, const T* b, float* dst, int m, int n, int k,
   skinny_kernel<T, M><<<grid, dim3(kThreads), 0, stream>>>(a, b, dst, m, n, k, chunk);
 }
 
-// wide: K or N past the other kernels' 32-bit offsets, where this kernel
-// takes every M up to kMaxM.
+template <typename T, int kMB>
+void launch_mfma(bool vec_a, const T* a, const T* b, float* dst, int m, int n, int k,
+                 int chunk, dim3 grid, hipStream_t stream) {
+  if (vec_a)
+    skinny_mfma_kernel<T, true, kMB><<<grid, dim3(kThreads), 0, stream>>>(a, b, dst, m, n, k,
+                                                                        chunk);
+  else
+    skinny_mfma_kernel<T, false, kMB><<<grid, dim3(kThreads), 0, stream>>>(a, b, dst, m, n, k,
+                                                                         chunk);
+}
+
+// wide: K or N past ksplit_kernel's 32-bit offsets, where the skinny kernels
+// take every M up to kMaxMfmaM.
 template <typename T>
 bool applies(const T* b, int m, int n, int k, bool wide) {
   const std::size_t bytes = static_cast<std::size_t>(k) * n * sizeof(T);
@@ -1409,7 +1634,7 @@ bool applies(const T* b, int m, int n, int k, bool wide) {
   // 12288 x 12288 111 vs 119.
   const int up_to = sizeof(T) == 4 && bytes >= (std::size_t(128) << 20) ? 8 : Cfg<T>::kUpToM;
   return n % Cfg<T>::kPerLane == 0 && opl::aligned16(b) &&
-         (wide ? m <= kMaxM : m <= up_to && bytes >= Cfg<T>::kMinBytes);
+         (wide ? m <= Cfg<T>::kMaxMfmaM : m <= up_to && bytes >= Cfg<T>::kMinBytes);
 }
 
 // K split of one call: `splits` workgroup rows of `chunk` K rows each (a
@@ -1464,11 +1689,27 @@ hipError_t launch(const T* a, const T* b, float* c, int m, int n, int k, const P
   float* dst = p.splits > 1 ? static_cast<float*>(partials) : c;
   const int chunk = p.chunk;
   const dim3 grid(static_cast<unsigned>(blocks_n), static_cast<unsigned>(p.splits));
-  if (m == 1) launch_m<T, 1>(a, b, dst, m, n, k, chunk, grid, stream);
-  else if (m <= 2) launch_m<T, 2>(a, b, dst, m, n, k, chunk, grid, stream);
-  else if (m <= 4) launch_m<T, 4>(a, b, dst, m, n, k, chunk, grid, stream);
-  else if (m <= 8) launch_m<T, 8>(a, b, dst, m, n, k, chunk, grid, stream);
-  else launch_m<T, 16>(a, b, dst, m, n, k, chunk, grid, stream);
+  if (m >= C::kMfmaMinM) {
+    const bool vec_a =
+        k % kLaneRows == 0 &&
+        reinterpret_cast<std::uintptr_t>(a) % (kLaneRows * sizeof(T)) == 0;
+    if (m <= 16) {
+      launch_mfma<T, 1>(vec_a, a, b, dst, m, n, k, chunk, grid, stream);
+    } else if (m <= 32) {
+      launch_mfma<T, 2>(vec_a, a, b, dst, m, n, k, chunk, grid, stream);
+    } else {
+      if constexpr (C::kMaxMfmaM > 32)
+        launch_mfma<T, 4>(vec_a, a, b, dst, m, n, k, chunk, grid, stream);
+    }
+  } else if (m == 1) {
+    launch_m<T, 1>(a, b, dst, m, n, k, chunk, grid, stream);
+  } else if (m <= 2) {
+    launch_m<T, 2>(a, b, dst, m, n, k, chunk, grid, stream);
+  } else if (m <= 4) {
+    launch_m<T, 4>(a, b, dst, m, n, k, chunk, grid, stream);
+  } else {
+    if constexpr (C::kMfmaMinM > 5) launch_m<T, 8>(a, b, dst, m, n, k, chunk, grid, stream);
+  }
   const hipError_t status = hipGetLastError();
   if (status != hipSuccess || p.splits == 1) return status;
   return sum_splits(dst, c, static_cast<long long>(m) * n, p.splits, lease);
@@ -2673,7 +2914,8 @@ GemmPlan plan_gemm(const T* a, const T* b, int m, int n, int k, std::size_t capa
       return p;
     }
   }
-  if (!(few_rows && n % skinny::Cfg<T>::kPerLane == 0) && narrow::applies(a, b, n, k)) {
+  if (!(few_rows && split_offsets_fit && n % skinny::Cfg<T>::kPerLane == 0) &&
+      narrow::applies(a, b, n, k)) {
     p.kind = GemmPlan::kNarrow;
     return p;
   }

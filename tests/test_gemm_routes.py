@@ -1,0 +1,69 @@
+"""Which kernel a GEMM call takes, asked of plan_gemm (csrc/gemm.hip) on the host.
+
+tests/host/gemm_plan.cpp is gemm.hip compiled for the host alone: the plan of any
+shape, alignment and scratch capacity, without a GPU and without memory behind
+the addresses. Shapes past the kernels' 32-bit offsets are pinned to the
+kernels that hold 64-bit ones.
+"""
+
+from __future__ import annotations
+
+import os
+import subprocess
+from pathlib import Path
+
+import pytest
+
+HERE = Path(__file__).resolve().parent
+REPO = HERE.parent
+CSRC = REPO / "orin-cuda-operator-library_amd" / "csrc"
+HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+
+
+@pytest.fixture(scope="module")
+def plans(tmp_path_factory):
+    """plans(cases) -> one dict per (dtype, m, n, k[, a_off, b_off, capacity])."""
+    out = tmp_path_factory.mktemp("gemm_plan")
+    obj, exe = out / "gemm_plan.o", out / "gemm_plan"
+    subprocess.run([HIPCC, "-O1", "-fPIC", "-std=c++17", "--offload-arch=gfx950",
+                    "--offload-host-only", "-fuse-cuid=none", "-x", "hip",
+                    f"-I{REPO / 'include'}", f"-I{CSRC}", "-c",
+                    str(HERE / "host" / "gemm_plan.cpp"), "-o", str(obj)],
+                   check=True, capture_output=True, text=True, timeout=300)
+    # The launches' symbols stay unresolved: a plan calls none of them.
+    subprocess.run(["g++", str(obj), "-Wl,--unresolved-symbols=ignore-all", "-o", str(exe)],
+                   check=True, capture_output=True, text=True, timeout=120)
+
+    def ask(cases):
+        text = "".join(" ".join(map(str, (*c, *(0, 0, 0)[len(c) - 4:]))) + "\n" for c in cases)
+        proc = subprocess.run([str(exe)], input=text, capture_output=True, text=True, check=True,
+                              timeout=60)
+        answers = [{key: value if key == "kind" else int(value) for key, value in
+                    (word.split("=") for word in line.split())}
+                   for line in proc.stdout.splitlines()]
+        assert len(answers) == len(cases)
+        return answers
+
+    return ask
+
+
+def test_few_rows_past_the_offset_limits(plans):
+    """K from 2^25 (fp16) / 2^23 (fp32) or N from 2^24 on, past the offsets of the
+    wavefront-split kernel: up to 32 / 64 aligned rows stream B once on the skinny
+    kernels; one row more, or rows of B off the vector, go to the narrow kernel
+    where N <= 16."""
+    cases, want = [], []
+    for dtype, most, first, limit in (("f16", 32, 5, 1 << 25), ("f32", 64, 9, 1 << 23)):
+        for m in (1, first - 1, first, 16, 17, most):
+            for n, k in ((16, limit), (8, limit + 64), ((1 << 24) + 8, 72)):
+                cases.append((dtype, m, n, k))
+                want.append(("skinny", m >= first))
+        cases += [(dtype, most + 1, 16, limit), (dtype, 20, 5, limit)]
+        want += [("narrow", None)] * 2
+        # just below the limits the wavefront-split kernel keeps the call
+        cases += [(dtype, 20, 16, limit - 64), (dtype, most, 64, limit - 64)]
+        want += [("split", None)] * 2
+    for case, plan, (kind, mfma) in zip(cases, plans(cases), want):
+        assert plan["kind"] == kind, (case, plan)
+        if mfma is not None:
+            assert plan["mfma"] == mfma, (case, plan)

@@ -619,6 +619,36 @@ def test_gemm_few_tiles_long_k(ops, mnk, wide, dtype):
     assert error <= math.sqrt(k) * 2.0 ** -24, error
 
 
+# K or N past ksplit_kernel's 32-bit offsets: the skinny kernels (64-bit ones) on
+# the matrix cores from 5 (fp16) or 9 (fp32) rows, one, two and four row blocks,
+# K a multiple of 4 (vector loads of A) and odd, a last chunk of K one row long;
+# the vector-ALU kernel below.
+PAST_OFFSETS = [("f16", 20, 8, (1 << 25) + 64), ("f16", 7, 16, (1 << 25) + 1),
+                ("f16", 3, 8, (1 << 25) + 64), ("f16", 32, (1 << 24) + 8, 40),
+                ("f16", 16, (1 << 24) + 8, 1), ("f32", 40, 4, (1 << 23) + 64),
+                ("f32", 9, 8, (1 << 23) + 1), ("f32", 24, 16, (1 << 23) + 3),
+                ("f32", 8, 4, (1 << 23) + 64), ("f32", 64, (1 << 24) + 4, 24)]
+
+
+@pytest.mark.parametrize("dtype,m,n,k", PAST_OFFSETS)
+def test_gemm_past_offsets(ops, dtype, m, n, k):
+    """Against float64 slabs on the GPU: a relative 2-norm of at most sqrt(K)
+    2^-24 (rounding of K fp32 additions in a random walk), for one slab of
+    columns after the other."""
+    g = torch.Generator(device="cuda").manual_seed(960 + m)
+    dt = torch.float16 if dtype == "f16" else torch.float32
+    a = torch.randn(m, k, generator=g, device="cuda", dtype=dt)
+    b = torch.randn(k, n, generator=g, device="cuda", dtype=dt)
+    y = ops.gemm(a, b)
+    for c in range(0, n, 1 << 21):
+        ref = torch.zeros(m, min(n - c, 1 << 21), dtype=torch.float64, device="cuda")
+        for i in range(0, k, 1 << 20):
+            ref += torch.mm(a[:, i:i + (1 << 20)].double(),
+                            b[i:i + (1 << 20), c:c + (1 << 21)].double())
+        error = ((y[:, c:c + (1 << 21)] - ref).norm() / ref.norm()).item()
+        assert error <= math.sqrt(k) * 2.0 ** -24, (c, error)
+
+
 # fp16 grids that one round of 128 x 256 tiles (first four) or 192 x 256 tiles
 # covers: ragged M, N and K, rows at a 2-byte phase, one K step and several,
 # a tile count that is no multiple of the eight XCDs.
