@@ -2059,19 +2059,20 @@ void ksplit_kernel(const T* __restrict__ A, const T* __restrict__ B, float* __re
     if (b_end) b_end_value = B[static_cast<std::size_t>(K) * N - 1];
   }
 
-  // Sums. kFold (every instance of few rows, which replaced kernels that cut K
-  // into chunks of 512): the products of each two steps start new chains of
-  // additions in kSets sets of sums, which are then added to `total`; four
-  // steps per chain from kLongSteps steps per wavefront on, where the additions
-  // to the total weigh more than the chains. Elsewhere a step's products go to
-  // one of kSets sets in turn, merged at the end (128 x 128 tiles, which ran
-  // there before, sum all of K in one chain). Measured on MI355X, relative
-  // 2-norm of the error against 64 bits (chunks of 512 before / two or four
-  // sets, no total / now): fp32 40 x 12288 x 12288 2.3e-7 / 5.0e-7 / 1.7e-7,
-  // 64 x 12288 x 12288 2.3e-7 / 3.6e-7 / 1.5e-7, 8 x 12288 x 2700 1.26e-7 /
-  // 1.77e-7 / 1.26e-7, fp16 32 x 12288 x 12288 1.3e-7 / 1.9e-7 / 1.1e-7; times
-  // within 5% of those without a total (fp32 64 x 4096 x 4096 24.2 -> 24.9 us).
-  constexpr bool kFold = FM <= (kSize == 2 ? 2 : 4);
+  // Sums. kFold: the products of each two steps (four from kLongSteps steps per
+  // wavefront on) start new chains of additions in kSets sets of sums, which are
+  // then added to `total`: the kernels that ran few rows before cut K into chunks
+  // of 512. The others, for medium grids, put a step's products into one of kSets
+  // sets in turn, merged at the end: short of registers (fp32 96-row tiles) or
+  // (fp16) well below the errors of the 128 x 128 tiles before, which sum all of K
+  // in one chain. Measured on MI355X, relative 2-norm of the error against 64 bits
+  // (kernels before / up to four sets, no total / now): fp32 40 x 12288 x 12288
+  // 2.3e-7 / 5.0e-7 / 1.8e-7, 64 x 12288 x 12288 2.3e-7 / 3.6e-7 / 1.5e-7, 8 x
+  // 12288 x 2700 1.26e-7 / 1.77e-7 / 1.26e-7, 128 x 8192 x 8192 5.8e-7 / 4.1e-7 /
+  // 1.7e-7, fp16 32 x 12288 x 12288 1.3e-7 / 1.9e-7 / 1.1e-7; times within 3% of
+  // those without a total (128 x 8192 x 8192 133.1 -> 136.1 us; 5% at a fold
+  // every two steps).
+  constexpr bool kFold = FM <= (sizeof(T) == 4 ? 5 : 2);
   constexpr int kSets = FM <= 2 ? 2 : kFold ? 1 : (kWaves == 4 || FM <= 5) ? 2 : 1;
   constexpr int kLongSteps = 16;
   const floatx4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -2188,7 +2189,7 @@ void ksplit_kernel(const T* __restrict__ A, const T* __restrict__ B, float* __re
   int s = wave;
   issue(st0, s);
   issue(st1, s + kWaves);
-  if constexpr (FM <= 2) {
+  if constexpr (kFold) {
     if (steps >= kLongSteps * kWaves) {
       for (; s + 3 * kWaves < steps; s += 4 * kWaves) {
         tile(st0, s, Index<0>{});

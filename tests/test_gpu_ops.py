@@ -567,8 +567,9 @@ def test_gemm_ksplit(hip, mnk, offset, dtype):
         assert np.linalg.norm(y - ref) <= 1e-4 * np.linalg.norm(ref)
 
 
-# Few rows on wide products, where K is not split over workgroups: the error
-# against 64 bits stays within that of K summed in chunks of 512. Additions of
+# Few rows on wide products, where K is not split over workgroups (and the 48- to
+# 80-row fp32 tiles of medium grids): the error against 64 bits stays within that
+# of K summed in chunks of 512. Additions of
 # equal random terms one after another leave a relative error of about 0.43 2^-24
 # (a uniform rounding error over a mantissa's range) times the root of half
 # their number. fp32: chains of 128 per chunk (32 for M <= 8, on 16 lane
@@ -578,6 +579,7 @@ def test_gemm_ksplit(hip, mnk, offset, dtype):
     ("f32", 40, 12288, 12288, 64 + 2), ("f32", 64, 8192, 12288, 64 + 2),
     ("f32", 33, 9000, 9000, 64 + 2), ("f32", 16, 12288, 12288, 64 + 2),
     ("f32", 8, 12288, 2700, 16 + 8), ("f32", 8, 8192, 4032, 16 + 8),
+    ("f32", 128, 8192, 8192, 64 + 2), ("f32", 300, 4096, 4096, 64 + 2),
     ("f16", 32, 12288, 12288, 16 + 2), ("f16", 22, 9152, 10624, 16 + 2)])
 def test_gemm_few_rows_error(ops, dtype, m, n, k, halves):
     g = torch.Generator(device="cuda").manual_seed(950 + m)
