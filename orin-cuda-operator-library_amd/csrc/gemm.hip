@@ -2269,9 +2269,10 @@ void ksplit_kernel(const T* __restrict__ A, const T* __restrict__ B, float* __re
 }
 
 constexpr int kMaxSplits = 16;
-// Fewer than 8 tiles would leave half the CUs idle at 16 splits (products of few
-// rows and columns and a long K): up to 256 there, in steps of a half.
-constexpr int kMaxSplitsFewTiles = 256;
+// Up to 8 tiles would leave half the CUs idle or more at 16 splits (products of
+// few rows and columns and a long K): from there in steps of a half, 181 at the
+// most (fp16 16 x 512 x 262144, 8 tiles, us: 85 on 16 splits, 60 on 64).
+constexpr int kMaxSplitsFewTiles = 181;
 // B that one row of tiles reads once, and that fills half the Infinity Cache
 // or more, is copied with the non-temporal hint. Measured on MI355X (us,
 // cached -> non-temporal, three sets of inputs / twenty): fp16 16 x 8192 x
@@ -2820,7 +2821,7 @@ ksplit::Plan ksplit_plan(int m, int n, int k, bool few_rows, std::size_t capacit
     // (8 x 8192 x 8192, us: 128 x 2 workgroups 48.0, x 4 55.6).
     const bool pairs = fm == 1 && (sizeof(T) == 2 || (static_cast<double>(m) + n) * k * sizeof(T) < kCachedUpTo);
     const long long slots = static_cast<long long>(cus) * (pairs ? 2 : 1);
-    const int max_splits = tiles < 8 ? ksplit::kMaxSplitsFewTiles : ksplit::kMaxSplits;
+    const int max_splits = tiles <= 8 ? ksplit::kMaxSplitsFewTiles : ksplit::kMaxSplits;
     for (int splits = 1; splits <= max_splits; splits += splits < 16 ? 1 : splits / 2) {
       // one split, or a grid the CUs hold at once with a step per wavefront
       if (splits > 1 && (tiles * splits > slots || k / (8 * dma::Elem<T>::kSubK) < splits)) break;

@@ -67,3 +67,17 @@ def test_few_rows_past_the_offset_limits(plans):
         assert plan["kind"] == kind, (case, plan)
         if mfma is not None:
             assert plan["mfma"] == mfma, (case, plan)
+
+
+def _check(plans, routes):
+    """routes: (call, what its plan must hold)."""
+    for (case, want), plan in zip(routes, plans([case for case, _ in routes])):
+        assert {key: plan.get(key) for key in want} == want, (case, plan)
+
+
+def test_eight_tiles_split_past_sixteen(plans):
+    """Eight 64-column tiles on 16 splits of K would leave half the CUs idle."""
+    _check(plans, [(("f16", 16, 512, 262144), dict(kind="split", fm=1, splits=54)),
+                   (("f16", 3, 512, 262144), dict(kind="split", fm=1, splits=54)),
+                   (("f16", 16, 576, 262144), dict(kind="split", fm=1, splits=16)),
+                   (("f16", 5, 16, 1 << 20), dict(kind="split", fm=1, splits=181))])
