@@ -2744,8 +2744,12 @@ TailPlan tail_plan(int m, int n, int k, std::size_t capacity) {
 // 1..8000, N and K 100..12288. What bounds these grids is the L2: a CU's
 // copies arrive at 64-75 bytes/ns (the eight L2s together deliver about 17
 // TB/s), so a tile of R x C costs (R + C) K elements per round of
-// workgroups; fp32 tiles cost their matrix-core time, 4.1 ns per 16 rows
-// and k of a 64-column tile. Rows off 64 bytes straddle twice the lines.
+// workgroups; fp32 tiles cost their matrix-core time, 3.7 ns per 16 rows and
+// k of a 64-column tile and 1.0 per k (B's fragments; 1.5 for 16 rows in several
+// rounds), after 3.5 us for 16 rows
+// and 0.4 more for each further 16 (82..112 timings of each height, 3-5% off
+// this line; with 4.1 ns throughout fp32 96 x 12288 x 12288 took 16-row tiles, 341
+// us against 280 on 96-row ones). Rows off 64 bytes straddle twice the lines.
 // The operands' stream from memory grows with the workgroups that ask for it
 // (towards 5500 bytes/ns, or 8000 where they fit the Infinity Cache several
 // times over); partial sums cost a launch and their traffic.
@@ -2765,7 +2769,9 @@ double ksplit_ns(int fm, int splits, int m, int n, int k, int cus) {
   const bool off_line = (n * sizeof(T)) % 64 != 0 || (k * sizeof(T)) % 64 != 0;
   const double copies = (16.0 * fm + 64) * k * size / splits / kTileBytesPerNs *
                         (off_line ? kOffLineFactor : 1.0);
-  const double mfma = sizeof(T) == 4 ? fm * static_cast<double>(k) / splits * 4.1 : 0.0;
+  const double mfma =
+      sizeof(T) == 4 ? (3.7 * fm + (fm == 1 && rounds > 1 ? 1.5 : 1.0)) * k / splits : 0.0;
+  const double start = sizeof(T) == 4 ? 2100 + 400.0 * fm : kNsRound;
   // (the shorter operand is read by every XCD, mostly from the Infinity Cache)
   const double operands = (std::max(m, n) + 4.0 * std::min(m, n)) * k * size;
   const bool cached = operands < kCachedUpTo;
@@ -2776,7 +2782,7 @@ double ksplit_ns(int fm, int splits, int m, int n, int k, int cus) {
   const double again = !cached && n >= m && m > 16 * fm ? 1.3 : 1.0;
   const double stream =
       operands / ((cached ? kCacheBytesPerNs : kMemoryBytesPerNs) * asked) * uneven * again;
-  return kNsLaunch + starts * kNsRound + std::max(rounds * std::max(copies, mfma), stream) +
+  return kNsLaunch + starts * start + std::max(rounds * std::max(copies, mfma), stream) +
          (splits > 1 ? kNsSum + 8.0 * splits * m * n / kPartialBytesPerNs : 0.0);
 }
 
@@ -2825,6 +2831,9 @@ ksplit::Plan ksplit_plan(int m, int n, int k, bool few_rows, std::size_t capacit
     for (int splits = 1; splits <= max_splits; splits += splits < 16 ? 1 : splits / 2) {
       // one split, or a grid the CUs hold at once with a step per wavefront
       if (splits > 1 && (tiles * splits > slots || k / (8 * dma::Elem<T>::kSubK) < splits)) break;
+      // fp32 96-row tiles hold no total: short chains only (96 x 12288 x 12288 in
+      // one, error against 64 bits 7.0e-7; on 48-row tiles 1.7e-7)
+      if (sizeof(T) == 4 && fm == 6 && k / splits > 3072) continue;
       const std::size_t bytes =
           splits > 1 ? static_cast<std::size_t>(splits) * m * n * sizeof(float) : 0;
       if (bytes > capacity) break;
@@ -2839,10 +2848,11 @@ ksplit::Plan ksplit_plan(int m, int n, int k, bool few_rows, std::size_t capacit
   }
   if (!few_rows) {
     // (whole rounds of unsplit tiles are estimated closely: a near tie there,
-    // fp16 5184 x 896 x 11712 170 against 175 us, is theirs)
+    // fp16 5184 x 896 x 11712 170 against 175 us, is theirs; an fp32 tie is
+    // ksplit_kernel's, whose chains of additions are shorter)
     const TailPlan tail = tail_plan<T>(m, n, k, capacity);
-    if (small_tiles_ns<T>(m, n, k, cus, tail) * (tail.splits > 0 ? 1.0 : 0.95) < best_ns)
-      return ksplit::Plan{};
+    const double bias = (tail.splits > 0 ? 1.0 : 0.95) * (sizeof(T) == 4 ? 1.08 : 1.0);
+    if (small_tiles_ns<T>(m, n, k, cus, tail) * bias < best_ns) return ksplit::Plan{};
   }
   // 128-byte A rows once each wavefront walks enough of them. Measured on
   // MI355X, fp16 (us, Wide vs Deep): 300 x 4096 x 4096 20.2 vs 18.4, 300 x

@@ -81,3 +81,15 @@ def test_eight_tiles_split_past_sixteen(plans):
                    (("f16", 3, 512, 262144), dict(kind="split", fm=1, splits=54)),
                    (("f16", 16, 576, 262144), dict(kind="split", fm=1, splits=16)),
                    (("f16", 5, 16, 1 << 20), dict(kind="split", fm=1, splits=181))])
+
+
+def test_fp32_tile_heights(plans):
+    """Matrix-core time per row falls with the tile's height (B's fragments), so a
+    long K does not run on 16-row tiles by default; 96-row tiles, which hold no
+    total of short chains, take up to 3072 of K each."""
+    _check(plans, [(("f32", 96, 12288, 12288), dict(kind="split", fm=3, splits=1)),
+                   (("f32", 64, 12288, 12288), dict(kind="split", fm=4, splits=1)),
+                   (("f32", 80, 11008, 4096), dict(kind="split", fm=5, splits=1)),
+                   (("f32", 1146, 2816, 3968), dict(kind="split", fm=5, splits=1)),
+                   (("f32", 96, 12288, 1024), dict(kind="split", fm=6, splits=1)),
+                   (("f32", 1000, 1000, 1000), dict(kind="split", fm=4, splits=1))])
