@@ -1170,12 +1170,12 @@ struct Cfg {
   // 1024^2 6.7 vs 6.5.
   static constexpr int kUpToM = sizeof(T) == 2 ? 2 : 4;
   static constexpr std::size_t kMinBytes = sizeof(T) == 2 ? std::size_t(8) << 20 : 0;
-  // Past ksplit_kernel's offsets skinny_mfma_kernel runs from kMfmaMinM to
-  // kMaxMfmaM rows (2 row blocks of 16, fp32 4). Measured on MI355X (us, this
-  // kernel vs skinny_mfma_kernel): fp16 M = 8 (N = 16, K = 2^25) 4190 vs 3860,
-  // M = 16 6150 vs 4020, M = 16 (N = 2^24 + 8, K = 72) 2390 vs 1150; fp32 M = 16
-  // (N = 16, K = 2^23) 1220 vs 950. 20 rows on the register-staged kernel 1.06 s
-  // vs 4210 us (fp16), 598 ms vs 1070 us (fp32).
+  // skinny_mfma_kernel's range: from kMfmaMinM to kMaxMfmaM rows past
+  // ksplit_kernel's offsets, up to 32 where skinny_mfma_faster (2 row blocks of
+  // 16, fp32 4). Measured on MI355X (us, this kernel vs skinny_mfma_kernel): fp16
+  // M = 8 (N = 16, K = 2^25) 4190 vs 3860, M = 16 6150 vs 4020, M = 16 (N = 2^24 +
+  // 8, K = 72) 2390 vs 1150; fp32 M = 16 (N = 16, K = 2^23) 1220 vs 950. 20 rows on
+  // the register-staged kernel 1.06 s vs 4210 us (fp16), 598 ms vs 1070 us (fp32).
   static constexpr int kMfmaMinM = sizeof(T) == 2 ? 5 : 9;
   static constexpr int kMaxMfmaM = sizeof(T) == 2 ? 32 : 64;
 };
@@ -1365,7 +1365,8 @@ void skinny_kernel(
 }
 
 // Matrix-core variant for M up to 32 (fp16) or 64 (fp32), in row blocks of 16,
-// where K or N passes ksplit_kernel's 32-bit offsets (64-bit addresses here):
+// where K or N passes ksplit_kernel's 32-bit offsets (64-bit addresses here) or
+// B's stream from memory is faster so (skinny_mfma_faster):
 // one v_mfma_f32_16x16x16_f16 (fp16) or v_mfma_f32_16x16x4_f32 (fp32) turns 16
 // rows of A times a 16 x 16 block of B into a 16 x 16 block of C, where the
 // vector-ALU kernel spends one dot product per (m, column pair) and becomes
@@ -1632,7 +1633,14 @@ bool applies(const T* b, int m, int n, int k, bool wide) {
   // throughout (us, this kernel vs ksplit_kernel): 8 x 8192 x 8192 52.0 vs
   // 48.8, 8 x 32000 x 4096 100 vs 89, but 5 x 8576 x 9856 62.8 vs 74.5, 8 x
   // 12288 x 12288 111 vs 119.
-  const int up_to = sizeof(T) == 4 && bytes >= (std::size_t(128) << 20) ? 8 : Cfg<T>::kUpToM;
+  // fp16 up to M = 4 on a B from memory that gives ksplit_kernel at most a
+  // workgroup per CU, or a long K (M = 3, us, this kernel vs ksplit_kernel): 12288
+  // x 12288 54.8 vs 66.0, 12288 x 4096 22.0 vs 23.1, 9216 x 12288 43.0 vs 43.8,
+  // 28672 x 8192 79.7 vs 94.6; 6144 x 12288 32.5 vs 29.3, 50304 x 4096 71.0 vs
+  // 71.4, 151936 x 4096 212 vs 190.
+  const bool memory = bytes >= (std::size_t(96) << 20) && n >= 8192 && (n <= 16384 || k >= 6144);
+  const int up_to = sizeof(T) == 4 ? (bytes >= (std::size_t(128) << 20) ? 8 : Cfg<T>::kUpToM)
+                                   : (memory ? 4 : Cfg<T>::kUpToM);
   return n % Cfg<T>::kPerLane == 0 && opl::aligned16(b) &&
          (wide ? m <= Cfg<T>::kMaxMfmaM : m <= up_to && bytes >= Cfg<T>::kMinBytes);
 }
@@ -2740,8 +2748,8 @@ TailPlan tail_plan(int m, int n, int k, std::size_t capacity) {
 }
 
 // Time estimates (ns) that choose between ksplit_kernel's tile heights and
-// splits and the 128 x 128 tiles, from sweeps on MI355X of 150 shapes with M
-// 1..8000, N and K 100..12288. What bounds these grids is the L2: a CU's
+// splits and the 128 x 128 tiles, from sweeps on MI355X of 600 shapes with M
+// 1..8000, N and K 16..262144. What bounds these grids is the L2: a CU's
 // copies arrive at 64-75 bytes/ns (the eight L2s together deliver about 17
 // TB/s), so a tile of R x C costs (R + C) K elements per round of
 // workgroups; fp32 tiles cost their matrix-core time, 3.7 ns per 16 rows and
@@ -2758,6 +2766,42 @@ constexpr double kTileBytesPerNs = 75, kOffLineFactor = 1.8;
 constexpr double kCacheBytesPerNs = 8000, kMemoryBytesPerNs = 5500, kCachedUpTo = 80e6;
 constexpr double kPartialBytesPerNs = 2500, kTilePartialBytesPerNs = 4500;
 
+// Bytes of the operands' stream (the shorter one is read by every XCD, mostly
+// from the Infinity Cache).
+template <typename T>
+double stream_bytes(int m, int n, int k) {
+  return (std::max(m, n) + 4.0 * std::min(m, n)) * k * sizeof(T);
+}
+
+// One row of tiles (M <= 16 fm, N from kRowStreamFrom) streams B from memory: a
+// CU draws its columns' rows at a rate that falls with M and with the power of
+// two in B's row pitch (128-byte pieces a pitch apart meet in fewer channels;
+// rows off 64 bytes draw as slowly), and all CUs together up to a limit.
+// Measured on MI355X (bytes/ns per CU, workgroups): fp16 M = 8, K = 12288: N 8704 (pitch 17 KiB) 26.8 (136),
+// 10240 (20 KiB) 23.9 (160), 11264 (22 KiB) 22.8 (176), 12288 (24 KiB) 24.0 (192),
+// 11008 (21.5 KiB) 30.7 (172), 8832 (17.25 KiB) 36.2 (138), 10000 24.5 (157);
+// M = 24: 23.4, 22.5, 22.8, 22.9, 28.2, 33.4, 23.5; fp32 N 8704 and 12288 M = 9
+// 31, 27.8, M = 16 28.6, 26.1, M = 32 23.9, 22.5. fp16 N = 16384, 256
+// workgroups 5700 in all, N = 16000 6700, N = 50264 4300; fp32 N = 16384 6450.
+constexpr int kRowStreamFrom = 2048;
+constexpr double kRowCachedUpTo = 92e6;  // (11008 x 4096 still draws at the cache's rate)
+
+template <typename T>
+double row_stream_ns(int splits, int m, int n, int k, double wgs, int cus) {
+  constexpr bool kHalf = sizeof(T) == 2;
+  const std::size_t pitch = static_cast<std::size_t>(n) * sizeof(T);
+  const bool slow = pitch % 1024 == 0 || pitch % 64 != 0;
+  double rate = kHalf ? (slow ? 26 : pitch % 512 == 0 ? 31 : 35) - m / 8.0
+                      : std::max(22.0, 32 - 0.3 * m);
+  double total = !slow ? 6500 : pitch % 64 != 0 ? 4300 : kHalf ? 5700 : 6100;
+  // (fp16 K splits that leave each CU one workgroup keep less in flight than
+  // pairs do: 16 x 5120 x 13824 40.3 us on 240, 35.1 on 480)
+  if (kHalf && splits > 1 && wgs <= cus) rate *= 0.96, total *= 0.96;
+  const double turns = wgs <= 2.0 * cus ? std::ceil(wgs / cus) : wgs / cus;
+  return std::max(stream_bytes<T>(m, n, k) / total,
+                  turns * 64.0 * k * sizeof(T) / splits / rate);
+}
+
 template <typename T>
 double ksplit_ns(int fm, int splits, int m, int n, int k, int cus) {
   const double size = sizeof(T);
@@ -2772,16 +2816,19 @@ double ksplit_ns(int fm, int splits, int m, int n, int k, int cus) {
   const double mfma =
       sizeof(T) == 4 ? (3.7 * fm + (fm == 1 && rounds > 1 ? 1.5 : 1.0)) * k / splits : 0.0;
   const double start = sizeof(T) == 4 ? 2100 + 400.0 * fm : kNsRound;
-  // (the shorter operand is read by every XCD, mostly from the Infinity Cache)
-  const double operands = (std::max(m, n) + 4.0 * std::min(m, n)) * k * size;
+  const double operands = stream_bytes<T>(m, n, k);
   const bool cached = operands < kCachedUpTo;
-  const double asked = wgs / (wgs + (cached && sizeof(T) == 2 ? 25 : 60));
-  const double uneven = std::sqrt(std::max(1.0, rounds * cus / std::max<double>(wgs, cus)));
-  // (a long B from memory is fetched again by a second row of tiles in part:
-  // fp16 32 x 8192 x 8192 44.3 us on 16-row tiles, 31.4 on 32-row ones)
-  const double again = !cached && n >= m && m > 16 * fm ? 1.3 : 1.0;
-  const double stream =
-      operands / ((cached ? kCacheBytesPerNs : kMemoryBytesPerNs) * asked) * uneven * again;
+  double stream;
+  if (operands >= kRowCachedUpTo && m <= 16 * fm && n >= kRowStreamFrom) {
+    stream = row_stream_ns<T>(splits, m, n, k, wgs, cus);
+  } else {
+    const double asked = wgs / (wgs + (cached && sizeof(T) == 2 ? 25 : 60));
+    const double uneven = std::sqrt(std::max(1.0, rounds * cus / std::max<double>(wgs, cus)));
+    // (a long B from memory is fetched again by a second row of tiles in part:
+    // fp16 32 x 8192 x 8192 44.3 us on 16-row tiles, 31.4 on 32-row ones)
+    const double again = !cached && n >= m && m > 16 * fm ? 1.3 : 1.0;
+    stream = operands / ((cached ? kCacheBytesPerNs : kMemoryBytesPerNs) * asked) * uneven * again;
+  }
   return kNsLaunch + starts * start + std::max(rounds * std::max(copies, mfma), stream) +
          (splits > 1 ? kNsSum + 8.0 * splits * m * n / kPartialBytesPerNs : 0.0);
 }
@@ -2807,11 +2854,39 @@ double small_tiles_ns(int m, int n, int k, int cus, const TailPlan& tail) {
          (splits > 1 ? kNsSum + splits * tiles * 131072.0 / kTilePartialBytesPerNs : 0.0);
 }
 
-// ksplit_kernel's plan for shapes it is the fastest estimate for (fm == 0:
-// it is not). Every shape of the skinny range, whose rows would fill an
-// eighth of a 128-row tile; otherwise grids of few 256 x 256 tiles.
+// Few rows of B from memory on more than half as many columns' tiles as CUs
+// (N 8193..16384, or any N whose rows are off 64 bytes): ksplit_kernel cannot
+// split K without a second turn of some CUs, and may draw less than
+// skinny_mfma_kernel does on its 512 and more workgroups (time: a launch and B at
+// 4.0-5.3 bytes/ps). Measured on MI355X (us, ksplit_kernel vs
+// skinny_mfma_kernel): fp16 24 x 8704 x 12288 70.6 vs 56.5, 8 x 10240 x 12288 50.0
+// (three splits) vs 54.3, 24 x 10240 x 6144 38.8 vs 34.7, 8 x 12288 x 12288 68.7 vs
+// 64.3, 24 x 12288 x 12288 72.1 vs 76.1, 24 x 11008 x 12288 59.3 vs 66.9, 16 x
+// 50264 x 4096 106.9 vs 98.7; fp32 32 x 8704 x 12288 135 vs 118, 24 x 12288 x
+// 12288 134 vs 150.
 template <typename T>
-ksplit::Plan ksplit_plan(int m, int n, int k, bool few_rows, std::size_t capacity) {
+bool skinny_mfma_faster(const T* b, int m, int n, int k, int splits, double split_ns) {
+  using C = skinny::Cfg<T>;
+  const int cus = device_cus() > 0 ? device_cus() : 256;
+  const long long tiles = (n + ksplit::kBN - 1LL) / ksplit::kBN;
+  const bool off_line = static_cast<std::size_t>(n) * sizeof(T) % 64 != 0;
+  if (m < C::kMfmaMinM || m > 32 || n % C::kPerLane != 0 || !opl::aligned16(b) ||
+      tiles <= cus / 2 || (tiles > cus && !off_line) || stream_bytes<T>(m, n, k) < kRowCachedUpTo)
+    return false;
+  const double rate = m <= 16 ? 5500 - 50.0 * m : 4600 - 18.0 * m;
+  const double ns = 5000 + (m <= 16 ? 0 : sizeof(T) == 2 ? 1500 : 6000) +
+                    static_cast<double>(n) * k * sizeof(T) / rate;
+  // (split K on pairs of workgroups draws more than its estimate: 8 x 8704 x 12288
+  // 43.9 vs 47.7)
+  return ns * (splits > 1 ? 1.12 : 0.97) < split_ns;
+}
+
+// ksplit_kernel's plan for shapes it is the fastest estimate for (fm == 0:
+// it is not): few rows, which would fill an eighth of a 128-row tile, and
+// otherwise grids of few 256 x 256 tiles. `best_ns`: the estimate.
+template <typename T>
+ksplit::Plan ksplit_plan(int m, int n, int k, bool few_rows, std::size_t capacity,
+                         double* estimate) {
   const long long big_tiles = (m + 255LL) / 256 * ((n + 255LL) / 256);
   if (!few_rows && big_tiles >= DmaTiles<T>::kSmallBelow) return ksplit::Plan{};
   int cus = device_cus();
@@ -2823,10 +2898,7 @@ ksplit::Plan ksplit_plan(int m, int n, int k, bool few_rows, std::size_t capacit
     if (fm > 1 && (m + 16LL * (fm - 1) - 1) / (16 * (fm - 1)) == rows) continue;  // more padding
     const long long tiles = rows * ((n + ksplit::kBN - 1) / ksplit::kBN);
     if (tiles > 0x3fffffffLL) continue;
-    // Pairs of fm = 1 workgroups, but not of fp32 ones that stream from memory
-    // (8 x 8192 x 8192, us: 128 x 2 workgroups 48.0, x 4 55.6).
-    const bool pairs = fm == 1 && (sizeof(T) == 2 || (static_cast<double>(m) + n) * k * sizeof(T) < kCachedUpTo);
-    const long long slots = static_cast<long long>(cus) * (pairs ? 2 : 1);
+    const long long slots = static_cast<long long>(cus) * (fm == 1 ? 2 : 1);  // pairs of fm = 1
     const int max_splits = tiles <= 8 ? ksplit::kMaxSplitsFewTiles : ksplit::kMaxSplits;
     for (int splits = 1; splits <= max_splits; splits += splits < 16 ? 1 : splits / 2) {
       // one split, or a grid the CUs hold at once with a step per wavefront
@@ -2854,6 +2926,7 @@ ksplit::Plan ksplit_plan(int m, int n, int k, bool few_rows, std::size_t capacit
     const double bias = (tail.splits > 0 ? 1.0 : 0.95) * (sizeof(T) == 4 ? 1.08 : 1.0);
     if (small_tiles_ns<T>(m, n, k, cus, tail) * bias < best_ns) return ksplit::Plan{};
   }
+  *estimate = best_ns;
   // 128-byte A rows once each wavefront walks enough of them. Measured on
   // MI355X, fp16 (us, Wide vs Deep): 300 x 4096 x 4096 20.2 vs 18.4, 300 x
   // 4096 x 11008 59.9 vs 54.7; 1024^3 8.6 vs 8.8, 1000^3 10.8 vs 11.9.
@@ -2918,21 +2991,24 @@ GemmPlan plan_gemm(const T* a, const T* b, int m, int n, int k, std::size_t capa
   const bool few_rows = m <= (sizeof(T) == 2 ? 32 : 64);
   const bool split_offsets_fit =
       dma_offsets_fit || (few_rows && k < (sizeof(T) == 2 ? (1 << 25) : (1 << 23)) && n < (1 << 24));
-  if (skinny::applies(b, m, n, k, !split_offsets_fit)) {
+  auto take_skinny = [&] {
     p.skinny = skinny::plan<T>(m, n, k, capacity);
-    if (p.skinny.ok) {
-      p.kind = GemmPlan::kSkinny;
-      p.bytes = p.skinny.bytes;
-      return p;
-    }
-  }
+    if (!p.skinny.ok) return false;
+    p.kind = GemmPlan::kSkinny;
+    p.bytes = p.skinny.bytes;
+    return true;
+  };
+  if (skinny::applies(b, m, n, k, !split_offsets_fit) && take_skinny()) return p;
   if (!(few_rows && split_offsets_fit && n % skinny::Cfg<T>::kPerLane == 0) &&
       narrow::applies(a, b, n, k)) {
     p.kind = GemmPlan::kNarrow;
     return p;
   }
   if (split_offsets_fit) {
-    p.split = ksplit_plan<T>(m, n, k, few_rows, capacity);
+    double split_ns = 0;
+    p.split = ksplit_plan<T>(m, n, k, few_rows, capacity, &split_ns);
+    if (few_rows && skinny_mfma_faster(b, m, n, k, p.split.splits, split_ns) && take_skinny())
+      return p;
     if (p.split.fm > 0) {
       p.kind = GemmPlan::kSplit;
       p.bytes = p.split.bytes;

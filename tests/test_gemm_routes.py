@@ -93,3 +93,25 @@ def test_fp32_tile_heights(plans):
                    (("f32", 1146, 2816, 3968), dict(kind="split", fm=5, splits=1)),
                    (("f32", 96, 12288, 1024), dict(kind="split", fm=6, splits=1)),
                    (("f32", 1000, 1000, 1000), dict(kind="split", fm=4, splits=1))])
+
+
+def test_few_rows_from_memory(plans):
+    """B past the Infinity Cache: each kernel where it draws the faster stream
+    (measured times beside the rules: row_stream_ns, skinny_mfma_faster and
+    skinny::applies), and the cached calls as they were."""
+    _check(plans, [(("f16", 24, 8704, 12288), dict(kind="skinny", mfma=1)),
+                   (("f16", 8, 12288, 12288), dict(kind="skinny", mfma=1)),
+                   (("f16", 16, 50264, 4096), dict(kind="skinny", mfma=1)),
+                   (("f32", 32, 8704, 12288), dict(kind="skinny", mfma=1)),
+                   (("f16", 3, 12288, 12288), dict(kind="skinny", mfma=0)),
+                   (("f16", 3, 28672, 8192), dict(kind="skinny", mfma=0)),
+                   (("f16", 3, 6144, 12288), dict(kind="split", fm=1, splits=5)),
+                   (("f16", 24, 11008, 12288), dict(kind="split", fm=2, splits=1)),
+                   (("f32", 24, 12288, 12288), dict(kind="split", fm=2, splits=1)),
+                   (("f16", 16, 16384, 8192), dict(kind="split", fm=1, splits=1)),
+                   (("f16", 16, 5120, 13824), dict(kind="split", fm=1, splits=6)),
+                   (("f32", 16, 8704, 12288), dict(kind="split", fm=1, splits=3)),
+                   # B off 16 bytes: ksplit_kernel at any alignment
+                   (("f16", 8, 12288, 12288, 0, 1), dict(kind="split", fm=1)),
+                   (("f16", 16, 11008, 4096), dict(kind="split", fm=1, splits=1)),
+                   (("f16", 16, 4096, 4096), dict(kind="split", fm=1, splits=3))])
