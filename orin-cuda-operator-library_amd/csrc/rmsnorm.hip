@@ -436,7 +436,8 @@ int rmsnorm_launch(const Args<T>& args, const opl::ScratchSource& src, hipStream
   const std::size_t bytes = split_bytes(args.rows, split);
   if (src.workspace_mode && !opl::workspace_ok(src.data, src.bytes, bytes))
     return hipErrorInvalidValue;
-  if (split.run<T>(hidden, opl::same_phase16(args.input, args.output))) {
+  if (split.run(hidden, opl::same_phase16(args.input, args.output),
+                opl::rmsnorm_split_above<T>(args.rows))) {
     // 4 bytes per (row, segment): fewer than 2 * kSplitTargetBlocks for
     // split rows, one per row otherwise; every plan fits the arena.
     opl::ScratchLease lease(stream, src.workspace_mode ? src.data : nullptr, src.bytes);

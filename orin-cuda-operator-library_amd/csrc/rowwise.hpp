@@ -303,34 +303,44 @@ struct Segment {
 // are that many rows); register-resident rows of a workgroup (kRowWaveMaxCols
 // < cols <= kRowBlockMaxCols) only when there are fewer than kSplitMaxRows
 // of them, which would leave most CUs idle, and they are longer than
-// kSplitAboveCols.
+// SplitAbove says.
 constexpr int kSplitThreads = 256;
 constexpr int kSplitWaves = kSplitThreads / kWaveSize;
 constexpr int kSplitUnroll = 4;          // 16-byte chunks in flight per thread
 constexpr int kSplitTargetBlocks = 512;  // two workgroups per CU of a 256-CU MI355X
 constexpr int kSplitMinSegment = 2048;   // elements
 constexpr int kSplitMaxRows = 64;
-// The split kernels run above these widths. A row in one workgroup's
-// registers needs one launch and no second read, and up to here that costs
-// less than the few CUs it keeps busy. Measured on MI355X (us, split -> one
-// workgroup per row): softmax fp16 1 x 12288 4.5 -> 2.9, 16 x 5120 5.1 -> 2.6,
-// 63 x 32768 6.7 -> 5.3; fp32 16 x 16384 5.0 -> 3.5, 16 x 24576 5.2 -> 4.7, 1 x
-// 32768 5.2 -> 5.4; RMSNorm fp32 16 x 8192 4.6 -> 2.7, 63 x 24576 6.0 -> 6.1, 1
-// x 32768 4.6 -> 5.7.
+// The split kernels run above these widths: `same` where input and output share
+// their 16-byte phase, `mixed` where they do not (element by element). A row in
+// one workgroup's registers needs one launch and no second read, and up to here
+// that costs less than the few CUs it keeps busy. Measured on MI355X (us, split
+// -> one workgroup per row): softmax fp16 1 x 12288 4.5 -> 2.9, 16 x 5120 5.1 ->
+// 2.6, 63 x 32768 6.5 -> 5.3, fp32 16 x 16384 5.0 -> 3.5, 63 x 24576 6.2 -> 6.0, 1 x
+// 32768 5.2 -> 5.4, mixed 16 x 12288 5.2 -> 3.6, 63 x 16384 5.9 -> 5.1; RMSNorm fp16
+// 16 x 32768 4.6 -> 4.5, 63 x 32768 5.9 -> 5.1, mixed 63 x 16384 5.2 -> 4.5, fp32 16 x
+// 16384 4.5 -> 3.6, 63 x 16384 5.4 -> 4.8, past it 1 x 20480 4.6 -> 4.3, 4 x 24576 4.5 ->
+// 4.5 but 16 x 24576 4.6 -> 5.3, 32 x 20480 4.9 -> 5.3; mixed 16 x 16384 4.6 -> 4.2 but
+// 32 x 16384 4.7 -> 5.1.
+struct SplitAbove {
+  int same, mixed;
+};
 template <typename T>
-constexpr int kSplitAboveCols = sizeof(T) == 2 ? 32768 : 24576;
-// Input and output in different 16-byte phases: element by element (softmax
-// fp32 16 x 12288 5.2 -> 3.6, fp16 63 x 20000 6.3 -> 7.9).
-constexpr int kSplitAboveMixedCols = 16384;
+constexpr SplitAbove softmax_split_above() {
+  return {sizeof(T) == 2 ? 32768 : 24576, 16384};
+}
+template <typename T>
+constexpr SplitAbove rmsnorm_split_above(int rows) {
+  if (sizeof(T) == 2) return {32768, 16384};
+  return {rows <= 4 ? 24576 : 16384, rows <= 16 ? 16384 : 12288};
+}
 
 struct SplitPlan {
   int segments = 0;  // 0: not split
   int seg_len = 0;   // elements, a multiple of 64
   // Whether to launch the split kernels: a workspace is asked for and checked
   // by `segments` alone, so queries and refusals keep their meaning.
-  template <typename T>
-  bool run(int cols, bool same_phase) const {
-    return segments > 0 && cols > (same_phase ? kSplitAboveCols<T> : kSplitAboveMixedCols);
+  bool run(int cols, bool same_phase, SplitAbove above) const {
+    return segments > 0 && cols > (same_phase ? above.same : above.mixed);
   }
 };
 

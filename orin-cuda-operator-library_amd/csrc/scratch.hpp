@@ -8,7 +8,7 @@
 // means fewer splits or a slower kernel, never an error):
 //   * reduce: one fp64 partial per workgroup (at most 2 KiB);
 //   * softmax and RMSNorm rows split over workgroups (rows longer than
-//     32768 columns, or few rows longer than kSplitAboveCols): one partial
+//     32768 columns, or few rows longer than SplitAbove says): one partial
 //     per row and segment (8 or 4 bytes);
 //   * decode and medium GEMMs (skinny_kernel, ksplit_kernel): split-K partial
 //     sums;

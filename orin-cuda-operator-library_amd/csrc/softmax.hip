@@ -450,7 +450,7 @@ int softmax_launch(const T* input, T* output, int rows, int cols,
   const std::size_t bytes = split_bytes(rows, split);
   if (src.workspace_mode && !opl::workspace_ok(src.data, src.bytes, bytes))
     return hipErrorInvalidValue;
-  if (split.run<T>(cols, opl::same_phase16(input, output))) {
+  if (split.run(cols, opl::same_phase16(input, output), opl::softmax_split_above<T>())) {
     // 8 bytes per (row, segment): fewer than 2 * kSplitTargetBlocks pairs
     // for split rows, one per row otherwise (a matrix that fits in HBM has
     // far fewer rows than the arena holds pairs).
