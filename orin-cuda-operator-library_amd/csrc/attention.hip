@@ -1382,6 +1382,14 @@ constexpr int kThirtyTwoRowsUpTo = 768;
 // groups) lose: B1 H8 6.9 -> 7.0.
 constexpr long long kThirtyTwoRowsCausalF32 = 768;
 constexpr int kThirtyTwoRowsCausalFrom = 512;
+// fp32 D64, every key visible: 48 rows per wavefront where that is one round (and
+// 32-row blocks are not) and four groups walk the keys in half the tiles that two
+// do, or nearly (us, 64-row blocks of two groups -> 48-row): H48 S192 11.6 -> 12.5
+// (2 tiles for 3), S240 14.4 -> 13.8 (2 for 4); H32 S257 16.1 -> 17.0, S272 16.3 ->
+// 17.1, S288 16.0 -> 16.1, S289 16.6 -> 16.2 (3 for 5), S336 18.5 -> 16.5 (3 for 6);
+// H64 S160 11.4 -> 12.4; H16 S513 25.4 -> 23.2, S640 27.3 -> 23.3; H12 S1000 41.7 ->
+// 34.7; H8 S1025 43.9 -> 37.0, S1536 59.8 -> 47.4; H1 S12288 451 -> 335.
+constexpr int kFortyEightRowsFrom = 289;
 // fp16 D64 causal grids from 768 tokens gain up to two: B1 H12 S1000 12.5 ->
 // 11.6, B1 H8 S2048 19.5 -> 16.4.
 constexpr long long kThirtyTwoRowsCausalF16 = 512;
@@ -1444,9 +1452,8 @@ void launch(const T* q, const T* k, const T* v, float* out, int bh, int s, int d
         (rows32 <= kOneRound ||
          (causal && s >= kThirtyTwoRowsCausalFrom && rows32 <= kThirtyTwoRowsCausalF32))) {
       OPL_RUN(64, 4, 1, 32);
-    } else if (!wide && s > 64 && !causal && rows48 <= kOneRound) {
-      // 48 rows per wavefront, where that is one round: B1 H12 S1000 44.5 ->
-      // 36.2 us
+    } else if (!wide && !causal && rows48 <= kOneRound &&
+               (s >= kFortyEightRowsFrom || (s > 192 && s <= 256))) {
       OPL_RUN(64, 4, 1, 32, 64, 3);
     } else if (wide && half_rows) {
       if (d96) OPL_RUN(128, 2, 2, 32, 96);

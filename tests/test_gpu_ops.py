@@ -1216,7 +1216,8 @@ PADDED_CASES = [(2, 333, 96, False), (12, 1000, 80, True), (100, 300, 96, True),
 # wavefront: both precisions, D 64, fp16 128 and 96 (80 and 72 inside), fewer
 # tiles than groups, one row past a block, the last length and grid on that
 # side of the rule (fp16 768 tokens; 256 blocks, causal fp32 D 64 768, fp16 D
-# 64 512). 48-row blocks (fp32 D 64, 257..341 blocks of 32 rows). Four groups
+# 64 512). 48-row blocks (fp32 D 64, 257..384 blocks of 32 rows, 193..256 or 289
+# and more keys). Four groups
 # of two wavefronts (fp16 D 64 from 769 tokens).
 SMALL_BLOCKS = [("f16", 1, 1, 128, False), ("f16", 3, 33, 128, True), ("f16", 16, 512, 128, True),
                 ("f16", 16, 512, 64, False), ("f16", 5, 97, 64, True), ("f16", 4, 289, 96, True),
@@ -1224,6 +1225,7 @@ SMALL_BLOCKS = [("f16", 1, 1, 128, False), ("f16", 3, 33, 128, True), ("f16", 16
                 ("f32", 1, 65, 64, False), ("f32", 3, 129, 64, True), ("f32", 8, 1024, 64, False),
                 ("f32", 24, 1001, 64, True), ("f32", 9, 1000, 64, False),
                 ("f32", 32, 257, 64, False), ("f32", 10, 900, 40, False),
+                ("f32", 32, 289, 64, False), ("f32", 43, 240, 64, False),
                 ("f16", 2, 768, 64, True), ("f16", 10, 768, 128, False), ("f16", 16, 1000, 64, False),
                 ("f16", 5, 1031, 56, True), ("f16", 16, 1000, 64, True), ("f16", 16, 1025, 64, False),
                 ("f32", 2, 333, 96, True), ("f32", 50, 500, 72, False), ("f32", 300, 150, 96, True)]

@@ -84,3 +84,22 @@ def test_few_rows_split_or_not(launches):
     for (call, want), got in zip(cases, launches([call for call, _ in cases])):
         assert len(got) == want, (call, got)
         assert (want == split) == ("split" in got[0][0]), (call, got)
+
+
+def _instances(launches, calls):
+    """[D, groups, wavefronts, tile keys, computed dims, row blocks] per call."""
+    got = launches([("attention", *call) for call in calls])
+    assert all(len(g) == 1 and g[0][0] == "attention_dma_kernel" for g in got), got
+    return [g[0][1] for g in got]
+
+
+def test_attention_48_row_blocks(launches):
+    """fp32 D64 with every key visible: 48 rows per wavefront only where four key
+    groups walk (nearly) half the tiles of two, on both sides of each line."""
+    calls = [(32, 257, False), (32, 288, False), (32, 289, True), (24, 512, False),
+             (64, 192, False), (48, 193, True), (48, 256, False), (42, 256, True),
+             (80, 128, False), (16, 513, True), (16, 768, True), (16, 769, False),
+             (1, 8193, True), (8, 1000, False)]
+    got = _instances(launches, [("f32", 1, h, s, 64, 0) for h, s, _ in calls])
+    for (h, s, want), inst in zip(calls, got):
+        assert (inst == [64, 4, 1, 32, 64, 3]) == want, (h, s, inst)
