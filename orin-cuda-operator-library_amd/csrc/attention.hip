@@ -1369,12 +1369,12 @@ void launch_instance(const T* q, const T* k, const T* v, float* out, int bh, int
 // two wavefronts wait for each other's tile. Measured on MI355X (us, 64-row
 // blocks before -> 32-row; non-causal / causal): fp16 D128 B1 H12 S128 7.9 ->
 // 6.4 / 8.4 -> 7.0, B1 H32 S256 9.5 -> 8.4 / 10.6 -> 9.3, B1 H12 S512 11.6 ->
-// 10.5 / 12.6 -> 11.4, B1 H4 S700 13.0 -> 12.2 / 13.9 -> 12.2, B1 H12 S1000 (384
-// blocks) 17.2 -> 29.7; D64 S512 8.0 -> 7.2 / 8.9 -> 7.5; fp32 D64 S128 9.4 ->
-// 7.4 / 10.4 -> 8.0, S512 24.1 -> 16.4 / 24.9 -> 16.7. fp16 stops at 768 tokens
-// (the K and V of a head are fetched once per block).
+// 10.5 / 12.6 -> 11.4, B1 H8 S768 12.7 -> 12.0 / 13.6 -> 12.2, S1024 15.3 -> 14.1 /
+// 16.0 -> 14.6, H4 S1500 19.6 -> 18.5 / 19.5 -> 17.4, H1 S8192 75.5 -> 73.4 / 74.4 ->
+// 68.5, but B1 H12 S1000 (384 blocks) 17.2 -> 29.7; D96 H4 S1024 12.5 -> 12.0 / 13.6 ->
+// 12.1; D64 S512 8.0 -> 7.2 / 8.9 -> 7.5, H8 S1024 10.3 -> 9.1, H1 S8192 48.7 -> 43.2;
+// fp32 D64 S128 9.4 -> 7.4 / 10.4 -> 8.0, S512 24.1 -> 16.4 / 24.9 -> 16.7.
 constexpr long long kOneRound = 256;
-constexpr int kThirtyTwoRowsUpTo = 768;
 // fp32 D64 causal grids from 512 tokens gain up to three rounds, as the blocks
 // are ordered heaviest first: B1 H12 S1000 (384) 43.3 -> 33.5, B1 H8 S2048
 // (512) 81.3 -> 53.0, B1 H32 S700 (704) 44.9 -> 40.2, B2 H16 S1024 (1024) 57.1
@@ -1393,10 +1393,10 @@ constexpr int kFortyEightRowsFrom = 289;
 // fp16 D64 causal grids from 768 tokens gain up to two: B1 H12 S1000 12.5 ->
 // 11.6, B1 H8 S2048 19.5 -> 16.4.
 constexpr long long kThirtyTwoRowsCausalF16 = 512;
-// fp16 D64, 64-row blocks of one round: four groups of two wavefronts on
-// 32-key tiles instead of two on 64-key ones from this many tokens: B1 H12
-// S1024 11.9 -> 11.0, B1 H8 S2048 19.0 -> 16.9, causal 19.6 -> 17.8; S512 8.0
-// -> 8.1.
+// fp16 D64, 64-row blocks of one round (and 32-row ones of more): four groups of
+// two wavefronts on 32-key tiles instead of two on 64-key ones from this many
+// tokens: B1 H12 S1024 11.9 -> 11.0, B1 H8 S2048 19.0 -> 16.9, causal 19.6 ->
+// 17.8; S512 8.0 -> 8.1.
 constexpr int kFourGroupsFrom = 768;
 
 // Chooses the instance. `blocks`: 128-row query blocks. Grids too small to
@@ -1419,7 +1419,7 @@ void launch(const T* q, const T* k, const T* v, float* out, int bh, int s, int d
 #define OPL_RUN(...) \
   launch_instance<T, __VA_ARGS__>(q, k, v, out, bh, s, dm, causal, scale, stream)
   if constexpr (sizeof(T) == 2) {
-    if (rows32 <= kOneRound && s <= kThirtyTwoRowsUpTo) {
+    if (rows32 <= kOneRound) {
       if (d96) OPL_RUN(128, 4, 1, 32, 96);
       else if (wide) OPL_RUN(128, 4, 1, 32);
       else OPL_RUN(64, 4, 1, 32);

@@ -1214,11 +1214,10 @@ PADDED_CASES = [(2, 333, 96, False), (12, 1000, 80, True), (100, 300, 96, True),
 
 # One-round grids of small blocks. 32-row blocks on four key groups of one
 # wavefront: both precisions, D 64, fp16 128 and 96 (80 and 72 inside), fewer
-# tiles than groups, one row past a block, the last length and grid on that
-# side of the rule (fp16 768 tokens; 256 blocks, causal fp32 D 64 768, fp16 D
-# 64 512). 48-row blocks (fp32 D 64, 257..384 blocks of 32 rows, 193..256 or 289
-# and more keys). Four groups
-# of two wavefronts (fp16 D 64 from 769 tokens).
+# tiles than groups, one row past a block, the last grid on that side of the rule
+# (256 blocks, causal fp32 D 64 768, fp16 D 64 512) and long sequences. 48-row
+# blocks (fp32 D 64, 257..384 blocks of 32 rows, 193..256 or 289 and more keys).
+# Four groups of two wavefronts (fp16 D 64 from 768 tokens, 257 blocks of 32 rows).
 SMALL_BLOCKS = [("f16", 1, 1, 128, False), ("f16", 3, 33, 128, True), ("f16", 16, 512, 128, True),
                 ("f16", 16, 512, 64, False), ("f16", 5, 97, 64, True), ("f16", 4, 289, 96, True),
                 ("f16", 7, 130, 80, False), ("f16", 2, 64, 72, True), ("f16", 11, 200, 40, True),
@@ -1227,6 +1226,7 @@ SMALL_BLOCKS = [("f16", 1, 1, 128, False), ("f16", 3, 33, 128, True), ("f16", 16
                 ("f32", 32, 257, 64, False), ("f32", 10, 900, 40, False),
                 ("f32", 32, 289, 64, False), ("f32", 43, 240, 64, False),
                 ("f16", 2, 768, 64, True), ("f16", 10, 768, 128, False), ("f16", 16, 1000, 64, False),
+                ("f16", 8, 1024, 128, True), ("f16", 5, 1601, 96, False), ("f16", 2, 2049, 64, False),
                 ("f16", 5, 1031, 56, True), ("f16", 16, 1000, 64, True), ("f16", 16, 1025, 64, False),
                 ("f32", 2, 333, 96, True), ("f32", 50, 500, 72, False), ("f32", 300, 150, 96, True)]
 

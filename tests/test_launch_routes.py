@@ -103,3 +103,14 @@ def test_attention_48_row_blocks(launches):
     got = _instances(launches, [("f32", 1, h, s, 64, 0) for h, s, _ in calls])
     for (h, s, want), inst in zip(calls, got):
         assert (inst == [64, 4, 1, 32, 64, 3]) == want, (h, s, inst)
+
+
+def test_attention_one_round_of_32_row_blocks(launches):
+    """fp16: 32-row blocks on four key groups wherever their grid is one round."""
+    for d, layout, dims in ((128, 128, 128), (96, 128, 96), (64, 64, 64)):
+        calls = [(12, 640, 0, True), (8, 1024, 0, True), (8, 1025, 0, False),
+                 (8, 1024, 1, True), (4, 1500, 1, True), (1, 8192, 0, True),
+                 (1, 8193, 0, False), (12, 1024, 0, False)]
+        got = _instances(launches, [("f16", 1, h, s, d, c) for h, s, c, _ in calls])
+        for (h, s, c, want), inst in zip(calls, got):
+            assert (inst == [layout, 4, 1, 32, dims, 2]) == want, (d, h, s, c, inst)
