@@ -114,3 +114,14 @@ def test_attention_one_round_of_32_row_blocks(launches):
         got = _instances(launches, [("f16", 1, h, s, d, c) for h, s, c, _ in calls])
         for (h, s, c, want), inst in zip(calls, got):
             assert (inst == [layout, 4, 1, 32, dims, 2]) == want, (d, h, s, c, inst)
+
+
+def test_attention_one_key_tile(launches):
+    """fp16, up to 32 tokens (one key tile) on many heads: one group per block."""
+    calls = [(256, 17, False), (256, 32, False), (129, 1, False), (128, 33, True),
+             (12, 16, True)]
+    got = _instances(launches, [("f16", 1, h, s, 128, 0) for h, s, _ in calls])
+    for (h, s, want), inst in zip(calls, got):
+        assert (inst == [128, 4, 1, 32, 128, 2]) == want, (h, s, inst)
+        if h > 128:
+            assert inst == [128, 1, 2, 32, 128, 2], (h, s, inst)
