@@ -319,8 +319,8 @@ constexpr int kSplitMaxRows = 64;
 // 32768 5.2 -> 5.4, mixed 16 x 12288 5.2 -> 3.6, 63 x 16384 5.9 -> 5.1; RMSNorm fp16
 // 16 x 32768 4.6 -> 4.5, 63 x 32768 5.9 -> 5.1, mixed 63 x 16384 5.2 -> 4.5, fp32 16 x
 // 16384 4.5 -> 3.6, 63 x 16384 5.4 -> 4.8, past it 1 x 20480 4.6 -> 4.3, 4 x 24576 4.5 ->
-// 4.5 but 16 x 24576 4.6 -> 5.3, 32 x 20480 4.9 -> 5.3; mixed 16 x 16384 4.6 -> 4.2 but
-// 32 x 16384 4.7 -> 5.1.
+// 4.5 but 16 x 20480 4.6 -> 5.0, 16 x 24576 4.6 -> 5.3 (4.7 on another GPU), 32 x 20480
+// 4.9 -> 5.3 (5.2); mixed 16 x 16384 4.6 -> 4.3, 32 x 16384 4.7 -> 5.1 (4.5).
 struct SplitAbove {
   int same, mixed;
 };
@@ -331,7 +331,7 @@ constexpr SplitAbove softmax_split_above() {
 template <typename T>
 constexpr SplitAbove rmsnorm_split_above(int rows) {
   if (sizeof(T) == 2) return {32768, 16384};
-  return {rows <= 4 ? 24576 : 16384, rows <= 16 ? 16384 : 12288};
+  return {rows <= 4 ? 24576 : 16384, 16384};
 }
 
 struct SplitPlan {

@@ -74,8 +74,7 @@ def test_few_rows_split_or_not(launches):
                 elif op == "softmax":
                     same, mixed = 24576, 16384
                 else:
-                    same = 24576 if rows <= 4 else 16384
-                    mixed = 16384 if rows <= 16 else 12288
+                    same, mixed = 24576 if rows <= 4 else 16384, 16384
                 for offsets, width in (((0, 0), same), ((3, 3), same), ((1, 0), mixed)):
                     cases += [((op, dtype, rows, 4097, *offsets), one),
                               ((op, dtype, rows, width, *offsets), one),
