@@ -14,6 +14,9 @@ from pathlib import Path
 
 import pytest
 
+from test_gpu_ops import FEW_TILES, KSPLIT_TILES, ONE_ROUND, SPLIT_TILES
+from test_shared_stream_threads import KSPLIT_MNK, SPLIT_MNK
+
 HERE = Path(__file__).resolve().parent
 REPO = HERE.parent
 CSRC = REPO / "orin-cuda-operator-library_amd" / "csrc"
@@ -125,3 +128,29 @@ def test_one_round_tiles_keep_their_xcd_order(plans):
                    (("f16", 768, 7168, 4224), dict(kind="dma", rows=128, one_round=1)),
                    (("f16", 2000, 3000, 512), dict(kind="dma", rows=128, one_round=1)),
                    (("f16", 3000, 3000, 3000), dict(kind="dma", rows=192, one_round=1))])
+
+
+def test_gpu_tests_reach_the_instances_they_name(plans):
+    """The shapes of tests/test_gpu_ops.py that stand for an instance run it, so a
+    change of an estimate cannot move one off its kernel unseen."""
+    _check(plans, [((dtype, m, n, k), dict(kind="split", fm=fm, deep=deep, edge=edge))
+                   for dtype, m, n, k, fm, deep, edge in KSPLIT_TILES])
+    seen = {(c[0], *c[4:]) for c in KSPLIT_TILES}
+    assert {("f16", fm, deep, edge) for fm in range(2, 7) for deep in (0, 1)
+            for edge in (0, 1)} - {("f16", 2, 0, 0)} <= seen
+    assert {("f32", fm, 0, edge) for fm in (4, 5, 6) for edge in (0, 1)} <= seen
+    split_tiles = [*SPLIT_TILES, ("f16", *SPLIT_MNK)]
+    for case, plan in zip(split_tiles, plans(split_tiles)):
+        assert plan["kind"] == "dma" and plan["rows"] == 128 and plan["tail"] > 1, (case, plan)
+    # the workspace, stream and graph tests' users of the arena
+    _check(plans, [(("f16", *KSPLIT_MNK), dict(kind="split", splits=7)),
+                   (("f16", 16, 4096, 4096), dict(kind="split", splits=3)),
+                   (("f16", 24, 8704, 6144), dict(kind="skinny", mfma=1))])
+    cases = [(dtype, *c) for c in FEW_TILES for dtype in ("f16", "f32")]
+    splits = set()
+    for case, plan in zip(cases, plans(cases)):
+        assert plan["kind"] == "split" and plan["splits"] > 16, (case, plan)
+        splits.add(plan["splits"])
+    assert len(splits) >= 4, splits
+    got = plans([("f16", *c) for c in ONE_ROUND])
+    assert [p["rows"] * p.get("one_round", 0) for p in got] == [128] * 3 + [192] * 5 + [0, 0], got

@@ -198,10 +198,11 @@ def test_softmax_masked_rows(hip, shape):
 
 
 # A few rows of 4097 to 32768 columns: one workgroup per row up to 24576 fp32
-# columns (16384 when input and output phases differ), split above. Both
-# sides of those widths and of the powers of two that set a thread's share.
+# columns (RMSNorm 16384 from 5 rows on, both 16384 when input and output phases
+# differ), split above. Both sides of those widths and of the powers of two that
+# set a thread's share.
 FEW_ROWS = [(1, 4097), (3, 8192), (16, 8193), (2, 16384), (5, 16385), (2, 24576), (2, 24577),
-            (1, 32767)]
+            (1, 32767), (5, 16384), (4, 16385), (17, 24576)]
 
 
 @pytest.mark.parametrize("shape", FEW_ROWS)
@@ -519,17 +520,18 @@ def test_gemm_skinny_row_blocks(hip, mnk, dtype):
     assert np.isfinite(y).all()
 
 
-# ksplit_kernel, whose wavefronts split K: every tile height (16 to 96 rows)
-# one row short, exact and one over; N around its 64-column tiles; K around
-# its steps (32 / 16, 64 at K >= 2048) and fewer steps than wavefronts; odd K
-# and N (the end elements a copy's range check drops); K split over
-# workgroups too (first and last range of uneven ones); M > N, whose items
-# run in the other order.
+# ksplit_kernel, whose wavefronts split K: rows of a tile one short, exact and
+# one over; N around its 64-column tiles; K around its steps (32 / 16, 64 at K >=
+# 2048) and fewer steps than wavefronts; odd K and N (the end elements a copy's
+# range check drops); K split over workgroups too (first and last range of uneven
+# ones); M > N, whose items run in the other order. (Some of them, in one type or
+# both, run the 128 x 128 tiles or, 20 x 8200 x 8192, skinny_mfma_kernel: the tile
+# height follows from an estimate of time. KSPLIT_TILES names each instance.)
 KSPLIT = [(15, 64, 256), (17, 65, 31), (33, 63, 33), (47, 130, 95), (80, 4096, 512),
           (81, 200, 1001), (97, 127, 64), (96, 3000, 2048), (300, 4100, 2049), (64, 4096, 2111),
           (5, 203, 4099), (16, 512, 8191), (3, 1, 1), (64, 33, 4097), (700, 40, 999),
           (1000, 70, 2050), (301, 333, 7),
-          (5, 33555, 2001), (20, 8200, 8192)]  # B past 128 MiB: non-temporal copies
+          (5, 33555, 2001), (20, 8200, 8192)]  # B past 128 MiB
 
 
 @pytest.mark.parametrize("mnk", KSPLIT)
@@ -567,6 +569,67 @@ def test_gemm_ksplit(hip, mnk, offset, dtype):
         assert np.linalg.norm(y - ref) <= 1e-4 * np.linalg.norm(ref)
 
 
+# Every tile height (16 FM rows) of ksplit_kernel in both types, fp16 on shallow and
+# deep stages, with and without the repaired last step (edge: K off the step, or odd
+# fp16 N and K), K whole or split over workgroups: (dtype, m, n, k, FM, deep, edge).
+# tests/test_gemm_routes.py holds each to its instance.
+KSPLIT_TILES = [
+    ("f16", 34, 667, 2755, 2, 0, 1), ("f16", 96, 3000, 2048, 2, 1, 0),
+    ("f16", 153, 2241, 2069, 2, 1, 1), ("f16", 33, 1608, 1984, 3, 0, 0),
+    ("f16", 1000, 70, 2050, 3, 0, 1), ("f16", 89, 3328, 4160, 3, 1, 0),
+    ("f16", 236, 2135, 2369, 3, 1, 1), ("f16", 97, 654, 4160, 4, 0, 0),
+    ("f16", 270, 2821, 353, 4, 0, 1), ("f16", 209, 1858, 4288, 4, 1, 0),
+    ("f16", 551, 1387, 2091, 4, 1, 1), ("f16", 76, 2148, 2496, 5, 0, 0),
+    ("f16", 67, 1615, 3595, 5, 0, 1), ("f16", 300, 4096, 4096, 5, 1, 0),
+    ("f16", 321, 1523, 4119, 5, 1, 1), ("f16", 84, 2788, 2304, 6, 0, 0),
+    ("f16", 82, 2151, 3937, 6, 0, 1), ("f16", 178, 2760, 4160, 6, 1, 0),
+    ("f16", 573, 2207, 2327, 6, 1, 1), ("f32", 48, 4352, 6144, 3, 0, 0),
+    ("f32", 97, 1399, 1664, 4, 0, 0), ("f32", 573, 1759, 69, 4, 0, 1),
+    ("f32", 66, 2251, 2176, 5, 0, 0), ("f32", 406, 2397, 123, 5, 0, 1),
+    ("f32", 85, 2728, 2624, 6, 0, 0), ("f32", 667, 2187, 241, 6, 0, 1),
+    # B past 128 MiB that one row of tiles reads: non-temporal copies
+    ("f16", 20, 11008, 8192, 2, 1, 0), ("f32", 20, 4352, 8192, 2, 0, 0),
+    ("f16", 5, 33555, 2001, 1, 0, 1), ("f32", 12, 16384, 2056, 1, 0, 1)]
+# The 128 x 128 tiles split along K into partial tiles, and their sum: (dtype, m, n,
+# k), K a whole number of steps and not, fp16 rows of odd length.
+SPLIT_TILES = [("f16", 619, 122, 2688), ("f16", 579, 128, 2725), ("f16", 111, 826, 5440),
+               ("f16", 245, 513, 1907), ("f32", 127, 2761, 2816), ("f32", 119, 2859, 2944),
+               ("f32", 99, 4352, 5558), ("f32", 250, 2106, 5318)]
+
+
+@pytest.mark.parametrize("dtype,m,n,k", [c[:4] for c in KSPLIT_TILES] + SPLIT_TILES)
+@pytest.mark.parametrize("offset", [0, 1])
+def test_gemm_split_instances(hip, dtype, m, n, k, offset):
+    """Against the oracle on the first and last rows of each 16 and a spread of
+    others: bounds, guards and repetition as test_gemm_ksplit."""
+    a, b = oracle.uniform(902 + m, (m, k)), oracle.uniform(903 + n, (k, n))
+    rows = np.unique(np.concatenate([np.arange(0, m, max(1, m // 20)), [0, 15, 16, m - 17, m - 1]]))
+    rows = rows[(rows >= 0) & (rows < m)].astype(np.int32)
+    if dtype == "f16":
+        a, b = oracle.to_f16_bits(a), oracle.to_f16_bits(b)
+        ref = oracle.gemm(oracle.from_f16_bits(a), oracle.from_f16_bits(b), rows)
+        fn, nan = hip.lib.operatorlib_gemm_f16, np.uint16(0x7e00)
+    else:
+        ref = oracle.gemm(a, b, rows)
+        fn, nan = hip.lib.operatorlib_gemm_f32, np.float32("nan")
+    pad = np.full(256, nan, dtype=a.dtype)
+    da, db = (to_device(np.concatenate([x.ravel(), pad]), offset) for x in (a, b))
+    outs = []
+    for _ in range(2):
+        out = torch.full((m * n + 512,), float("nan"), device="cuda")
+        check(fn(ptr(da), ptr(db), ptr(out[256:]), m, n, k, stream_handle()), "gemm")
+        torch.cuda.synchronize()
+        outs.append(out)
+    assert torch.isnan(outs[0][:256]).all() and torch.isnan(outs[0][256 + m * n:]).all()
+    y = outs[0][256:256 + m * n].view(m, n)
+    assert torch.isfinite(y).all() and torch.equal(y, outs[1][256:256 + m * n].view(m, n))
+    got = y[torch.from_numpy(rows).long().cuda()].cpu().numpy().astype(np.float64)
+    if dtype == "f16":
+        assert np.max(np.abs(got - ref)) <= 2e-3
+    else:
+        assert np.linalg.norm(got - ref) <= 1e-4 * np.linalg.norm(ref)
+
+
 # Few rows on wide products, where K is not split over workgroups (and the 48- to
 # 80-row fp32 tiles of medium grids): the error against 64 bits stays within that
 # of K summed in chunks of 512. Additions of
@@ -591,10 +654,11 @@ def test_gemm_few_rows_error(ops, dtype, m, n, k, halves):
     assert error <= 0.43 * 2.0 ** -24 * math.sqrt(halves + k / 1024), error
 
 
-# A few tiles and a long K: ksplit_kernel split over more than 16 workgroups per
-# tile (each count of the steps 24, 36, 54 .. from fewest to most), and K from
-# 2^22 (fp16) or 2^21 (fp32) on, past the tiled kernels' 32-bit offsets.
-FEW_TILES = [(5, 40, 8191), (33, 100, 30001), (100, 130, 20000), (20, 64, 262145)]
+# Up to eight tiles and a long K: ksplit_kernel split over more than 16 workgroups
+# per tile (24 to 181 of them), and K from 2^22 (fp16) or 2^21 (fp32) on, past the
+# tiled kernels' 32-bit offsets.
+FEW_TILES = [(5, 40, 8191), (33, 100, 30001), (100, 130, 20000), (20, 64, 262145),
+             (16, 512, 65536)]
 FEW_TILES_WIDE = [(18, 16, 2), (32, 5, 1), (3, 40, 3)]
 
 
@@ -651,11 +715,13 @@ def test_gemm_past_offsets(ops, dtype, m, n, k):
         assert error <= math.sqrt(k) * 2.0 ** -24, (c, error)
 
 
-# fp16 grids that one round of 128 x 256 tiles (first four) or 192 x 256 tiles
+# fp16 grids that one round of 128 x 256 tiles (first three) or 192 x 256 tiles
 # covers: ragged M, N and K, rows at a 2-byte phase, one K step and several,
-# a tile count that is no multiple of the eight XCDs.
+# a tile count that is no multiple of the eight XCDs. (The last, 288 tiles, and
+# 771 x 7168, out of XCD order, are just off the rule: 256 x 256 and 128 x 128.)
 ONE_ROUND = [(1290, 4090, 130), (2000, 3000, 512), (1409, 3330, 65), (3840, 2304, 33),
-             (3000, 3000, 96), (3001, 2999, 161), (2300, 5120, 64), (1537, 8000, 127)]
+             (3000, 3000, 96), (3001, 2999, 161), (2300, 5120, 64), (1537, 7000, 127),
+             (771, 7168, 130), (1537, 8000, 127)]
 
 
 @pytest.mark.parametrize("mnk", ONE_ROUND)

@@ -84,7 +84,9 @@ SHAPES = [(19, 128), (17, 1024), (17, 1003), (5, 1), (3, 7), (3, 15), (3, 16),
           (1, 4096), (7, 4100), (3, 9000), (2, 32768), (2, 40000), (3, 33333),
           (4096, 1024), (4097, 1023), (2048, 4096), (2047, 4095),
           # short rows in lane groups; rows split over workgroups
-          (50000, 24), (3001, 256), (1, 1 << 20), (700, 40003)]
+          (50000, 24), (3001, 256), (1, 1 << 20), (700, 40003),
+          # a few rows on both sides of the widths where they are split
+          (63, 32767), (5, 32769), (5, 16385)]
 OFFSETS = [0, 1, 3, 7]          # elements: every 16-byte phase parity
 
 
@@ -96,7 +98,8 @@ def test_softmax_f16_matches_oracle(lib, shape, offset):
     assert_fp16_rounding_of(softmax_f16(lib, x, offset, offset), ref)
 
 
-@pytest.mark.parametrize("shape", [(17, 1003), (5, 40), (3, 9000), (2, 40000)])
+@pytest.mark.parametrize("shape", [(17, 1003), (5, 40), (3, 9000), (2, 40000), (5, 16384),
+                                   (5, 16385)])
 @pytest.mark.parametrize("in_off,out_off", [(1, 0), (0, 3), (2, 7)])
 def test_softmax_f16_mixed_phases(lib, shape, in_off, out_off):
     x = oracle.to_f16_bits(oracle.normal(710 + shape[1], shape, 0.0, 3.0))
@@ -127,7 +130,7 @@ RMS_CASES = [((32, 4096), 1e-5), ((17, 1003), 1e-5), ((21, 1024), 1e-5),
              ((3, 1), 1e-5), ((3, 15), 1e-5), ((4, 10000), 1e-6), ((2, 32768), 1e-6),
              ((2, 40001), 1e-6), ((2048, 4096), 1e-6), ((2047, 4095), 1e-6),
              ((50000, 24), 1e-6), ((3001, 256), 1e-5), ((2, 1 << 20), 1e-6),
-             ((700, 40003), 1e-6)]
+             ((700, 40003), 1e-6), ((63, 32767), 1e-6), ((5, 32769), 1e-6)]
 
 
 @pytest.mark.parametrize("shape,eps", RMS_CASES)
@@ -139,7 +142,8 @@ def test_rmsnorm_f16_matches_oracle(lib, shape, eps, offset):
     assert_fp16_rounding_of(rmsnorm_f16(lib, x, w, eps, offset, offset, 0), ref)
 
 
-@pytest.mark.parametrize("shape", [(17, 1003), (5, 40), (3, 9000), (2, 40000)])
+@pytest.mark.parametrize("shape", [(17, 1003), (5, 40), (3, 9000), (2, 40000), (5, 16384),
+                                   (5, 16385)])
 @pytest.mark.parametrize("in_off,out_off,w_off", [(1, 0, 0), (0, 3, 1), (5, 5, 3), (7, 7, 0)])
 def test_rmsnorm_f16_mixed_phases(lib, shape, in_off, out_off, w_off):
     x = oracle.to_f16_bits(oracle.normal(740 + shape[1], shape))

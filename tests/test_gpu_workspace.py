@@ -4,11 +4,11 @@ Every plan that fits the arena is the plan an unlimited workspace gives, so
 a *_ws call with exactly the queried bytes must return the plain entry
 point's bits; a workspace one byte short must be rejected before anything
 is enqueued (the output keeps its NaN fill). Cases: every launch sequence
-that uses scratch (reduce partials, decode split-K partials on both skinny
-kernels, padded fp16 operands at the 4095^3 BASELINE edge shape, the split
-last round of 256 x 256-tile fp16 and fp32 grids, small grids split along
-K, split fp32 and fp16 register-staged attention, softmax and RMSNorm rows
-split over workgroups).
+that uses scratch (reduce partials, split-K partials of both skinny kernels
+and the wavefront-split one, padded fp16 operands at the 4095^3 BASELINE edge
+shape, the split last round of 256 x 256-tile fp16 and fp32 grids, small
+grids of 128 x 128 tiles split along K, split fp32 and fp16 register-staged
+attention, softmax and RMSNorm rows split over workgroups).
 """
 
 from __future__ import annotations
@@ -65,8 +65,11 @@ def test_reduce_ws_matches_plain(lib, n):
 
 
 # (rows, cols): few long rows split over workgroups, rows past 32768
-# columns (one segment each), and shapes that need no scratch.
-ROW_CASES = [(1, 1 << 20), (32, 50257), (63, 5000), (600, 40003), (4096, 1024), (100000, 8)]
+# columns (one segment each), a few rows below the split widths (a workspace is
+# asked for and checked, but one workgroup per row runs), and shapes that need no
+# scratch.
+ROW_CASES = [(1, 1 << 20), (32, 50257), (63, 33000), (63, 5000), (600, 40003), (4096, 1024),
+             (100000, 8)]
 
 
 @pytest.mark.parametrize("rows,cols", ROW_CASES)
@@ -104,17 +107,21 @@ def test_rmsnorm_ws_matches_plain(lib, rows, cols, dtype):
           lambda: query(rows, cols), out)
 
 
-# (m, n, k, dtype): narrow decode shapes (split K) on both skinny kernels,
-# padded fp16 operands (4095^3), unaligned operands read in place (1000^3,
-# 999 x 1001 x 1003, 4095^3 fp32, 500 x 500 x 999), 272-tile fp16 and fp32
-# grids whose last round is split, an unaligned grid with a split last round
-# (4097 x 4095 x 4093), small grids split along K (64 x 4096 x 4096,
-# 1000^3), shapes that need no scratch.
+# (m, n, k, dtype): decode shapes, K split on the vector skinny kernel (1 row),
+# the wavefront-split one (16 rows; 16 x 512 x 65536 over 24 and more workgroups a
+# tile) and, B from memory, the matrix-core skinny one (24 x 8704 x 6144); padded
+# fp16 operands (4095^3), unaligned operands read in place (999 x 1001 x 1003,
+# 4095^3 fp32, 500 x 500 x 999), 272-tile fp16 and fp32 grids whose last round is
+# split, an unaligned grid with a split last round (4097 x 4095 x 4093), small
+# grids of 128 x 128 tiles split along K (619 x 122 x 2688 fp16, 127 x 2761 x 2816
+# fp32), shapes that need no scratch.
 GEMM_CASES = [(1, 1024, 4096, "f16"), (16, 1024, 4096, "f16"), (1, 1024, 4096, "f32"),
               (16, 1024, 4096, "f32"), (1000, 1000, 1000, "f16"), (4095, 4095, 4095, "f16"),
               (4352, 4096, 512, "f16"), (4352, 4096, 512, "f32"), (1024, 1024, 1024, "f16"),
               (999, 1001, 1003, "f32"), (4095, 4095, 4095, "f32"), (4097, 4095, 4093, "f32"),
-              (500, 500, 999, "f32"), (64, 4096, 4096, "f16"), (64, 4096, 4096, "f32")]
+              (500, 500, 999, "f32"), (64, 4096, 4096, "f16"), (64, 4096, 4096, "f32"),
+              (16, 512, 65536, "f16"), (16, 512, 65536, "f32"), (24, 8704, 6144, "f16"),
+              (619, 122, 2688, "f16"), (127, 2761, 2816, "f32")]
 
 
 @pytest.mark.parametrize("m,n,k,dtype", GEMM_CASES)

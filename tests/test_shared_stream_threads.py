@@ -6,8 +6,10 @@ library together):
   * reduce_sum_f32 over 1,000,003 values (one fp64 partial per workgroup,
     then the combine kernel);
   * gemm_f16 1 x 1024 x 4096 (decode GEMM, split-K partials + split sum);
-  * gemm_f16 1000^3 (64 tiles of 128 x 128, fewer than the CUs: every
-    tile split along K into partial tiles, then the split sum);
+  * gemm_f16 16 x 1024 x 4096 (wavefront-split kernel: split-K partials, then
+    the split sum);
+  * gemm_f16 619 x 122 x 2688 (5 tiles of 128 x 128, fewer than the CUs: every
+    tile split along K into partial tiles, then the tail sum);
   * attention_f32 B1 H4 S256 D99 (register-staged on a small grid: keys
     split over workgroups, partials, then the combine kernel);
   * gemm_f16 4352 x 4096 x 512 (272 tiles of 256 x 256: the last round's 16
@@ -17,7 +19,7 @@ library together):
 All of them take their scratch from the GPU's arena, which every stream
 shares: the arena's event chain must order the two threads' sequences.
 Each thread has its own inputs and its own output for every call, and
-enqueues 50 rounds of the six calls on ONE shared stream: an explicit
+enqueues 50 rounds of the seven calls on ONE shared stream: an explicit
 stream, the null stream, and hipStreamPerThread (where the two threads'
 streams differ although the handle is the same). Every output must match
 the oracle to the tolerances of test_gpu_ops.py, and repeated calls must
@@ -51,6 +53,9 @@ pytestmark = pytest.mark.gpu
 ROUNDS = 50
 SKINNY_N = 1024  # decode GEMM width: 8 column blocks x 64 K splits
 HIP_STREAM_PER_THREAD = 2  # hipStreamPerThread, include/hip/hip_runtime_api.h
+# tests/test_gemm_routes.py holds both to their kernels.
+KSPLIT_MNK = (16, SKINNY_N, 4096)
+SPLIT_MNK = (619, 122, 2688)
 # Split-tail GEMM: [M, K] x [K, N]; rows checked against the oracle: two in
 # every 256-row tile row, its first and last.
 TAIL_MK = (4352, 512)
@@ -73,8 +78,9 @@ class Case:
         self.x = oracle.uniform(seed, 1_000_003)
         self.a1 = oracle.to_f16_bits(oracle.uniform(seed + 1, (1, 4096)))
         self.b1 = oracle.to_f16_bits(oracle.uniform(seed + 2, (4096, SKINNY_N)))
-        self.ap = oracle.to_f16_bits(oracle.uniform(seed + 3, (1000, 1000)))
-        self.bp = oracle.to_f16_bits(oracle.uniform(seed + 4, (1000, 1000)))
+        self.ap = oracle.to_f16_bits(oracle.uniform(seed + 3, (SPLIT_MNK[0], SPLIT_MNK[2])))
+        self.bp = oracle.to_f16_bits(oracle.uniform(seed + 4, (SPLIT_MNK[2], SPLIT_MNK[1])))
+        self.ak = oracle.to_f16_bits(oracle.uniform(seed + 11, (KSPLIT_MNK[0], KSPLIT_MNK[2])))
         self.q, self.k, self.v = (oracle.normal(seed + 5 + i, (1, 4, 256, ATTN_D)) for i in range(3))
         self.at = oracle.to_f16_bits(oracle.uniform(seed + 8, TAIL_MK))
         self.bt = oracle.to_f16_bits(oracle.uniform(seed + 9, (TAIL_MK[1], TAIL_N)))
@@ -84,16 +90,18 @@ class Case:
             "reduce": oracle.reduce_sum(self.x),
             "skinny": oracle.gemm(f(self.a1), f(self.b1)),
             "split_k": oracle.gemm(f(self.ap), f(self.bp)),
+            "ksplit": oracle.gemm(f(self.ak), f(self.b1)),
             "attn": oracle.attention(self.q, self.k, self.v, False),
             "tail": oracle.gemm(f(self.at), f(self.bt), TAIL_ROWS),
             "softmax": oracle.softmax(self.sm),
         }
         self.dev = {name: to_device(getattr(self, name))
-                    for name in ("x", "a1", "b1", "ap", "bp", "q", "k", "v", "at", "bt", "sm")}
+                    for name in ("x", "a1", "b1", "ap", "bp", "ak", "q", "k", "v", "at", "bt", "sm")}
         self.out = {
             "reduce": torch.full((rounds,), float("nan"), device="cuda"),
             "skinny": torch.full((rounds, 1, SKINNY_N), float("nan"), device="cuda"),
-            "split_k": torch.full((rounds, 1000, 1000), float("nan"), device="cuda"),
+            "split_k": torch.full((rounds, *SPLIT_MNK[:2]), float("nan"), device="cuda"),
+            "ksplit": torch.full((rounds, *KSPLIT_MNK[:2]), float("nan"), device="cuda"),
             "attn": torch.full((rounds, 1, 4, 256, ATTN_D), float("nan"), device="cuda"),
             "tail": torch.full((rounds, TAIL_MK[0], TAIL_N), float("nan"), device="cuda"),
             "softmax": torch.full((rounds, *SPLIT_ROWS), float("nan"), device="cuda"),
@@ -106,7 +114,9 @@ class Case:
         check(lib.operatorlib_gemm_f16(ptr(d["a1"]), ptr(d["b1"]), ptr(o["skinny"][r]),
                                        1, SKINNY_N, 4096, stream), "gemm_f16 skinny")
         check(lib.operatorlib_gemm_f16(ptr(d["ap"]), ptr(d["bp"]), ptr(o["split_k"][r]),
-                                       1000, 1000, 1000, stream), "gemm_f16 split_k")
+                                       *SPLIT_MNK, stream), "gemm_f16 split_k")
+        check(lib.operatorlib_gemm_f16(ptr(d["ak"]), ptr(d["b1"]), ptr(o["ksplit"][r]),
+                                       *KSPLIT_MNK, stream), "gemm_f16 ksplit")
         check(lib.operatorlib_attention_f32(ptr(d["q"]), ptr(d["k"]), ptr(d["v"]),
                                             ptr(o["attn"][r]), 1, 4, 256, ATTN_D, 0, stream),
               "attention_f32")
@@ -117,15 +127,15 @@ class Case:
                                           stream), "softmax split rows")
 
     def workspace_bytes(self, lib) -> int:
-        """The largest workspace query of the six calls."""
+        """The largest workspace query of the seven calls."""
         d = self.dev
         tmp = torch.empty(TAIL_MK[0] * TAIL_N, device="cuda")
         return max(
             lib.operatorlib_reduce_sum_f32_workspace_size(ptr(d["x"]), d["x"].numel()),
             lib.operatorlib_gemm_f16_workspace_size(ptr(d["a1"]), ptr(d["b1"]), 1, SKINNY_N,
                                                     4096),
-            lib.operatorlib_gemm_f16_workspace_size(ptr(d["ap"]), ptr(d["bp"]), 1000, 1000,
-                                                    1000),
+            lib.operatorlib_gemm_f16_workspace_size(ptr(d["ap"]), ptr(d["bp"]), *SPLIT_MNK),
+            lib.operatorlib_gemm_f16_workspace_size(ptr(d["ak"]), ptr(d["b1"]), *KSPLIT_MNK),
             lib.operatorlib_attention_f32_workspace_size(ptr(d["q"]), ptr(d["k"]), ptr(d["v"]),
                                                          ptr(tmp), 1, 4, 256, ATTN_D, 0),
             lib.operatorlib_gemm_f16_workspace_size(ptr(d["at"]), ptr(d["bt"]), TAIL_MK[0],
@@ -133,7 +143,7 @@ class Case:
             lib.operatorlib_softmax_f32_workspace_size(*SPLIT_ROWS))
 
     def enqueue_ws(self, lib, stream, r: int, ws: torch.Tensor) -> None:
-        """The six calls through the *_ws entry points, one after another
+        """The seven calls through the *_ws entry points, one after another
         on `stream` in one workspace."""
         d, o = self.dev, self.out
         w, nb = ptr(ws), ws.numel()
@@ -142,7 +152,9 @@ class Case:
         check(lib.operatorlib_gemm_f16_ws(ptr(d["a1"]), ptr(d["b1"]), ptr(o["skinny"][r]),
                                           1, SKINNY_N, 4096, w, nb, stream), "gemm_f16_ws skinny")
         check(lib.operatorlib_gemm_f16_ws(ptr(d["ap"]), ptr(d["bp"]), ptr(o["split_k"][r]),
-                                          1000, 1000, 1000, w, nb, stream), "gemm_f16_ws split_k")
+                                          *SPLIT_MNK, w, nb, stream), "gemm_f16_ws split_k")
+        check(lib.operatorlib_gemm_f16_ws(ptr(d["ak"]), ptr(d["b1"]), ptr(o["ksplit"][r]),
+                                          *KSPLIT_MNK, w, nb, stream), "gemm_f16_ws ksplit")
         check(lib.operatorlib_attention_f32_ws(ptr(d["q"]), ptr(d["k"]), ptr(d["v"]),
                                                ptr(o["attn"][r]), 1, 4, 256, ATTN_D, 0, w, nb,
                                                stream), "attention_f32_ws")
@@ -157,6 +169,7 @@ class Case:
         red = self.out["reduce"].cpu().numpy()
         sk = self.out["skinny"].cpu().numpy().astype(np.float64)
         pd = self.out["split_k"].cpu().numpy().astype(np.float64)
+        ks = self.out["ksplit"].cpu().numpy().astype(np.float64)
         at = self.out["attn"].cpu().numpy().astype(np.float64)
         smx = self.out["softmax"].cpu().numpy().astype(np.float64)
         ref = self.ref
@@ -165,6 +178,7 @@ class Case:
             assert abs(red[r] - ref["reduce"]) <= 1e-5 * abs(ref["reduce"]), where
             assert np.max(np.abs(sk[r] - ref["skinny"])) <= 2e-3, where
             assert np.max(np.abs(pd[r] - ref["split_k"])) <= 2e-3, where
+            assert np.max(np.abs(ks[r] - ref["ksplit"])) <= 2e-3, where
             err = np.abs(at[r] - ref["attn"])
             assert np.all(err <= 1e-4 + 1e-4 * np.abs(ref["attn"])), where
             assert np.max(np.abs(smx[r] - ref["softmax"])) <= 1e-6, where
@@ -173,6 +187,7 @@ class Case:
             assert red[r] == red[rounds[0]], where
             assert np.array_equal(sk[r], sk[rounds[0]]), where
             assert np.array_equal(pd[r], pd[rounds[0]]), where
+            assert np.array_equal(ks[r], ks[rounds[0]]), where
             assert np.array_equal(at[r], at[rounds[0]]), where
             # the split-tail GEMM: checked on the device (3.5 GiB of rounds)
             tail = self.out["tail"][r]
@@ -321,12 +336,12 @@ def test_capture_workspace_entry_points_overlap_eager_calls(lib, cases):
 
 GRAPHS = 20
 # Device memory the runtime itself may take for 20 instantiated graphs of
-# six calls each (graph objects, kernel arguments); the library adds none.
+# seven calls each (graph objects, kernel arguments); the library adds none.
 GRAPH_MEMORY_SLACK = 32 << 20
 
 
 def test_twenty_graphs_hold_no_library_memory(lib, cases):
-    """Capturing the six arena-using calls into 20 graphs leaves library-held
+    """Capturing the seven arena-using calls into 20 graphs leaves library-held
     device memory where it was (the arena is static), and every replay gives
     the eager result's bits."""
     _reset(cases)

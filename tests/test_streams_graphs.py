@@ -39,6 +39,7 @@ def _inputs(device):
         "ah": mk(1000, 1000, dtype=torch.float16), "bh": mk(1000, 1000, dtype=torch.float16),
         "a1": mk(1, 4096, dtype=torch.float16), "b1": mk(4096, 4096, dtype=torch.float16),
         "a16": mk(16, 4096, dtype=torch.float16),
+        "at": mk(619, 2688, dtype=torch.float16), "bt": mk(2688, 122, dtype=torch.float16),
         "a12": mk(12, 1024), "b32": mk(1024, 2048),
         "q": mk(1, 4, 256, 128, dtype=torch.float16),
         "k": mk(1, 4, 256, 128, dtype=torch.float16),
@@ -64,10 +65,11 @@ def _all_ops(ops, t):
         ops.softmax(t["sm"].half()),
         ops.rmsnorm(t["rn"].half(), t["w"].half(), 1e-6),
         ops.gemm(t["a"], t["b"]),
-        ops.gemm(t["ah"], t["bh"]),      # tiles split along K: workspace partials
+        ops.gemm(t["ah"], t["bh"]),      # wavefront-split kernel, no scratch
+        ops.gemm(t["at"], t["bt"]),      # 128 x 128 tiles split along K: workspace partials
         ops.gemm(t["a1"], t["b1"]),      # skinny path with K splits
-        ops.gemm(t["a16"], t["b1"]),     # matrix-core skinny kernel, vector A
-        ops.gemm(t["a1"], t["b1"][:, :1024].contiguous()),   # narrow: more K splits
+        ops.gemm(t["a16"], t["b1"]),     # wavefront-split kernel, K split over workgroups
+        ops.gemm(t["a1"], t["b1"][:, :1024].contiguous()),   # narrower: more K splits
         ops.gemm(t["a16"], t["b1"][:, :1024].contiguous()),
         ops.gemm(t["a12"], t["b32"]),    # same, fp32
         ops.attention(t["q"], t["k"], t["v"], True),
