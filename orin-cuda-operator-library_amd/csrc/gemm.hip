@@ -2685,10 +2685,14 @@ int one_round_rows(int m, int n) {
   // (not where 256-column tiles pad N by over a tenth more than 128-column ones)
   const long long small = (m + 127LL) / 128 * ((n + 127) / 128);
   if (small < cus || 20 * cols > 11LL * ((n + 127) / 128)) return 0;
-  // (nor 128 x 256 ones that xcd_regroup leaves in launch order where it regroups
-  // the 128 x 128 ones: 386 x 10981 x 3904, 172 against 344 tiles, 96 against 76 us;
-  // 771 x 7168 x 4224, 196 against 392, 76 against 60)
-  if (tiles128 <= cus) return tiles128 % kXcds != 0 && small % kXcds == 0 ? 0 : 128;
+  // (nor, up to one group of tile rows, 128 x 256 ones that xcd_regroup leaves in
+  // launch order where it regroups the 128 x 128 ones: 771 x 7168 x 4224, 196 against
+  // 392 tiles, 76 against 60 us; 868 x 5056 x 2176 36.6 against 32.6; 15 random shapes
+  // to 868 rows 7% slower on them, one, 622 x 9128 x 7296, faster by over 1%, 156
+  // against 168. Of 34 taller ones 21 are faster by over 3%: 2064 x 3072 x 7360, 204
+  // against 408, 109 against 125)
+  if (tiles128 <= cus)
+    return m <= kGroupM * 128 && tiles128 % kXcds != 0 && small % kXcds == 0 ? 0 : 128;
   return tiles192 <= cus ? 192 : 0;
 }
 

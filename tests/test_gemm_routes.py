@@ -122,10 +122,11 @@ def test_few_rows_from_memory(plans):
 
 def test_one_round_tiles_keep_their_xcd_order(plans):
     """fp16 grids of one round of 128 x 256 tiles whose count is no multiple of the
-    eight XCDs, where that of the 128 x 128 ones is: the latter."""
+    eight XCDs, where that of the 128 x 128 ones is: the latter, up to 1024 rows."""
     _check(plans, [(("f16", 386, 10981, 3904), dict(kind="dma", rows=128, one_round=None)),
                    (("f16", 771, 7168, 4224), dict(kind="dma", rows=128, one_round=None)),
                    (("f16", 768, 7168, 4224), dict(kind="dma", rows=128, one_round=1)),
+                   (("f16", 2064, 3072, 7360), dict(kind="dma", rows=128, one_round=1)),
                    (("f16", 2000, 3000, 512), dict(kind="dma", rows=128, one_round=1)),
                    (("f16", 3000, 3000, 3000), dict(kind="dma", rows=192, one_round=1))])
 
