@@ -2277,10 +2277,14 @@ void ksplit_kernel(const T* __restrict__ A, const T* __restrict__ B, float* __re
 }
 
 constexpr int kMaxSplits = 16;
-// Up to 8 tiles would leave half the CUs idle or more at 16 splits (products of
+// Fewer than 8 tiles would leave over half the CUs idle at 16 splits (products of
 // few rows and columns and a long K): from there in steps of a half, 181 at the
-// most (fp16 16 x 512 x 262144, 8 tiles, us: 85 on 16 splits, 60 on 64).
+// most. 8 tiles, half the CUs, only on a long K (us, the best of up to 16 splits /
+// of 20..64): fp16 16 x 512 x 262144 85 / 60, 9 x 512 x 65536 18.7 / 17.6, x 49152
+// 15.3 / 14.7, x 13000 8.2 / 8.3, 65 x 256 x 13000 8.8 / 9.5; fp32 9 x 512 x 49152
+// 31.6 / 24.4, x 32768 18.3 / 18.2, 48 x 512 x 49152 43.4 / 35.1, x 24576 20.6 / 21.8.
 constexpr int kMaxSplitsFewTiles = 181;
+constexpr int kEightTilesFromK = 49152;
 // B that one row of tiles reads once, and that fills half the Infinity Cache
 // or more, is copied with the non-temporal hint. Measured on MI355X (us,
 // cached -> non-temporal, three sets of inputs / twenty): fp16 16 x 8192 x
@@ -2906,7 +2910,8 @@ ksplit::Plan ksplit_plan(int m, int n, int k, bool few_rows, std::size_t capacit
     const long long tiles = rows * ((n + ksplit::kBN - 1) / ksplit::kBN);
     if (tiles > 0x3fffffffLL) continue;
     const long long slots = static_cast<long long>(cus) * (fm == 1 ? 2 : 1);  // pairs of fm = 1
-    const int max_splits = tiles <= 8 ? ksplit::kMaxSplitsFewTiles : ksplit::kMaxSplits;
+    const bool few_tiles = tiles < 8 || (tiles == 8 && k >= ksplit::kEightTilesFromK);
+    const int max_splits = few_tiles ? ksplit::kMaxSplitsFewTiles : ksplit::kMaxSplits;
     for (int splits = 1; splits <= max_splits; splits += splits < 16 ? 1 : splits / 2) {
       // one split, or a grid the CUs hold at once with a step per wavefront
       if (splits > 1 && (tiles * splits > slots || k / (8 * dma::Elem<T>::kSubK) < splits)) break;

@@ -79,11 +79,14 @@ def _check(plans, routes):
 
 
 def test_eight_tiles_split_past_sixteen(plans):
-    """Eight 64-column tiles on 16 splits of K would leave half the CUs idle."""
+    """Eight 64-column tiles on 16 splits of K leave half the CUs idle: a long K is
+    split further, a shorter one is not."""
     _check(plans, [(("f16", 16, 512, 262144), dict(kind="split", fm=1, splits=54)),
                    (("f16", 3, 512, 262144), dict(kind="split", fm=1, splits=54)),
                    (("f16", 16, 576, 262144), dict(kind="split", fm=1, splits=16)),
-                   (("f16", 5, 16, 1 << 20), dict(kind="split", fm=1, splits=181))])
+                   (("f16", 5, 16, 1 << 20), dict(kind="split", fm=1, splits=181)),
+                   (("f16", 9, 450, 6464), dict(kind="split", fm=1, splits=16)),
+                   (("f16", 65, 256, 10193), dict(kind="split", fm=2, splits=16))])
 
 
 def test_fp32_tile_heights(plans):
