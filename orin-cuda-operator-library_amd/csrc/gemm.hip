@@ -2763,12 +2763,8 @@ TailPlan tail_plan(int m, int n, int k, std::size_t capacity) {
 // 1..8000, N and K 16..262144. What bounds these grids is the L2: a CU's
 // copies arrive at 64-75 bytes/ns (the eight L2s together deliver about 17
 // TB/s), so a tile of R x C costs (R + C) K elements per round of
-// workgroups; fp32 tiles cost their matrix-core time, 3.7 ns per 16 rows and
-// k of a 64-column tile and 1.0 per k (B's fragments; 1.5 for 16 rows in several
-// rounds), after 3.5 us for 16 rows
-// and 0.4 more for each further 16 (82..112 timings of each height, 3-5% off
-// this line; with 4.1 ns throughout fp32 96 x 12288 x 12288 took 16-row tiles, 341
-// us against 280 on 96-row ones). Rows off 64 bytes straddle twice the lines.
+// workgroups; fp32 tiles cost their matrix-core time, 4.1 ns per 16 rows and
+// k of a 64-column tile. Rows off 64 bytes straddle twice the lines.
 // The operands' stream from memory grows with the workgroups that ask for it
 // (towards 5500 bytes/ns, or 8000 where they fit the Infinity Cache several
 // times over); partial sums cost a launch and their traffic.
@@ -2813,8 +2809,12 @@ double row_stream_ns(int splits, int m, int n, int k, double wgs, int cus) {
                   turns * 64.0 * k * sizeof(T) / splits / rate);
 }
 
+// `heights`: to choose between tile heights, where fp32 16-row tiles in several
+// rounds cost 1.5 ns per k more on a long K (64 x 12288 x 12288 246 us on them, 198 on
+// 64-row ones; 96 x 12288 x 12288 331, on 48-row ones 300; but 104 x 8960 x 2240 44.5
+// against 60 on 48-row ones).
 template <typename T>
-double ksplit_ns(int fm, int splits, int m, int n, int k, int cus) {
+double ksplit_ns(int fm, int splits, int m, int n, int k, int cus, bool heights) {
   const double size = sizeof(T);
   const double tiles = static_cast<double>((m + 16 * fm - 1) / (16 * fm)) * ((n + 63) / 64);
   const double wgs = tiles * splits;
@@ -2825,8 +2825,9 @@ double ksplit_ns(int fm, int splits, int m, int n, int k, int cus) {
   const double copies = (16.0 * fm + 64) * k * size / splits / kTileBytesPerNs *
                         (off_line ? kOffLineFactor : 1.0);
   const double mfma =
-      sizeof(T) == 4 ? (3.7 * fm + (fm == 1 && rounds > 1 ? 1.5 : 1.0)) * k / splits : 0.0;
-  const double start = sizeof(T) == 4 ? 2100 + 400.0 * fm : kNsRound;
+      sizeof(T) == 4
+          ? (4.1 * fm + (heights && fm == 1 && rounds > 1 && k >= 6144 ? 1.5 : 0.0)) * k / splits
+          : 0.0;
   const double operands = stream_bytes<T>(m, n, k);
   const bool cached = operands < kCachedUpTo;
   double stream;
@@ -2840,7 +2841,7 @@ double ksplit_ns(int fm, int splits, int m, int n, int k, int cus) {
     const double again = !cached && n >= m && m > 16 * fm ? 1.3 : 1.0;
     stream = operands / ((cached ? kCacheBytesPerNs : kMemoryBytesPerNs) * asked) * uneven * again;
   }
-  return kNsLaunch + starts * start + std::max(rounds * std::max(copies, mfma), stream) +
+  return kNsLaunch + starts * kNsRound + std::max(rounds * std::max(copies, mfma), stream) +
          (splits > 1 ? kNsSum + 8.0 * splits * m * n / kPartialBytesPerNs : 0.0);
 }
 
@@ -2889,7 +2890,7 @@ bool skinny_mfma_faster(const T* b, int m, int n, int k, int splits, double spli
                     static_cast<double>(n) * k * sizeof(T) / rate;
   // (split K on pairs of workgroups draws more than its estimate: 8 x 8704 x 12288
   // 43.9 vs 47.7)
-  return ns * (splits > 1 ? 1.12 : 0.97) < split_ns;
+  return ns * (splits > 1 ? 1.12 : sizeof(T) == 2 ? 0.97 : 1.0) < split_ns;
 }
 
 // ksplit_kernel's plan for shapes it is the fastest estimate for (fm == 0:
@@ -2903,7 +2904,7 @@ ksplit::Plan ksplit_plan(int m, int n, int k, bool few_rows, std::size_t capacit
   int cus = device_cus();
   if (cus <= 0) cus = 256;
   ksplit::Plan best;
-  double best_ns = 0;
+  double best_ns = 0, least_ns = 1e300;
   for (int fm = 1; fm <= 6; ++fm) {
     const long long rows = (m + 16LL * fm - 1) / (16 * fm);
     if (fm > 1 && (m + 16LL * (fm - 1) - 1) / (16 * (fm - 1)) == rows) continue;  // more padding
@@ -2915,13 +2916,14 @@ ksplit::Plan ksplit_plan(int m, int n, int k, bool few_rows, std::size_t capacit
     for (int splits = 1; splits <= max_splits; splits += splits < 16 ? 1 : splits / 2) {
       // one split, or a grid the CUs hold at once with a step per wavefront
       if (splits > 1 && (tiles * splits > slots || k / (8 * dma::Elem<T>::kSubK) < splits)) break;
-      // fp32 96-row tiles hold no total: short chains only (96 x 12288 x 12288 in
-      // one, error against 64 bits 7.0e-7; on 48-row tiles 1.7e-7)
-      if (sizeof(T) == 4 && fm == 6 && k / splits > 3072) continue;
       const std::size_t bytes =
           splits > 1 ? static_cast<std::size_t>(splits) * m * n * sizeof(float) : 0;
       if (bytes > capacity) break;
-      const double ns = ksplit_ns<T>(fm, splits, m, n, k, cus);
+      least_ns = std::min(least_ns, ksplit_ns<T>(fm, splits, m, n, k, cus, false));
+      // fp32 96-row tiles hold no total: not past chains that leave the error below
+      // the 128 x 128 tiles' (96 x 12288 x 12288 in one: 7.0e-7, on 48 rows 1.7e-7)
+      if (sizeof(T) == 4 && fm == 6 && k / splits > 9216) continue;
+      const double ns = ksplit_ns<T>(fm, splits, m, n, k, cus, true);
       if (best.fm == 0 || ns < best_ns) {
         best_ns = ns;
         best.fm = fm;
@@ -2932,8 +2934,8 @@ ksplit::Plan ksplit_plan(int m, int n, int k, bool few_rows, std::size_t capacit
   }
   if (!few_rows) {
     // (whole rounds of unsplit tiles are estimated closely: a near tie there,
-    // fp16 5184 x 896 x 11712 170 against 175 us, is theirs; an fp32 tie is
-    // ksplit_kernel's, whose chains of additions are shorter)
+    // fp16 5184 x 896 x 11712 170 against 175 us, is theirs; what chooses the height
+    // alone sends no fp32 product to them, whose error is 2-5 times as large)
     const TailPlan tail = tail_plan<T>(m, n, k, capacity);
     const double bias = (tail.splits > 0 ? 1.0 : 0.95) * (sizeof(T) == 4 ? 1.08 : 1.0);
     if (small_tiles_ns<T>(m, n, k, cus, tail) * bias < best_ns) return ksplit::Plan{};

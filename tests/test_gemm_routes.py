@@ -90,13 +90,13 @@ def test_eight_tiles_split_past_sixteen(plans):
 
 
 def test_fp32_tile_heights(plans):
-    """Matrix-core time per row falls with the tile's height (B's fragments), so a
-    long K does not run on 16-row tiles by default; 96-row tiles, which hold no
-    total of short chains, take up to 3072 of K each."""
+    """fp32 16-row tiles in several rounds cost more on a long K, where they do not
+    run by default; 96-row tiles, which hold no total of short chains, take up to
+    9216 of K each."""
     _check(plans, [(("f32", 96, 12288, 12288), dict(kind="split", fm=3, splits=1)),
                    (("f32", 64, 12288, 12288), dict(kind="split", fm=4, splits=1)),
-                   (("f32", 80, 11008, 4096), dict(kind="split", fm=5, splits=1)),
-                   (("f32", 1146, 2816, 3968), dict(kind="split", fm=5, splits=1)),
+                   (("f32", 104, 8960, 2240), dict(kind="split", fm=1, splits=1)),
+                   (("f32", 2564, 1792, 12352), dict(kind="split", fm=3, splits=1)),
                    (("f32", 96, 12288, 1024), dict(kind="split", fm=6, splits=1)),
                    (("f32", 1000, 1000, 1000), dict(kind="split", fm=4, splits=1))])
 
