@@ -2937,8 +2937,8 @@ ksplit::Plan ksplit_plan(int m, int n, int k, bool few_rows, std::size_t capacit
     // fp16 5184 x 896 x 11712 170 against 175 us, is theirs; what chooses the height
     // alone sends no fp32 product to them, whose error is 2-5 times as large)
     const TailPlan tail = tail_plan<T>(m, n, k, capacity);
-    const double bias = (tail.splits > 0 ? 1.0 : 0.95) * (sizeof(T) == 4 ? 1.08 : 1.0);
-    if (small_tiles_ns<T>(m, n, k, cus, tail) * bias < best_ns) return ksplit::Plan{};
+    if (small_tiles_ns<T>(m, n, k, cus, tail) * (tail.splits > 0 ? 1.0 : 0.95) < least_ns)
+      return ksplit::Plan{};
   }
   *estimate = best_ns;
   // 128-byte A rows once each wavefront walks enough of them. Measured on
