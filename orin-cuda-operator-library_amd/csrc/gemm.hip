@@ -1637,8 +1637,10 @@ bool applies(const T* b, int m, int n, int k, bool wide) {
   // workgroup per CU, or a long K (M = 3, us, this kernel vs ksplit_kernel): 12288
   // x 12288 54.8 vs 66.0, 12288 x 4096 22.0 vs 23.1, 9216 x 12288 43.0 vs 43.8,
   // 28672 x 8192 79.7 vs 94.6; 6144 x 12288 32.5 vs 29.3, 50304 x 4096 71.0 vs
-  // 71.4, 151936 x 4096 212 vs 190.
-  const bool memory = bytes >= (std::size_t(96) << 20) && n >= 8192 && (n <= 16384 || k >= 6144);
+  // 71.4, 151936 x 4096 212 vs 190. Only rows a whole number of 512 bytes apart:
+  // 12224 x 4416 23.1 vs 20.3, 13376 x 9408 45.5 vs 40.3, 11840 x 12853 54.3 vs 50.9.
+  const bool memory = bytes >= (std::size_t(96) << 20) && n >= 8192 && n % 256 == 0 &&
+                      (n <= 16384 || k >= 6144);
   const int up_to = sizeof(T) == 4 ? (bytes >= (std::size_t(128) << 20) ? 8 : Cfg<T>::kUpToM)
                                    : (memory ? 4 : Cfg<T>::kUpToM);
   return n % Cfg<T>::kPerLane == 0 && opl::aligned16(b) &&
@@ -2784,12 +2786,15 @@ double stream_bytes(int m, int n, int k) {
 // CU draws its columns' rows at a rate that falls with M and with the power of
 // two in B's row pitch (128-byte pieces a pitch apart meet in fewer channels;
 // rows off 64 bytes draw as slowly), and all CUs together up to a limit.
-// Measured on MI355X (bytes/ns per CU, workgroups): fp16 M = 8, K = 12288: N 8704 (pitch 17 KiB) 26.8 (136),
-// 10240 (20 KiB) 23.9 (160), 11264 (22 KiB) 22.8 (176), 12288 (24 KiB) 24.0 (192),
+// Measured on MI355X (bytes/ns per CU, workgroups): fp16 M = 8, K = 12288: N 8704
+// (pitch 17 KiB) 26.8 (136), 10240 (20 KiB) 23.9 (160), 11264 (22 KiB) 22.8 (176),
+// 12288 (24 KiB) 24.0 (192),
 // 11008 (21.5 KiB) 30.7 (172), 8832 (17.25 KiB) 36.2 (138), 10000 24.5 (157);
 // M = 24: 23.4, 22.5, 22.8, 22.9, 28.2, 33.4, 23.5; fp32 N 8704 and 12288 M = 9
 // 31, 27.8, M = 16 28.6, 26.1, M = 32 23.9, 22.5. fp16 N = 16384, 256
-// workgroups 5700 in all, N = 16000 6700, N = 50264 4300; fp32 N = 16384 6450.
+// workgroups 5700 in all, N = 16000 6700; fp32 N = 16384 6450. fp16 N up to 8192 on
+// other pitches than whole 512 bytes draws more on more splits still: M = 9, 8096 x
+// 8192 27.4 us on four, 31.7 on three, M = 12, 4480 x 13376 25.6 on seven, 27.8 on six.
 constexpr int kRowStreamFrom = 2048;
 constexpr double kRowCachedUpTo = 92e6;  // (11008 x 4096 still draws at the cache's rate)
 
@@ -2800,7 +2805,7 @@ double row_stream_ns(int splits, int m, int n, int k, double wgs, int cus) {
   const bool slow = pitch % 1024 == 0 || pitch % 64 != 0;
   double rate = kHalf ? (slow ? 26 : pitch % 512 == 0 ? 31 : 35) - m / 8.0
                       : std::max(22.0, 32 - 0.3 * m);
-  double total = !slow ? 6500 : pitch % 64 != 0 ? 4300 : kHalf ? 5700 : 6100;
+  double total = !slow ? 6500 : kHalf ? 5700 : 6100;
   // (fp16 K splits that leave each CU one workgroup keep less in flight than
   // pairs do: 16 x 5120 x 13824 40.3 us on 240, 35.1 on 480)
   if (kHalf && splits > 1 && wgs <= cus) rate *= 0.96, total *= 0.96;
@@ -2831,7 +2836,9 @@ double ksplit_ns(int fm, int splits, int m, int n, int k, int cus, bool heights)
   const double operands = stream_bytes<T>(m, n, k);
   const bool cached = operands < kCachedUpTo;
   double stream;
-  if (operands >= kRowCachedUpTo && m <= 16 * fm && n >= kRowStreamFrom) {
+  const bool row = operands >= kRowCachedUpTo && m <= 16 * fm && n >= kRowStreamFrom &&
+                   (sizeof(T) == 4 || n > 8192 || n % 256 == 0);
+  if (row) {
     stream = row_stream_ns<T>(splits, m, n, k, wgs, cus);
   } else {
     const double asked = wgs / (wgs + (cached && sizeof(T) == 2 ? 25 : 60));
@@ -2867,24 +2874,26 @@ double small_tiles_ns(int m, int n, int k, int cus, const TailPlan& tail) {
 }
 
 // Few rows of B from memory on more than half as many columns' tiles as CUs
-// (N 8193..16384, or any N whose rows are off 64 bytes): ksplit_kernel cannot
-// split K without a second turn of some CUs, and may draw less than
-// skinny_mfma_kernel does on its 512 and more workgroups (time: a launch and B at
-// 4.0-5.3 bytes/ps). Measured on MI355X (us, ksplit_kernel vs
-// skinny_mfma_kernel): fp16 24 x 8704 x 12288 70.6 vs 56.5, 8 x 10240 x 12288 50.0
-// (three splits) vs 54.3, 24 x 10240 x 6144 38.8 vs 34.7, 8 x 12288 x 12288 68.7 vs
-// 64.3, 24 x 12288 x 12288 72.1 vs 76.1, 24 x 11008 x 12288 59.3 vs 66.9, 16 x
-// 50264 x 4096 106.9 vs 98.7; fp32 32 x 8704 x 12288 135 vs 118, 24 x 12288 x
-// 12288 134 vs 150.
+// (N 8193..16384): ksplit_kernel cannot split K without a second turn of some
+// CUs, and may draw less than skinny_mfma_kernel does on its 512 and more
+// workgroups (time: a launch and B at 4.0-5.3 bytes/ps), where B's rows are a whole
+// number of 512 bytes apart; in fp32 only 17..32 rows, 1024 bytes and K from 6144.
+// Measured on MI355X (us, ksplit_kernel vs skinny_mfma_kernel): fp16 24 x 8704 x 12288
+// 70.6 vs 56.5, 8 x 10240 x 12288 50.0 (three splits) vs 54.3, 24 x 10240 x 6144 38.8
+// vs 34.7, 8 x 12288 x 12288 68.7 vs 64.3, 24 x 12288 x 12288 72.1 vs 76.1, 24 x 11008
+// x 12288 59.3 vs 66.9; fp32 32 x 8704 x 12288 135 vs 118, x 4096 46.3 vs 48.3, 32 x
+// 10240 x 12288 142 vs 134, 24 x 12288 x 12288 134 vs 150; 512 bytes: 29 x 10880 x 12929
+// 146 vs 174; others 32 x 8640 x 6133 70.5 vs 77.0, 9 x 11072 x 7552 60.4 vs 63.2.
 template <typename T>
 bool skinny_mfma_faster(const T* b, int m, int n, int k, int splits, double split_ns) {
   using C = skinny::Cfg<T>;
   const int cus = device_cus() > 0 ? device_cus() : 256;
   const long long tiles = (n + ksplit::kBN - 1LL) / ksplit::kBN;
-  const bool off_line = static_cast<std::size_t>(n) * sizeof(T) % 64 != 0;
   if (m < C::kMfmaMinM || m > 32 || n % C::kPerLane != 0 || !opl::aligned16(b) ||
-      tiles <= cus / 2 || (tiles > cus && !off_line) || stream_bytes<T>(m, n, k) < kRowCachedUpTo)
+      n % 256 != 0 || tiles <= cus / 2 || tiles > cus ||
+      stream_bytes<T>(m, n, k) < kRowCachedUpTo)
     return false;
+  if (sizeof(T) == 4 && (m <= 16 || k < 6144)) return false;
   const double rate = m <= 16 ? 5500 - 50.0 * m : 4600 - 18.0 * m;
   const double ns = 5000 + (m <= 16 ? 0 : sizeof(T) == 2 ? 1500 : 6000) +
                     static_cast<double>(n) * k * sizeof(T) / rate;

@@ -107,11 +107,18 @@ def test_few_rows_from_memory(plans):
     skinny::applies), and the cached calls as they were."""
     _check(plans, [(("f16", 24, 8704, 12288), dict(kind="skinny", mfma=1)),
                    (("f16", 8, 12288, 12288), dict(kind="skinny", mfma=1)),
-                   (("f16", 16, 50264, 4096), dict(kind="skinny", mfma=1)),
+                   (("f16", 16, 50264, 4096), dict(kind="split", fm=1, splits=1)),
                    (("f32", 32, 8704, 12288), dict(kind="skinny", mfma=1)),
                    (("f16", 3, 12288, 12288), dict(kind="skinny", mfma=0)),
                    (("f16", 3, 28672, 8192), dict(kind="skinny", mfma=0)),
                    (("f16", 3, 6144, 12288), dict(kind="split", fm=1, splits=5)),
+                   # B's rows no multiple of 512 bytes apart
+                   (("f16", 3, 12224, 4416), dict(kind="split", fm=1)),
+                   (("f16", 4, 13376, 9408), dict(kind="split", fm=1)),
+                   (("f32", 32, 8640, 6133), dict(kind="split")),
+                   (("f16", 9, 8096, 8192), dict(kind="split", fm=1, splits=4)),
+                   (("f32", 29, 10880, 12929), dict(kind="split")),
+                   (("f32", 32, 8704, 2688), dict(kind="split")),
                    (("f16", 24, 11008, 12288), dict(kind="split", fm=2, splits=1)),
                    (("f32", 24, 12288, 12288), dict(kind="split", fm=2, splits=1)),
                    (("f16", 16, 16384, 8192), dict(kind="split", fm=1, splits=1)),
