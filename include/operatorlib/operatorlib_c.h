@@ -156,11 +156,13 @@ int operatorlib_rmsnorm_f16(const operatorlib_half_t* input,
 
 /*
  * Workspace forms of the softmax and RMSNorm entry points (see the top of
- * this file). Rows longer than 32768 columns, and fewer than 64 rows longer
- * than 4096, are cut into segments over workgroups whose partials (8 bytes
- * per row and segment for softmax, 4 for RMSNorm) go to scratch; every
- * other shape needs none (the queries return 0). The result bits are those
- * of the plain forms.
+ * this file). Rows longer than 32768 columns, and some of fewer than 64 rows
+ * longer than 16384, are cut into segments over workgroups whose partials (8
+ * bytes per row and segment for softmax, 4 for RMSNorm) go to scratch. The
+ * queries ask for that scratch for every row longer than 32768 columns and for
+ * fewer than 64 rows longer than 4096, also where one workgroup per row is
+ * launched and leaves it unused; every other shape needs none (they return 0).
+ * The result bits are those of the plain forms.
  * Errors: as the plain forms; a workspace smaller than the query's answer,
  * or NULL or not 256-byte aligned when that is non-zero. The queries
  * return 0 for invalid sizes.

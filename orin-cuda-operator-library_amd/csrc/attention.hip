@@ -711,9 +711,9 @@ struct HalfScores {
 // each group with its own K/V stages; at the end the groups merge their
 // (O, max, sum) through LDS in group order, every wavefront taking a share
 // of the rows.
-// kW = wavefronts per group, 32 query rows each: 4 (128-row blocks), or 2 or 1
-// (64- or 32-row blocks) for the smallest grids, whose 128-row blocks would leave
-// CUs idle.
+// kW = wavefronts per group, 16 kQ query rows each (32; 48 in one instance): 4
+// (128-row blocks), or 2 or 1 (64-row, 48- or 32-row blocks) for the smallest grids,
+// whose 128-row blocks would leave CUs idle.
 // kTileKeys = keys per K/V tile: 64 (two 32-key halves per tile), or 32,
 // which halves the stages so that four groups fit the LDS of two.
 // A D = 128 workgroup with two groups and 64-key tiles, or four groups and
@@ -726,15 +726,15 @@ struct HalfScores {
 // against 20.5 us for two 64-key stages), so the tile loop is not waiting
 // on its copies; four groups, two wavefronts per SIMD, are what helps.
 // fp32 rows are twice as long: its instances use 32-key tiles (64 KiB of
-// K/V stages per group at D = 128), and at most two groups.
+// K/V stages per group at D = 128, where at most two groups fit).
 // Wavefronts per SIMD an instance must fit: one when four wavefronts hold
 // more than half a CU's LDS, else two.
 template <typename T, int D, int kGroups, int kW, int kTileKeys>
 constexpr int kMinWavesPerSimd =
     2 * kGroups * Layout<T, D, kTileKeys>::kStage > 80 * 1024 && kGroups * kW == 4 ? 1 : 2;
 
-// kQ: 16-row query blocks per wavefront, 2 except in the fp32 D = 64
-// instances of one wavefront per group.
+// kQ: 16-row query blocks per wavefront, 2 except in the instance of 48-row blocks
+// (fp32 D = 64, one wavefront per group).
 template <typename T, int D, int kGroups, int kW, int kTileKeys, int Dc = D, int kQ = 2>
 __global__ __launch_bounds__(kW * opl::kWaveSize * kGroups)
 __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<T, D, kGroups, kW, kTileKeys>, 2)))
@@ -1401,7 +1401,7 @@ constexpr int kFourGroupsFrom = 768;
 
 // Chooses the instance. `blocks`: 128-row query blocks. Grids too small to
 // fill the CUs split each query block's keys between groups of wavefronts in
-// the workgroup; the smallest also take 64- or 32-row blocks.
+// the workgroup; the smallest also take 64-, 48- or 32-row blocks.
 template <typename T>
 void launch(const T* q, const T* k, const T* v, float* out, int bh, int s, int dm, int causal,
             float scale, long long blocks, hipStream_t stream) {

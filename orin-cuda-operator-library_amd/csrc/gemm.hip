@@ -7,19 +7,24 @@
 // Reference: operatorlib::gemm_f16 / gemm_f32 (src/gemm.cu:440-479). The
 // reference dispatches between WMMA, cp.async register-tiled and scalar
 // kernels on divisibility; here the dispatch is, in order:
-//   * M <= 2 (fp16, B from 8 MiB) or M <= 4 (fp32, 8 from 128 MiB): the skinny kernel
-//     (namespace skinny), an HBM stream over B with split K and an ordered
-//     split sum (up to 32 fp16 / 64 fp32 rows, from M = 5 / 9 on the matrix
-//     cores, where K or N passes ksplit_kernel's 32-bit limits);
-//   * N <= 16 (matrix-vector products): namespace narrow, an HBM stream
-//     over A, one launch;
-//   * gemm_dma_kernel (any K, N and alignment, K below 2^22 fp16 / 2^21
-//     fp32 and N below 2^24): direct global->LDS loads that read the
-//     operands in place, described before the kernel; 256 x 256 tiles, or
-//     128 x 128 when the grid would leave CUs idle. Large fp16 products
-//     whose rows are not 4-byte aligned (e.g. 4095^3) first copy those
-//     operands into chunk-padded rows in scratch (the GPU's arena or the
-//     caller's workspace), see PadPlan;
+//   * M <= 2 (fp16, B from 8 MiB; 4 on some longer ones) or M <= 4 (fp32, 8 from 128
+//     MiB): the skinny kernel (namespace skinny), an HBM stream over B with split K and
+//     an ordered split sum (up to 32 fp16 / 64 fp32 rows, from M = 5 / 9 on the matrix
+//     cores, where K reaches 2^25 fp16 / 2^23 fp32 or N 2^24, past ksplit_kernel's
+//     32-bit offsets);
+//   * N <= 16 (matrix-vector products), but not those few rows where N fills 16-byte
+//     chunks: namespace narrow, an HBM stream over A, one launch;
+//   * ksplit_kernel, 16..96 x 64 tiles whose wavefronts split K (any alignment): those
+//     few rows, except where skinny_mfma_kernel draws a B from memory faster
+//     (skinny_mfma_faster), and grids of fewer than 160 (fp16) or 256 (fp32) tiles of
+//     256 x 256 that its time estimate takes from the next one (ksplit_plan);
+//   * gemm_dma_kernel (any N and alignment, K below 2^22 fp16 / 2^21 fp32 and N below
+//     2^24): direct global->LDS loads that read the operands in place, described before
+//     the kernel; 256 x 256 tiles, or where that grid would leave CUs idle 128 x 128
+//     (split along K where they are fewer than the CUs), in fp16 128 x 256 or 192 x 256
+//     where those make one round (one_round_rows). Large fp16 products whose rows are
+//     not 4-byte aligned (e.g. 4095^3) first copy those operands into chunk-padded rows
+//     in scratch (the GPU's arena or the caller's workspace), see PadPlan;
 //   * gemm_mfma_kernel, register-staged (Staging below), for K or N past
 //     those limits: 16-byte chunks from 16-byte aligned rows (K, N
 //     multiples of the chunk, aligned operands), or 16-byte chunks at
@@ -1124,9 +1129,9 @@ __global__ __launch_bounds__(256) void sum_tail_kernel(float* __restrict__ C, in
 }  // namespace dma
 
 // ---------------------------------------------------------------------------
-// Skinny GEMM, M <= 16 (the reference's M == 1 and M <= 16 configurations,
-// src/gemm.cu:445-448 and :464-467; LLM decode shapes such as 1 x 4096 x
-// 4096). The product is a stream over B (K x N): 2 MNK flops for 2-4 bytes
+// Skinny GEMM: M of one to eight on the vector ALU, up to 32 (fp16) or 64 (fp32) on
+// the matrix cores (the reference's M == 1 and M <= 16 configurations,
+// src/gemm.cu:445-448 and :464-467; LLM decode shapes such as 1 x 4096 x 4096). The product is a stream over B (K x N): 2 MNK flops for 2-4 bytes
 // of B per (k, n) pair, far below the matrix cores' balance, so the kernel
 // is built to stream B at HBM rate with vector-ALU dot products:
 //   * a 256-thread workgroup takes a 256-byte-wide column block of B (64
@@ -1144,7 +1149,7 @@ __global__ __launch_bounds__(256) void sum_tail_kernel(float* __restrict__ C, in
 //     go to scratch (arena or workspace) and a second kernel sums them in split
 //     order, so results are deterministic;
 //   * from M = 3 (fp16) or 5 (fp32) ksplit_kernel is faster and takes over
-//     (Cfg::kUpToM).
+//     (Cfg::kUpToM; `applies` names the exceptions).
 namespace skinny {
 
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
@@ -1161,8 +1166,8 @@ struct Cfg {
   static constexpr int kPerLane = 16 / sizeof(T);       // columns per lane
   static constexpr int kBlockN = kLanesPerRow * kPerLane;  // 64 fp32, 128 fp16
   static constexpr int kRowsPerStep = sizeof(T) == 2 ? 2 : 1;  // dot2 pairs
-  // The largest M this kernel takes, while B holds at least kMinBytes;
-  // beyond, and on smaller B, ksplit_kernel. Measured on MI355X (us, this
+  // The largest M that skinny_kernel takes on any B of at least kMinBytes (longer
+  // ones in `applies`); beyond, and on smaller B, ksplit_kernel. Measured on MI355X (us, this
   // kernel vs ksplit_kernel): fp16 M = 1 4096 x 4096 8.9 vs 10.2, 12288 x
   // 4096 (N x K) 20.0 vs 22.0; M = 4 4096^2 10.8 vs 10.4, 4096 x 11008 22.1
   // vs 18.2; M = 1 1024^2 5.5 vs 4.2, 768 x 3072 7.9 vs 5.7. fp32 M = 1
@@ -1884,8 +1889,8 @@ hipError_t launch(const T* a, const T* b, float* c, int m, int n, int k, hipStre
 //   * K is split over `splits` workgroups as well where the tiles are fewer
 //     than the CUs; their partial sums go to scratch and sum_splits_kernel
 //     adds them in order. The split inside the workgroup keeps those
-//     partials few: at most 6 M x N at M = 16, N = K = 4096, where the skinny
-//     matrix-core kernel this one replaced wrote 16.
+//     partials few: 3 M x N at M = 16, N = K = 4096, where skinny_mfma_kernel
+//     writes 16.
 //   * Workgroups of one panel of the longer operand and one K range are
 //     neighbours on one XCD, so that operand is read from memory once and
 //     the shorter one comes from the XCD's L2.
@@ -1898,11 +1903,11 @@ hipError_t launch(const T* a, const T* b, float* c, int m, int n, int k, hipStre
 // (Wide). 256 workgroups of 80 x 64 move (80 + 64) K 2 bytes each, 302 MB in
 // all, at 17 TB/s. fp32 is bound by its MFMAs from 32 rows on.
 // Measured on MI355X (us, inputs cycling through three sets; the kernels that
-// ran before -> this one): fp16 16 x 4096 x 4096 13.4 -> 11.0, 32 17.6 ->
-// 11.5, 64 21.5 -> 12.9, 128 22.7 -> 14.4, 200 22.9 -> 16.5, 300 31.9 ->
-// 18.7, 640 49.7 -> 37.3; 300 x 4096 x 11008 69.4 -> 54.7; 1024^3 21.9 ->
-// 8.6, 333 x 777 x 999 12.3 -> 7.8; fp32 1000^3 31.5 -> 22.4, 512^3 22.5 ->
-// 6.2, 64 x 4096 x 4096 41.5 -> 24.3, 300 x 4096 x 4096 108 -> 82.
+// ran before -> this one): fp16 16 x 4096 x 4096 13.4 -> 10.8, 32 17.7 ->
+// 12.4, 64 21.6 -> 13.2, 128 22.7 -> 14.3, 200 23.1 -> 17.9, 300 32.1 ->
+// 19.6, 640 49.6 -> 36.1; 300 x 4096 x 11008 69.7 -> 53.2; 1024^3 21.2 ->
+// 8.9, 333 x 777 x 999 12.3 -> 8.0; fp32 1000^3 32.3 -> 23.5, 512^3 22.4 ->
+// 5.9, 64 x 4096 x 4096 41.5 -> 24.6, 300 x 4096 x 4096 107 -> 82.
 // ---------------------------------------------------------------------------
 namespace ksplit {
 
@@ -2712,9 +2717,10 @@ struct TailPlan {
 
 // Grids of 128 x 128 tiles (two workgroups per CU) with fewer tiles than
 // CUs split every tile along K instead, into as many parts as fill the
-// workgroup slots (same limits). Small M past the skinny kernels' 16 rows
-// is the case: M = 17..128, N = K = 4096 is 32 tiles. Measured on MI355X
-// (us, whole tiles -> split, B cycling through 8 copies):
+// workgroup slots (same limits). ksplit_kernel takes most of these grids by its
+// estimate; what stays is medium and ragged: fp16 619 x 122 x 2688, 1500^3, fp32 99 x
+// 4564 x 9153, 634 x 832 x 6080. Measured on MI355X before it did (us, whole tiles ->
+// split, B cycling through 8 copies; N = K = 4096, 32 tiles at M up to 128):
 //   fp16 M = 17 30.4 -> 19.7, M = 64 31.8 -> 23.1, M = 128 37.1 -> 29.5,
 //     M = 256 39.4 -> 32.7;
 //   fp32 M = 17 236.8 -> 43.4, M = 64 238.3 -> 46.1, M = 128 237.9 ->
