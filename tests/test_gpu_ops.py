@@ -525,8 +525,8 @@ def test_gemm_skinny_row_blocks(hip, mnk, dtype):
 # 2048) and fewer steps than wavefronts; odd K and N (the end elements a copy's
 # range check drops); K split over workgroups too (first and last range of uneven
 # ones); M > N, whose items run in the other order. (Some of them, in one type or
-# both, run the 128 x 128 tiles or, 20 x 8200 x 8192, skinny_mfma_kernel: the tile
-# height follows from an estimate of time. KSPLIT_TILES names each instance.)
+# both, run the 128 x 128 tiles: the tile height follows from an estimate of time.
+# KSPLIT_TILES names each instance.)
 KSPLIT = [(15, 64, 256), (17, 65, 31), (33, 63, 33), (47, 130, 95), (80, 4096, 512),
           (81, 200, 1001), (97, 127, 64), (96, 3000, 2048), (300, 4100, 2049), (64, 4096, 2111),
           (5, 203, 4099), (16, 512, 8191), (3, 1, 1), (64, 33, 4097), (700, 40, 999),
